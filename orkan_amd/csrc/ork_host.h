@@ -47,6 +47,13 @@ typedef struct {
 ork_dev_t *ork_dev(void);
 /* runtime of the current device if it has been created, else NULL (creates nothing) */
 ork_dev_t *ork_dev_existing(void);
+/* device memory for state storage and scratch, kept for the next request when it is given back (ork_runtime.c).
+ * ork_mem_get: at least `bytes`, contents undefined, NULL when the device has none left.  ork_mem_put: returns a block
+ * whose last use is ordered before whatever the library stream runs next.  ork_mem_release: returns a block or frees
+ * any other device pointer after waiting for the device, as hipFree would. */
+void *ork_mem_get(size_t bytes);
+void ork_mem_put(void *p);
+void ork_mem_release(void *p);
 /* does p address device memory? */
 int ork_is_dev_ptr(const void *p);
 void ork_lock(void);

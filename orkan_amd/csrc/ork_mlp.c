@@ -368,8 +368,8 @@ int ork_topk(void *stream, const float *y, long n, int k, int *idx, float *vals,
 int orkan_topk_f32(const float *y_dev, long n, int k, int *idx_host, float *val_host) {
     if (!y_dev || !idx_host || k <= 0 || k > n || k > 65536) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    void *scratch = NULL;
-    int e = (int)hipMalloc(&scratch, ork_topk_state_bytes() + (size_t)k * (sizeof(int) + sizeof(float)));
+    void *scratch = ork_mem_get(ork_topk_state_bytes() + (size_t)k * (sizeof(int) + sizeof(float)));
+    int e = scratch ? 0 : (int)hipErrorOutOfMemory;
     float *vals = malloc((size_t)k * sizeof(float));
     int *idx = malloc((size_t)k * sizeof(int));
     int *ord = malloc((size_t)k * sizeof(int));
@@ -400,7 +400,7 @@ int orkan_topk_f32(const float *y_dev, long n, int k, int *idx_host, float *val_
     free(vals);
     free(idx);
     free(ord);
-    if (scratch) (void)hipFree(scratch);
+    ork_mem_put(scratch);
     return e;
 }
 

@@ -340,10 +340,9 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
 int orkan_maxcut_diag_dev(int n, int nedges, const int *ei, const int *ej, const double *w, double *out_dev) {
     ork_dev_t *d = ork_dev();
     hipStream_t st = (hipStream_t)d->stream;
-    int *ed = NULL;
-    double *wd = NULL;
-    int e = (int)hipMalloc((void **)&ed, (size_t)(2 * nedges + 1) * sizeof(int));
-    if (!e) e = (int)hipMalloc((void **)&wd, (size_t)(nedges + 1) * sizeof(double));
+    int *ed = ork_mem_get((size_t)(2 * nedges + 1) * sizeof(int));
+    double *wd = ork_mem_get((size_t)(nedges + 1) * sizeof(double));
+    int e = ed && wd ? 0 : (int)hipErrorOutOfMemory;
     if (!e && nedges > 0) {
         e |= (int)hipMemcpyAsync(ed, ei, (size_t)nedges * sizeof(int), hipMemcpyHostToDevice, st);
         e |= (int)hipMemcpyAsync(ed + nedges, ej, (size_t)nedges * sizeof(int), hipMemcpyHostToDevice, st);
@@ -351,7 +350,7 @@ int orkan_maxcut_diag_dev(int n, int nedges, const int *ei, const int *ej, const
     }
     if (!e) e = ork_maxcut_diag(st, out_dev, n, nedges, ed, ed + nedges, wd);
     if (!e) e = (int)hipStreamSynchronize(st);
-    if (ed) (void)hipFree(ed);
-    if (wd) (void)hipFree(wd);
+    ork_mem_put(ed);
+    ork_mem_put(wd);
     return e;
 }

@@ -85,6 +85,152 @@ const double *ork_dev_doubles(const double *src, size_t count) {
 }
 
 /* ------------------------------------------------------------------------------------------------
+ * device memory of states and scratch
+ *
+ * hipMalloc and hipFree map and unmap pages: a state_cp, relayout and precision conversion of a 12-qubit density
+ * matrix (134 MB each) spent 9.2 of their 9.6 ms there, a sample_matrix call on 18 qubits about 1 of 4 ms.  Blocks given
+ * back are therefore kept, per device, for the next request of nearly the same size.  At most ORK_MEM_KEEP bytes are
+ * kept (the oldest blocks go back to the device first, larger ones at once), and all of them go back when the device
+ * runs out.  A block is only handed out for use on the library stream, after everything that used it.
+ * ---------------------------------------------------------------------------------------------- */
+#define ORK_MEM_KEEP ((size_t)8 << 30)
+#define ORK_MEM_BUCKETS 1024
+
+typedef struct mem_block {
+    void *p;
+    size_t bytes;
+    int dev;
+    int kept;                          /* given back, in its device's list */
+    struct mem_block *chain;           /* next block of the same bucket */
+    struct mem_block *older, *newer;   /* kept blocks of a device, by the time they came back */
+} mem_block_t;
+
+static pthread_mutex_t g_mem_mu = PTHREAD_MUTEX_INITIALIZER;
+static mem_block_t *g_mem_table[ORK_MEM_BUCKETS];
+static mem_block_t *g_mem_oldest[ORK_MAX_DEV], *g_mem_newest[ORK_MAX_DEV];
+static size_t g_mem_kept[ORK_MAX_DEV];
+
+static mem_block_t **mem_slot(const void *p) {
+    mem_block_t **s = &g_mem_table[((uintptr_t)p >> 12) % ORK_MEM_BUCKETS];
+    while (*s && (*s)->p != p) s = &(*s)->chain;
+    return s;
+}
+
+static void mem_unkeep(mem_block_t *b) {
+    *(b->older ? &b->older->newer : &g_mem_oldest[b->dev]) = b->newer;
+    *(b->newer ? &b->newer->older : &g_mem_newest[b->dev]) = b->older;
+    g_mem_kept[b->dev] -= b->bytes;
+    b->kept = 0;
+}
+
+static void mem_forget(const void *p) {
+    mem_block_t **s = mem_slot(p), *b = *s;
+    if (!b) return;
+    if (b->kept) mem_unkeep(b);
+    *s = b->chain;
+    free(b);
+}
+
+/* kept blocks of the device back to it, the oldest first, until at most `keep` bytes are left */
+static void mem_trim(int dev, size_t keep) {
+    while (g_mem_kept[dev] > keep) {
+        void *p = g_mem_oldest[dev]->p;
+        mem_forget(p);
+        (void)hipFree(p);
+    }
+}
+
+void *ork_mem_get(size_t bytes) {
+    int dev = 0;
+    void *p = NULL;
+    ork_dev();
+    if (hipGetDevice(&dev) != hipSuccess) return NULL;
+    if (bytes < 256) bytes = 256;
+    pthread_mutex_lock(&g_mem_mu);
+    /* the smallest kept block that holds the request and is at most an eighth larger */
+    mem_block_t *best = NULL;
+    for (mem_block_t *b = g_mem_newest[dev]; b; b = b->older)
+        if (b->bytes >= bytes && b->bytes - bytes <= bytes / 8 && (!best || b->bytes < best->bytes)) best = b;
+    if (best) {
+        mem_unkeep(best);
+        p = best->p;
+    } else {
+        if (hipMalloc(&p, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            mem_trim(dev, 0);
+            p = NULL;
+            if (hipMalloc(&p, bytes) != hipSuccess) {
+                (void)hipGetLastError();
+                p = NULL;
+            }
+        }
+        if (p) {
+            mem_forget(p);   /* an entry of this address is of a block that was freed elsewhere */
+            mem_block_t *b = calloc(1, sizeof(*b));
+            if (b) {
+                b->p = p;
+                b->bytes = bytes;
+                b->dev = dev;
+                *mem_slot(p) = b;
+            }
+        }
+    }
+    pthread_mutex_unlock(&g_mem_mu);
+    return p;
+}
+
+/* the block of p, if p is one that is out and still the allocation this table knows (a caller may have freed it with
+ * hipFree and have been given the address again) */
+static mem_block_t *mem_live(void *p) {
+    mem_block_t *b = *mem_slot(p);
+    if (!b || b->kept) return NULL;
+    hipDeviceptr_t base = NULL;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+        (void)hipGetLastError();
+        base = NULL;
+    }
+    if (base == (hipDeviceptr_t)p && size >= b->bytes && size - b->bytes < 4096) return b;
+    mem_forget(p);
+    return NULL;
+}
+
+void ork_mem_put(void *p) {
+    if (!p) return;
+    pthread_mutex_lock(&g_mem_mu);
+    mem_block_t *b = mem_live(p);
+    if (b && b->bytes <= ORK_MEM_KEEP) {
+        b->kept = 1;
+        b->newer = NULL;
+        b->older = g_mem_newest[b->dev];
+        *(b->older ? &b->older->newer : &g_mem_oldest[b->dev]) = b;
+        g_mem_newest[b->dev] = b;
+        g_mem_kept[b->dev] += b->bytes;
+        mem_trim(b->dev, ORK_MEM_KEEP);
+    } else {
+        mem_forget(p);
+        (void)hipFree(p);
+    }
+    pthread_mutex_unlock(&g_mem_mu);
+}
+
+void ork_mem_release(void *p) {
+    if (!p) return;
+    ork_dev();
+    int cur = 0, dev = -1;
+    (void)hipGetDevice(&cur);
+    pthread_mutex_lock(&g_mem_mu);
+    const mem_block_t *b = *mem_slot(p);
+    if (b) dev = b->dev;
+    pthread_mutex_unlock(&g_mem_mu);
+    /* work of the caller's own streams may still use the memory, on the device it belongs to */
+    if (dev >= 0 && dev != cur) (void)hipSetDevice(dev);
+    (void)hipDeviceSynchronize();
+    if (dev >= 0 && dev != cur) (void)hipSetDevice(cur);
+    ork_mem_put(p);
+}
+
+/* ------------------------------------------------------------------------------------------------
  * extension API: stream access, device arrays, timing
  * ---------------------------------------------------------------------------------------------- */
 
@@ -139,10 +285,7 @@ int orkan_copy_to_device(void *dst_dev, const void *src_host, size_t bytes) {
 }
 
 void orkan_dev_free(void *p) {
-    if (!p) return;
-    ork_dev();
-    (void)hipDeviceSynchronize();
-    (void)hipFree(p);
+    ork_mem_release(p);
 }
 
 #define ORK_MAX_EVENTS 65536

@@ -95,14 +95,11 @@ qs_error_t sample_matrix(state_t *iota, const double *obs, const ansatz_channel_
     double *o = NULL;
     cplx_t *Gh = malloc((size_t)B * B * sizeof(cplx_t));
     qs_error_t rc = Gh ? QS_OK : QS_ERR_OOM;
-    if (rc == QS_OK && (hipMalloc((void **)&tmp, vec) != hipSuccess || hipMalloc((void **)&acc, vec) != hipSuccess ||
-                        hipMalloc((void **)&phj, vec * B) != hipSuccess || hipMalloc((void **)&phi, vec * B) != hipSuccess ||
-                        hipMalloc((void **)&part, part_bytes) != hipSuccess ||
-                        hipMalloc((void **)&G, (size_t)B * B * sizeof(cplx_t)) != hipSuccess ||
-                        hipMalloc((void **)&o, (size_t)N * sizeof(double)) != hipSuccess)) {
-        (void)hipGetLastError();
+    if (rc == QS_OK && (!(tmp = ork_mem_get(vec)) || !(acc = ork_mem_get(vec)) || !(phj = ork_mem_get(vec * B)) ||
+                        !(phi = ork_mem_get(vec * B)) || !(part = ork_mem_get(part_bytes)) ||
+                        !(G = ork_mem_get((size_t)B * B * sizeof(cplx_t))) ||
+                        !(o = ork_mem_get((size_t)N * sizeof(double)))))
         rc = QS_ERR_OOM;
-    }
     int e = 0;
     if (rc == QS_OK)
         e = (int)hipMemcpyAsync(o, obs, (size_t)N * sizeof(double), hipMemcpyDefault, (hipStream_t)d->stream);
@@ -137,8 +134,7 @@ qs_error_t sample_matrix(state_t *iota, const double *obs, const ansatz_channel_
     }
     (void)hipStreamSynchronize((hipStream_t)d->stream);
     void *bufs[] = {tmp, acc, phj, phi, part, G, o};
-    for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i)
-        if (bufs[i]) (void)hipFree(bufs[i]);
+    for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i) ork_mem_put(bufs[i]);
     free(Gh);
     if (e) ork_hip_fail("sample_matrix", e);   /* a failed HIP call exits like every other entry point */
     return rc;

@@ -38,15 +38,9 @@ idx_t state_len(const state_t *state) {
 }
 
 static void *dev_zeros(size_t bytes) {
-    void *p = NULL;
-    if (bytes == 0) bytes = 16;
-    if (hipMalloc(&p, bytes) != hipSuccess) {
-        (void)hipGetLastError();
-        return NULL;
-    }
-    ork_dev_t *d = ork_dev();
-    if (hipMemsetAsync(p, 0, bytes, (hipStream_t)d->stream) != hipSuccess) {
-        (void)hipFree(p);
+    void *p = ork_mem_get(bytes);
+    if (p && hipMemsetAsync(p, 0, bytes, (hipStream_t)ork_dev()->stream) != hipSuccess) {
+        ork_mem_put(p);
         return NULL;
     }
     return p;
@@ -62,30 +56,40 @@ static int is_dev(const void *p) {
     return at.type == hipMemoryTypeDevice;
 }
 
-static void dev_release(void *p) {
-    if (!p) return;
-    (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
-    (void)hipFree(p);
-}
-
-void state_init(state_t *state, qubit_t qubits, cplx_t **data) {
-    assert(state != NULL);
-    ork_dev();
+/* the state's old storage goes, storage for `qubits` comes (zero-filled or undefined) */
+static void new_storage(state_t *state, qubit_t qubits, int zeros) {
     if (state->data) {
-        dev_release(state->data);
+        ork_mem_release(state->data);
         state->data = NULL;
     }
     state->qubits = qubits;
     const idx_t len = state_len(state);
     const size_t bytes = (size_t)len * ork_elem_bytes(state);
+    state->data = zeros ? dev_zeros(bytes) : ork_mem_get(bytes);
+    if (!state->data) {
+        fprintf(stderr, "state_init(): allocation failed for %zu elements\n", (size_t)len);
+        state->qubits = 0;
+    }
+}
+
+void state_init(state_t *state, qubit_t qubits, cplx_t **data) {
+    assert(state != NULL);
+    ork_dev();
     if (data && *data) {
+        if (state->data) {
+            ork_mem_release(state->data);
+            state->data = NULL;
+        }
+        state->qubits = qubits;
+        const idx_t len = state_len(state);
+        const size_t bytes = (size_t)len * ork_elem_bytes(state);
         if (is_dev(*data)) {
             /* a device buffer becomes the state's storage as it is */
             state->data = *data;
         } else {
             /* a host buffer: copied into HBM, then released like the reference's
              * re-aligning copy (src/state/state.c:72-87) */
-            state->data = dev_zeros(bytes);
+            state->data = ork_mem_get(bytes);
             if (!state->data) {
                 fprintf(stderr, "state_init(): aligned realloc failed for %zu elements\n", (size_t)len);
                 state->qubits = 0;
@@ -93,7 +97,6 @@ void state_init(state_t *state, qubit_t qubits, cplx_t **data) {
                 *data = NULL;
                 return;
             }
-            /* on the library stream, after the zero fill that dev_zeros enqueued there */
             hipStream_t st = (hipStream_t)ork_dev()->stream;
             ORK_HIP("state_init upload", hipMemcpyAsync(state->data, *data, bytes, hipMemcpyHostToDevice, st));
             ORK_HIP("state_init upload", hipStreamSynchronize(st));
@@ -102,16 +105,12 @@ void state_init(state_t *state, qubit_t qubits, cplx_t **data) {
         *data = NULL;
         return;
     }
-    state->data = dev_zeros(bytes);
-    if (!state->data) {
-        fprintf(stderr, "state_init(): allocation failed for %zu elements\n", (size_t)len);
-        state->qubits = 0;
-    }
+    new_storage(state, qubits, 1);
 }
 
 void state_free(state_t *state) {
     if (!state) return;
-    dev_release(state->data);
+    ork_mem_release(state->data);
     state->data = NULL;
     state->qubits = 0;
 }
@@ -119,11 +118,12 @@ void state_free(state_t *state) {
 void state_plus(state_t *state, qubit_t qubits) {
     assert(state != NULL);
     assert(ork_type_ok(state) && "state_plus(): invalid state type");
-    state_init(state, qubits, NULL);
-    if (!state->data) return;
-    ork_dev_t *d = ork_dev();
     const int layout = ork_layout(state), prec = ork_prec(state);
     const idx_t dim = (idx_t)1 << qubits;
+    /* only the padded tile keeps zeros: every other entry is written below */
+    new_storage(state, qubits, layout == MIXED_TILED && qubits < LOG_TILE_DIM);
+    if (!state->data) return;
+    ork_dev_t *d = ork_dev();
     if (layout == PURE) {
         ORK_HIP("state_plus", ork_fill(d->stream, prec, state->data, dim, 1.0 / sqrt((double)dim), 0.0));
     } else if (layout == MIXED_TILED && qubits < LOG_TILE_DIM) {
@@ -137,7 +137,7 @@ state_t state_cp(const state_t *state) {
     assert(state != NULL && state->data != NULL);
     state_t out = *state;
     const size_t bytes = (size_t)state_len(state) * ork_elem_bytes(state);
-    out.data = dev_zeros(bytes);
+    out.data = ork_mem_get(bytes);
     if (!out.data) {
         fprintf(stderr, "state_cp(): allocation failed\n");
         out.qubits = 0;
@@ -315,7 +315,7 @@ state_t orkan_state_convert(const state_t *state, int to_fp32) {
     state_t out = *state;
     out.type = (state_type_t)(((int)state->type & ~ORKAN_FP32) | (to_fp32 ? ORKAN_FP32 : 0));
     const idx_t len = state_len(state);
-    out.data = dev_zeros((size_t)len * ork_elem_bytes(&out));
+    out.data = ork_mem_get((size_t)len * ork_elem_bytes(&out));
     if (!out.data) {
         out.qubits = 0;
         return out;
@@ -339,7 +339,7 @@ qs_error_t orkan_state_relayout(const state_t *src, state_t *dst, state_type_t l
     out.type = (state_type_t)((int)layout | ((int)src->type & ORKAN_FP32));
     out.qubits = src->qubits;
     const idx_t len = ork_len((int)layout, src->qubits);
-    out.data = dev_zeros((size_t)len * ork_elem_bytes(&out));
+    out.data = ork_mem_get((size_t)len * ork_elem_bytes(&out));
     if (!out.data) return QS_ERR_OOM;
     ork_dev_t *d = ork_dev();
     ORK_HIP("orkan_state_relayout", ork_relayout(d->stream, ork_prec(src), src->data, ork_layout(src), out.data,
@@ -454,7 +454,7 @@ qs_error_t orkan_state_load(state_t *state, const char *path) {
         }
     }
     if (rc == QS_OK) {
-        dev = dev_zeros(total);
+        dev = ork_mem_get(total);
         if (!dev) rc = QS_ERR_OOM;
     }
     char *buf = rc == QS_OK ? malloc(total < ORK_FILE_CHUNK ? (total ? total : 1) : ORK_FILE_CHUNK) : NULL;
@@ -475,7 +475,7 @@ qs_error_t orkan_state_load(state_t *state, const char *path) {
     free(buf);
     fclose(f);
     if (rc != QS_OK) {
-        if (dev) dev_release(dev);
+        if (dev) ork_mem_release(dev);
         return rc;
     }
     state_free(state);
