@@ -11,11 +11,7 @@
 //
 // No reference counterpart: this is the learned screening stage on top of the
 // simulator.
-#include "k_common.hpp"
-
-typedef __bf16 bf16;
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
+#include "k_mlp.hpp"
 
 namespace {
 
@@ -23,47 +19,12 @@ constexpr int BM = 128, BN = 128, BK = 32;
 constexpr int KP = BK + 8;            // padded LDS row (bf16 elements)
 constexpr int GT = 256;               // threads per GEMM workgroup
 
-enum { EPI_F32 = 0, EPI_BIAS_GELU = 1, EPI_GELU_BWD = 2, EPI_F32_ACC = 3 };
-
-// erf(x) by Abramowitz & Stegun, Handbook of Mathematical Functions, 7.1.26 (Hastings):
-// 1 - (a1 t + ... + a5 t^5) exp(-x^2), t = 1 / (1 + p |x|), |error| <= 1.5e-7, far below the
-// bf16 rounding of the activations it feeds; branch-free, unlike a piecewise erff, which
-// dominated the GEMM epilogue.
-__device__ __forceinline__ float erf_as(float x) {
-    const float ax = fabsf(x);
-    // hardware reciprocal (1 ulp): the approximation's own error is 1.5e-7
-    const float t = __builtin_amdgcn_rcpf(fmaf(0.3275911f, ax, 1.0f));
-    const float poly =
-        t * (0.254829592f + t * (-0.284496736f + t * (1.421413741f + t * (-1.453152027f + t * 1.061405429f))));
-    return copysignf(1.0f - poly * __expf(-ax * ax), x);
-}
-__device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + erf_as(x * 0.70710678118654752f)); }
-__device__ __forceinline__ float gelu_grad(float x) {
-    const float cdf = 0.5f * (1.0f + erf_as(x * 0.70710678118654752f));
-    const float pdf = 0.39894228040143268f * __expf(-0.5f * x * x);
-    return cdf + x * pdf;
-}
-
-struct EpiArgs {
-    float *c32;          // EPI_F32 / EPI_F32_ACC: fp32 C, ldc
-    int ldc;
-    const float *bias;   // EPI_BIAS_GELU: bias[N]
-    float *pre;          // EPI_BIAS_GELU: pre-activation out (fp32, ldc); EPI_GELU_BWD: pre-activation in
-    bf16 *act;           // EPI_BIAS_GELU: gelu(pre) out (bf16, ldc); EPI_GELU_BWD: dPre out (bf16, ldc)
-    long zstride;        // split K (gemm_nt_kernel, EPI_F32): c32 offset between the gridDim.z slices
-};
-
 template <int EPI>
 __global__ __launch_bounds__(GT) void gemm_nt_kernel(const bf16 *__restrict__ A, int lda, const bf16 *__restrict__ B,
                                                      int ldb, int K, EpiArgs ep) {
     __shared__ __attribute__((aligned(16))) bf16 As[2][BM * KP];
     __shared__ __attribute__((aligned(16))) bf16 Bs[2][BN * KP];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (gridDim.z > 1) {   // split K: slice z covers columns [z K, z K + K) of A and B
-        A += (long)blockIdx.z * K;
-        B += (long)blockIdx.z * K;
-        ep.c32 += (long)blockIdx.z * ep.zstride;
-    }
     const int wm = wave >> 1, wn = wave & 1;
     const long m0 = (long)blockIdx.y * BM, n0 = (long)blockIdx.x * BN;
     // global -> register staging: each thread moves 16 bf16 of A and 16 of B per K step
@@ -362,20 +323,6 @@ __global__ __launch_bounds__(GT3) void gemm_nt_dma_kernel(const bf16 *__restrict
 
 
 // ---- small kernels -----------------------------------------------------------------------------
-__global__ void transpose_bf16_kernel(const bf16 *__restrict__ in, bf16 *__restrict__ out, int R, int Cc) {
-    __shared__ bf16 t[32][33];
-    const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
-    for (int y = threadIdx.y; y < 32; y += 8)
-        if (by + y < R && bx + threadIdx.x < Cc) t[y][threadIdx.x] = in[(long)(by + y) * Cc + bx + threadIdx.x];
-    __syncthreads();
-    for (int y = threadIdx.y; y < 32; y += 8)
-        if (bx + y < Cc && by + threadIdx.x < R) out[(long)(bx + y) * R + by + threadIdx.x] = t[threadIdx.x][y];
-}
-
-__global__ void f32_to_bf16_kernel(const float *__restrict__ in, bf16 *__restrict__ out, long n) {
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) out[i] = (bf16)in[i];
-}
-
 // y[m] = sum_k h[m][k] w[k] + b   (one wave per row); optional loss gradient and
 // per-row squared error (target given)
 __global__ __launch_bounds__(256) void head_forward_kernel(const bf16 *__restrict__ h, const float *__restrict__ w, float b,
@@ -405,98 +352,6 @@ __global__ __launch_bounds__(256) void head_forward_kernel(const bf16 *__restric
             const float e = (row < valid) ? (v - target[row]) : 0.0f;
             dy[row] = 2.0f * e * scale;
             sqerr[row] = e * e;
-        }
-    }
-}
-
-// dPre3[m][k] = dy[m] w[k] gelu'(pre3[m][k])   (bf16 out)
-__global__ void head_backward_kernel(const float *__restrict__ dy, const float *__restrict__ w,
-                                     const float *__restrict__ pre, bf16 *__restrict__ dpre, int M, int K) {
-    const long n = (long)M * K;
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-        const long m = i / K;
-        const int k = (int)(i % K);
-        dpre[i] = (bf16)(dy[m] * w[k] * gelu_grad(pre[i]));
-    }
-}
-
-// out[k] = sum_m a[m][k] * s[m] (a bf16 [M][K]); bias grads use s = null (sum of rows).
-// Stage 1: COLSUM_CHUNKS row chunks in parallel into part[chunk][K]; stage 2 adds the
-// chunks in a fixed order (deterministic, no atomics).
-constexpr int COLSUM_CHUNKS = 64;
-__global__ __launch_bounds__(256) void colsum_part_kernel(const bf16 *__restrict__ a, const float *__restrict__ s, int M,
-                                                         int K, float *__restrict__ part) {
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= K) return;
-    const int rows = (M + COLSUM_CHUNKS - 1) / COLSUM_CHUNKS;
-    const int m0 = blockIdx.y * rows, m1 = min(M, m0 + rows);
-    float acc = 0.0f;
-    for (int m = m0; m < m1; ++m) acc += (float)a[(long)m * K + k] * (s ? s[m] : 1.0f);
-    part[(long)blockIdx.y * K + k] = acc;
-}
-// 8 columns per thread (16 B loads), 4 row subgroups of a chunk summed through LDS in a fixed order
-__global__ __launch_bounds__(256) void colsum_part8_kernel(const bf16 *__restrict__ a, const float *__restrict__ s,
-                                                          int M, int K, float *__restrict__ part) {
-    __shared__ float red[4][512];
-    const int tx = threadIdx.x & 63, ty = threadIdx.x >> 6;
-    const int k0 = blockIdx.x * 512 + tx * 8;
-    const int rows = (M + COLSUM_CHUNKS - 1) / COLSUM_CHUNKS;
-    const int m0 = blockIdx.y * rows, m1 = min(M, m0 + rows);
-    float acc[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-    if (k0 < K)
-        for (int m = m0 + ty; m < m1; m += 4) {
-            const bf16x8 v = *(const bf16x8 *)(a + (long)m * K + k0);
-            const float sc = s ? s[m] : 1.0f;
-#pragma unroll
-            for (int t = 0; t < 8; ++t) acc[t] += (float)v[t] * sc;
-        }
-#pragma unroll
-    for (int t = 0; t < 8; ++t) red[ty][tx * 8 + t] = acc[t];
-    __syncthreads();
-    if (ty == 0 && k0 < K)
-#pragma unroll
-        for (int t = 0; t < 8; ++t) {
-            const int c = tx * 8 + t;
-            part[(long)blockIdx.y * K + k0 + t] = ((red[0][c] + red[1][c]) + red[2][c]) + red[3][c];
-        }
-}
-
-__global__ __launch_bounds__(256) void colsum_finish_kernel(const float *__restrict__ part, int K,
-                                                           float *__restrict__ out) {
-    const int k = blockIdx.x * 256 + threadIdx.x;
-    if (k >= K) return;
-    float acc = 0.0f;
-    for (int c = 0; c < COLSUM_CHUNKS; ++c) acc += part[(long)c * K + k];
-    out[k] = acc;
-}
-
-__global__ void sum_kernel(const float *__restrict__ v, int n, float *__restrict__ out) {
-    __shared__ float red[4];
-    float acc = 0.0f;
-    for (int i = threadIdx.x; i < n; i += 256) acc += v[i];
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) out[0] = red[0] + red[1] + red[2] + red[3];
-}
-
-// Adam on fp32 master weights; refresh the bf16 copies W [K][N] and Wt [N][K]
-__global__ void adam_kernel(float *__restrict__ w, const float *__restrict__ g, float *__restrict__ m,
-                            float *__restrict__ v, long n, int ncols, float lr, float b1, float b2, float eps,
-                            float c1, float c2, bf16 *__restrict__ wb, bf16 *__restrict__ wtb, int nrows) {
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < n; i += (long)gridDim.x * 256) {
-        const float gi = g[i];
-        const float mi = b1 * m[i] + (1.0f - b1) * gi;
-        const float vi = b2 * v[i] + (1.0f - b2) * gi * gi;
-        m[i] = mi;
-        v[i] = vi;
-        const float wi = w[i] - lr * (mi / c1) / (sqrtf(vi / c2) + eps);
-        w[i] = wi;
-        if (wb) wb[i] = (bf16)wi;
-        if (wtb) {
-            const long r = i / ncols, c = i % ncols;
-            wtb[c * nrows + r] = (bf16)wi;
         }
     }
 }
@@ -650,6 +505,10 @@ extern "C" int ork_mlp_gemm_select(int variant) {
     return 0;
 }
 
+extern "C" int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N,
+                                int K, float *c32, int ldc, const float *bias, float *pre, void *act, void *actT,
+                                long ldt);
+
 // epi: 0 fp32 C, 1 bias+GELU, 2 GELU backward, 3 fp32 C +=
 extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
                             float *c32, int ldc, const float *bias, float *pre, void *act) {
@@ -659,7 +518,8 @@ extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const
     const bf16 *a = (const bf16 *)A, *b = (const bf16 *)B;
     // the DMA moves 16 B per lane: rows of both operands must start on 16 B boundaries
     const bool aligned16 = lda % 8 == 0 && ldb % 8 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0;
-    if (g_gemm_big == 2 && aligned16 && M % BM2 == 0 && N % BN2 == 0 && K % (4 * BK3) == 0 && K > 0) {
+    if (g_gemm_big == 2 && aligned16 && M % BM2 == 0 && N % BN2 == 0 && K % (4 * BK3) == 0 &&
+        (long)(M / BM2) * (N / BN2) >= 256) {
         dim3 grid3(N / BN2, M / BM2);
         switch (epi) {
         case EPI_F32: gemm_nt_dma_kernel<EPI_F32><<<grid3, GT3, 0, st>>>(a, lda, b, ldb, K, ep); break;
@@ -671,7 +531,7 @@ extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const
         ORK_LAUNCH_CHECK();
         return 0;
     }
-    if (g_gemm_big && M % BM2 == 0 && N % BN2 == 0 && K % BK2 == 0) {
+    if (g_gemm_big == 1 && M % BM2 == 0 && N % BN2 == 0 && K % BK2 == 0) {
         dim3 grid2(N / BN2, M / BM2);
         switch (epi) {
         case EPI_F32: gemm_nt_big_kernel<EPI_F32><<<grid2, GT2, BIG_LDS, st>>>(a, lda, b, ldb, K, ep); break;
@@ -683,6 +543,10 @@ extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const
         ORK_LAUNCH_CHECK();
         return 0;
     }
+    // Fewer 256 x 256 tiles than CUs: 128 x 64 tiles, four times the workgroups (4096 x 512 x 512 with its fused
+    // epilogue: 11 us against 28 on 32 workgroups of 256 x 256); also for shapes the large tile does not divide
+    if (g_gemm_big == 2 && aligned16 && epi != EPI_F32_ACC)
+        return ork_mlp_gemm_mid(stream, epi, A, lda, B, ldb, M, N, K, c32, ldc, bias, pre, act, nullptr, 0);
     dim3 grid(N / BN, M / BM);
     switch (epi) {
     case EPI_F32: gemm_nt_kernel<EPI_F32><<<grid, GT, 0, st>>>(a, lda, b, ldb, K, ep); break;
@@ -695,79 +559,10 @@ extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const
     return 0;
 }
 
-// c[r][col] = sum over the slices, in slice order (deterministic)
-__global__ void splitk_sum_kernel(const float *__restrict__ work, int slices, long mn, int N, float *__restrict__ c,
-                                  int ldc) {
-    for (long i = (long)blockIdx.x * 256 + threadIdx.x; i < mn; i += (long)gridDim.x * 256) {
-        float s = 0.0f;
-        for (int z = 0; z < slices; ++z) s += work[z * mn + i];
-        c[(i / N) * ldc + i % N] = s;
-    }
-}
-
-// C = A B^T with K split into `slices` equal slices on the 128 x 128 tile (fp32 partial products in
-// work[slices][M][N], then summed in slice order): the batch-length weight-gradient products, whose
-// M x N has only a few tiles
-extern "C" int ork_mlp_gemm_splitk(void *stream, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
-                                   int slices, float *work, float *c32, int ldc) {
-    if (slices < 1 || slices > 65535 || K % slices || (K / slices) % BK || K <= 0 || M % BM || N % BN || M <= 0 ||
-        N <= 0)
-        return (int)hipErrorInvalidValue;
-    hipStream_t st = (hipStream_t)stream;
-    EpiArgs ep{work, N, nullptr, nullptr, nullptr, (long)M * N};
-    dim3 grid(N / BN, M / BM, slices);
-    gemm_nt_kernel<EPI_F32><<<grid, GT, 0, st>>>((const bf16 *)A, lda, (const bf16 *)B, ldb, K / slices, ep);
-    ORK_LAUNCH_CHECK();
-    splitk_sum_kernel<<<g1((long)M * N), 256, 0, st>>>(work, slices, (long)M * N, N, c32, ldc);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
-extern "C" int ork_mlp_transpose(void *stream, const void *in, void *out, int R, int Cc) {
-    dim3 grid((Cc + 31) / 32, (R + 31) / 32), blk(32, 8);
-    transpose_bf16_kernel<<<grid, blk, 0, (hipStream_t)stream>>>((const bf16 *)in, (bf16 *)out, R, Cc);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
-extern "C" int ork_mlp_to_bf16(void *stream, const float *in, void *out, long n) {
-    f32_to_bf16_kernel<<<g1(n), 256, 0, (hipStream_t)stream>>>(in, (bf16 *)out, n);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
 extern "C" int ork_mlp_head_forward(void *stream, const void *h, const float *w, float b, int M, int K, float *y,
                                     const float *target, float *dy, float *sqerr, int valid, float scale) {
     head_forward_kernel<<<(M + 3) / 4, 256, 0, (hipStream_t)stream>>>((const bf16 *)h, w, b, M, K, y, target, dy,
                                                                       sqerr, valid, scale);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
-extern "C" int ork_mlp_head_backward(void *stream, const float *dy, const float *w, const float *pre, void *dpre,
-                                     int M, int K) {
-    head_backward_kernel<<<g1((long)M * K), 256, 0, (hipStream_t)stream>>>(dy, w, pre, (bf16 *)dpre, M, K);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
-// part: scratch of COLSUM_CHUNKS * K floats
-extern "C" int ork_mlp_colsum(void *stream, const void *a, const float *s, int M, int K, float *out, float *part) {
-    if (K % 8 == 0 && ((uintptr_t)a & 15) == 0) {
-        dim3 g8((K + 511) / 512, COLSUM_CHUNKS);
-        colsum_part8_kernel<<<g8, 256, 0, (hipStream_t)stream>>>((const bf16 *)a, s, M, K, part);
-    } else {
-        dim3 g1d((K + 255) / 256, COLSUM_CHUNKS);
-        colsum_part_kernel<<<g1d, 256, 0, (hipStream_t)stream>>>((const bf16 *)a, s, M, K, part);
-    }
-    ORK_LAUNCH_CHECK();
-    colsum_finish_kernel<<<(K + 255) / 256, 256, 0, (hipStream_t)stream>>>(part, K, out);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
-extern "C" int ork_mlp_sum(void *stream, const float *v, int n, float *out) {
-    sum_kernel<<<1, 256, 0, (hipStream_t)stream>>>(v, n, out);
     ORK_LAUNCH_CHECK();
     return 0;
 }
@@ -819,14 +614,6 @@ extern "C" int ork_topk(void *stream, const float *y, long n, int k, int *idx, f
     topk_compact_kernel<<<(unsigned)g, 256, 0, st>>>(y, n, ts, k, idx);
     ORK_LAUNCH_CHECK();
     gather_f32_kernel<<<(k + 255) / 256, 256, 0, st>>>(y, idx, vals, k);
-    ORK_LAUNCH_CHECK();
-    return 0;
-}
-
-extern "C" int ork_mlp_adam(void *stream, float *w, const float *g, float *m, float *v, long n, int ncols, float lr,
-                            float b1, float b2, float eps, float c1, float c2, void *wb, void *wtb, int nrows) {
-    adam_kernel<<<g1(n), 256, 0, (hipStream_t)stream>>>(w, g, m, v, n, ncols, lr, b1, b2, eps, c1, c2, (bf16 *)wb,
-                                                         (bf16 *)wtb, nrows);
     ORK_LAUNCH_CHECK();
     return 0;
 }

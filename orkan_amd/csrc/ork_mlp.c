@@ -16,24 +16,28 @@
 
 int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
                  float *c32, int ldc, const float *bias, float *pre, void *act);
-int ork_mlp_gemm_splitk(void *stream, const void *A, int lda, const void *B, int ldb, int M, int N, int K, int slices,
-                        float *work, float *c32, int ldc);
-int ork_mlp_transpose(void *stream, const void *in, void *out, int R, int Cc);
-int ork_mlp_to_bf16(void *stream, const float *in, void *out, long n);
+int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
+                     float *c32, int ldc, const float *bias, float *pre, void *act, void *actT, long ldt);
+int ork_mlp_stage_input(void *stream, const float *x, int rows, int M, int K, void *x16, void *x16t, long ldt);
 int ork_mlp_head_forward(void *stream, const void *h, const float *w, float b, int M, int K, float *y,
                          const float *target, float *dy, float *sqerr, int valid, float scale);
-int ork_mlp_head_backward(void *stream, const float *dy, const float *w, const float *pre, void *dpre, int M, int K);
-int ork_mlp_colsum(void *stream, const void *a, const float *s, int M, int K, float *out, float *part);
-int ork_mlp_sum(void *stream, const float *v, int n, float *out);
+int ork_mlp_head_backward_t(void *stream, const float *dy, const float *w, const float *pre, int M, int K, void *dpre,
+                            void *dpret, long ldt);
+int ork_mlp_weight_grads(void *stream, int nl, const void *const *xt, const void *const *dt, float *const *g,
+                         const int *K, int N, int rows, long ldt, int max_slices);
+int ork_mlp_colsums(void *stream, int count, const void *const *a, const float *const *s, float *const *out, int M,
+                    int K, float *part, const float *v0, const float *v1, float *vout);
 int ork_mlp_first_layer_graph(void *stream, const float *gf, int ng, const void *w, int N, float *u);
 int ork_mlp_first_layer_rows(void *stream, const float *angles, int na, long r0, int rows, int Mp, const float *u,
                              const void *wa, const float *bias, int N, void *act);
-int ork_mlp_adam(void *stream, float *w, const float *g, float *m, float *v, long n, int ncols, float lr, float b1,
-                 float b2, float eps, float c1, float c2, void *wb, void *wtb, int nrows);
+int ork_mlp_adam_all(void *stream, int count, float *const *w, const float *const *g, float *const *m, float *const *v,
+                     void *const *wb, void *const *wtb, const int *rows, const int *cols, float lr, float b1, float b2,
+                     float eps, float c1, float c2);
 
 #define MLP_MAX_LAYERS 4
 #define SPLITK_MAX 32   /* K slices of the weight-gradient products */
 #define TILE 128
+#define TPAD 64         /* row padding of the transposed operands: rows a power of two apart share memory channels */
 
 typedef struct {
     int K, N;
@@ -47,17 +51,17 @@ struct orkan_mlp {
     layer_t L[MLP_MAX_LAYERS];
     float *w_out, *g_out, *m_out, *v_out;   /* [hidden] */
     float b_out, mb_out, vb_out;
-    float *gb_out_d;                        /* device scalar: d loss / d b_out */
     /* activations (max_batch rows, padded to TILE) */
     float *x32;                 /* [M][in_dim] staged input */
     void *x16;                  /* bf16 [M][in_dim] */
     float *pre[MLP_MAX_LAYERS]; /* fp32 [M][hidden] */
     void *act[MLP_MAX_LAYERS];  /* bf16 [M][hidden] */
-    void *dpre, *dpre2;         /* bf16 [M][hidden] ping-pong */
-    void *tA, *tB;              /* bf16 transposes [hidden][M] */
-    float *y, *dy, *sq, *tgt, *scal;
-    float *colpart;             /* 64 x hidden partial column sums */
-    float *splitk;              /* SPLITK_MAX x max(in_dim, hidden) x hidden split-K partial products */
+    void *dpre[MLP_MAX_LAYERS]; /* bf16 [M][hidden] */
+    /* transposed operands of the weight gradients: the layers' inputs and dpre, bf16 [width][M + TPAD] */
+    void *in_t[MLP_MAX_LAYERS], *dpre_t[MLP_MAX_LAYERS];
+    float *y, *dy, *sq, *tgt;
+    float *scal;                /* sum of squared errors, d loss / d b_out */
+    float *colpart;             /* (nl + 1) x 64 x hidden partial column sums */
     float *gf_dev, *u1;         /* screening: graph features [in_dim], their layer-1 share [hidden] */
     long step;
 };
@@ -100,20 +104,19 @@ orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch
         q->pre[l] = dmalloc(M * H * 4, &err);
         q->act[l] = dmalloc(M * H * 2, &err);
     }
+    for (int l = 0; l < nhidden; ++l) {
+        q->dpre[l] = dmalloc(M * H * 2, &err);
+        q->in_t[l] = dmalloc((M + TPAD) * (size_t)q->L[l].K * 2, &err);
+        q->dpre_t[l] = dmalloc((M + TPAD) * H * 2, &err);
+    }
     q->w_out = dmalloc(H * 4, &err); q->g_out = dmalloc(H * 4, &err);
     q->m_out = dmalloc(H * 4, &err); q->v_out = dmalloc(H * 4, &err);
-    q->gb_out_d = dmalloc(16, &err);
     q->x32 = dmalloc(M * in_dim * 4, &err);
     q->x16 = dmalloc(M * in_dim * 2, &err);
-    q->dpre = dmalloc(M * H * 2, &err);
-    q->dpre2 = dmalloc(M * H * 2, &err);
-    q->tA = dmalloc(M * H * 2, &err);
-    q->tB = dmalloc(M * H * 2, &err);
     q->y = dmalloc(M * 4, &err); q->dy = dmalloc(M * 4, &err);
     q->sq = dmalloc(M * 4, &err); q->tgt = dmalloc(M * 4, &err);
     q->scal = dmalloc(64, &err);
-    q->colpart = dmalloc((size_t)64 * H * 4, &err);
-    q->splitk = dmalloc((size_t)SPLITK_MAX * (size_t)(in_dim > H ? in_dim : H) * H * 4, &err);
+    q->colpart = dmalloc((size_t)(nhidden + 1) * 64 * H * 4, &err);
     q->gf_dev = dmalloc((size_t)in_dim * 4, &err);
     q->u1 = dmalloc(H * 4, &err);
     if (err) {
@@ -130,7 +133,6 @@ orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch
     }
     (void)hipMemsetAsync(q->m_out, 0, H * 4, st);
     (void)hipMemsetAsync(q->v_out, 0, H * 4, st);
-    (void)hipMemsetAsync(q->x32, 0, M * in_dim * 4, st);
     (void)hipStreamSynchronize(st);
     return q;
 }
@@ -140,25 +142,37 @@ void orkan_mlp_destroy(orkan_mlp_t *q) {
     (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
     for (int l = 0; l < MLP_MAX_LAYERS; ++l) {
         layer_t *L = &q->L[l];
-        void *p[] = {L->w, L->g, L->m, L->v, L->b, L->gb, L->mb, L->vb, L->wb, L->wtb, q->pre[l], q->act[l]};
+        void *p[] = {L->w, L->g, L->m, L->v, L->b, L->gb, L->mb, L->vb, L->wb, L->wtb, q->pre[l], q->act[l],
+                     q->dpre[l], q->in_t[l], q->dpre_t[l]};
         for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
             if (p[i]) (void)hipFree(p[i]);
     }
-    void *p[] = {q->w_out, q->g_out, q->m_out, q->v_out, q->gb_out_d, q->x32, q->x16, q->dpre, q->dpre2,
-                 q->tA, q->tB, q->y, q->dy, q->sq, q->tgt, q->scal, q->colpart, q->splitk, q->gf_dev, q->u1};
+    void *p[] = {q->w_out, q->g_out, q->m_out, q->v_out, q->x32, q->x16, q->y, q->dy, q->sq, q->tgt, q->scal,
+                 q->colpart, q->gf_dev, q->u1};
     for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
         if (p[i]) (void)hipFree(p[i]);
     free(q);
 }
 
-static int refresh_bf16(orkan_mlp_t *q, int l) {
-    /* an Adam step with lr = 0 only rewrites the bf16 copies */
-    layer_t *L = &q->L[l];
-    hipStream_t st = (hipStream_t)ork_dev()->stream;
-    const long n = (long)L->K * L->N;
-    int e = (int)hipMemsetAsync(L->g, 0, (size_t)n * 4, st);
-    if (e) return e;
-    return ork_mlp_adam(st, L->w, L->g, L->m, L->v, n, L->N, 0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f, L->wb, L->wtb, L->K);
+/* one Adam launch over the weight matrices (without `all`: zero gradients) and, with `all`, every bias and the head */
+static int adam(orkan_mlp_t *q, int all, float lr, float b1, float b2, float eps, float c1, float c2) {
+    float *w[2 * MLP_MAX_LAYERS + 1], *m[2 * MLP_MAX_LAYERS + 1], *v[2 * MLP_MAX_LAYERS + 1];
+    const float *g[2 * MLP_MAX_LAYERS + 1];
+    void *wb[2 * MLP_MAX_LAYERS + 1], *wtb[2 * MLP_MAX_LAYERS + 1];
+    int rows[2 * MLP_MAX_LAYERS + 1], cols[2 * MLP_MAX_LAYERS + 1], n = 0;
+    for (int l = 0; l < q->nl; ++l, ++n) {
+        const layer_t *L = &q->L[l];
+        w[n] = L->w; g[n] = all ? L->g : NULL; m[n] = L->m; v[n] = L->v;
+        wb[n] = L->wb; wtb[n] = L->wtb; rows[n] = L->K; cols[n] = L->N;
+    }
+    for (int l = 0; all && l <= q->nl; ++l, ++n) {
+        const layer_t *L = &q->L[l < q->nl ? l : 0];
+        const int head = l == q->nl;
+        w[n] = head ? q->w_out : L->b; g[n] = head ? q->g_out : L->gb;
+        m[n] = head ? q->m_out : L->mb; v[n] = head ? q->v_out : L->vb;
+        wb[n] = wtb[n] = NULL; rows[n] = 1; cols[n] = q->hidden;
+    }
+    return ork_mlp_adam_all(ork_dev()->stream, n, w, g, m, v, wb, wtb, rows, cols, lr, b1, b2, eps, c1, c2);
 }
 
 /* W[l]: fp32 [K_l][hidden] row-major; b[l]: [hidden]; w_out: [hidden] */
@@ -171,8 +185,9 @@ int orkan_mlp_set_weights(orkan_mlp_t *q, const float *const *W, const float *co
         layer_t *L = &q->L[l];
         e |= (int)hipMemcpyAsync(L->w, W[l], (size_t)L->K * L->N * 4, hipMemcpyHostToDevice, st);
         e |= (int)hipMemcpyAsync(L->b, b[l], (size_t)L->N * 4, hipMemcpyHostToDevice, st);
-        if (!e) e = refresh_bf16(q, l);
     }
+    /* a step of zero gradients and lr = 0 only rewrites the bf16 copies (and clears the matrices' moments) */
+    if (!e) e = adam(q, 0, 0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f);
     if (!e) e = (int)hipMemcpyAsync(q->w_out, w_out, (size_t)q->hidden * 4, hipMemcpyHostToDevice, st);
     q->b_out = b_out;
     if (!e) e = (int)hipStreamSynchronize(st);
@@ -194,15 +209,20 @@ int orkan_mlp_get_weights(orkan_mlp_t *q, float *const *W, float *const *b, floa
     return e;
 }
 
-/* forward over rows [0, Mp) of the staged bf16 input; keep_pre stores the pre-activations */
-static int forward_rows(orkan_mlp_t *q, int Mp, int keep_pre) {
+/* forward over rows [0, Mp) of the staged bf16 input; for training it keeps the pre-activations and the transposed
+ * activations */
+static int forward_rows(orkan_mlp_t *q, int Mp, int training) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     const void *in = q->x16;
     int ld = q->in_dim;
     for (int l = 0; l < q->nl; ++l) {
         layer_t *L = &q->L[l];
-        int e = ork_mlp_gemm(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b,
-                             keep_pre ? q->pre[l] : NULL, q->act[l]);
+        int e;
+        if (training)
+            e = ork_mlp_gemm_mid(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, q->pre[l], q->act[l],
+                                 l + 1 < q->nl ? q->in_t[l + 1] : NULL, (long)Mp + TPAD);
+        else
+            e = ork_mlp_gemm(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, NULL, q->act[l]);
         if (e) return e;
         in = q->act[l];
         ld = L->N;
@@ -210,12 +230,11 @@ static int forward_rows(orkan_mlp_t *q, int Mp, int keep_pre) {
     return 0;
 }
 
-static int stage_input(orkan_mlp_t *q, const float *x, int rows, int Mp) {
+/* x (host or device) -> bf16, padding rows zero; for training also its transpose */
+static int stage_input(orkan_mlp_t *q, const float *x, int rows, int Mp, int training) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     int e = (int)hipMemcpyAsync(q->x32, x, (size_t)rows * q->in_dim * 4, hipMemcpyDefault, st);
-    if (!e && Mp > rows)
-        e = (int)hipMemsetAsync(q->x32 + (size_t)rows * q->in_dim, 0, (size_t)(Mp - rows) * q->in_dim * 4, st);
-    if (!e) e = ork_mlp_to_bf16(st, q->x32, q->x16, (long)Mp * q->in_dim);
+    if (!e) e = ork_mlp_stage_input(st, q->x32, rows, Mp, q->in_dim, q->x16, training ? q->in_t[0] : NULL, (long)Mp + TPAD);
     return e;
 }
 
@@ -226,7 +245,7 @@ int orkan_mlp_forward(orkan_mlp_t *q, int batch, const float *x, float *y) {
     for (int r0 = 0; r0 < batch; r0 += q->max_batch) {
         const int rows = batch - r0 < q->max_batch ? batch - r0 : q->max_batch;
         const int Mp = pad_rows(rows);
-        int e = stage_input(q, x + (size_t)r0 * q->in_dim, rows, Mp);
+        int e = stage_input(q, x + (size_t)r0 * q->in_dim, rows, Mp, 0);
         if (!e) e = forward_rows(q, Mp, 0);
         if (!e) e = ork_mlp_head_forward(st, q->act[q->nl - 1], q->w_out, q->b_out, Mp, q->hidden, q->y, NULL, NULL,
                                          NULL, rows, 1.0f);
@@ -266,79 +285,67 @@ int orkan_mlp_forward_candidates(orkan_mlp_t *q, const float *gf_host, int ng, c
     return e;
 }
 
-/* loss = mean squared error; gradients of all parameters into the g buffers */
-static int backward(orkan_mlp_t *q, int rows, const float *target, float *loss) {
+/* gradients of the mean squared error of the staged batch into the g buffers; the sum of squared errors and
+ * d loss / d b_out into scal[0] and scal[1].  12 launches (one step of 4096 rows of a 128 -> 512 -> 512 -> 512 -> 1
+ * network, host batches and every fourth step's weights included: 302 us against 545 with a launch per layer and operand, 37 in all) */
+static int backward(orkan_mlp_t *q, int rows, const float *target) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    const int Mp = pad_rows(rows), H = q->hidden;
+    const int Mp = pad_rows(rows), H = q->hidden, nl = q->nl;
+    const long ldt = (long)Mp + TPAD;
     int e = (int)hipMemcpyAsync(q->tgt, target, (size_t)rows * 4, hipMemcpyDefault, st);
     if (!e) e = forward_rows(q, Mp, 1);
-    if (!e) e = ork_mlp_head_forward(st, q->act[q->nl - 1], q->w_out, q->b_out, Mp, H, q->y, q->tgt, q->dy, q->sq,
+    if (!e) e = ork_mlp_head_forward(st, q->act[nl - 1], q->w_out, q->b_out, Mp, H, q->y, q->tgt, q->dy, q->sq,
                                      rows, 1.0f / (float)rows);
-    if (!e) e = ork_mlp_sum(st, q->sq, Mp, q->scal);          /* sum of squared errors */
-    if (!e) e = ork_mlp_sum(st, q->dy, Mp, q->gb_out_d);      /* d loss / d b_out */
-    if (!e) e = ork_mlp_colsum(st, q->act[q->nl - 1], q->dy, Mp, H, q->g_out, q->colpart);
-    if (!e) e = ork_mlp_head_backward(st, q->dy, q->w_out, q->pre[q->nl - 1], q->dpre, Mp, H);
-    void *dcur = q->dpre, *dnext = q->dpre2;
-    for (int l = q->nl - 1; l >= 0 && !e; --l) {
+    if (!e) e = ork_mlp_head_backward_t(st, q->dy, q->w_out, q->pre[nl - 1], Mp, H, q->dpre[nl - 1], q->dpre_t[nl - 1],
+                                        ldt);
+    /* dP_{l-1} = (dP_l W_l^T) * gelu'(pre_{l-1}) */
+    for (int l = nl - 1; l > 0 && !e; --l) {
         layer_t *L = &q->L[l];
-        const void *xin = l == 0 ? q->x16 : q->act[l - 1];
-        /* dW_l = X^T dP: transposes to [K][M] and [N][M], then C = A B^T over the batch */
-        e = ork_mlp_transpose(st, xin, q->tA, Mp, L->K);
-        if (!e) e = ork_mlp_transpose(st, dcur, q->tB, Mp, L->N);
-        if (!e) {
-            /* K = the batch (thousands) but only (K_l / 128) x (N / 128) output tiles: split the batch
-             * into up to SPLITK_MAX slices of >= 128 rows until ~512 workgroups run */
-            const int tiles = (L->K / 128) * (L->N / 128);
-            int slices = 1;
-            while (slices < SPLITK_MAX && tiles * slices < 512 && Mp % (slices * 2 * 128) == 0) slices *= 2;
-            e = slices > 1 ? ork_mlp_gemm_splitk(st, q->tA, Mp, q->tB, Mp, L->K, L->N, Mp, slices, q->splitk, L->g, L->N)
-                           : ork_mlp_gemm(st, 0, q->tA, Mp, q->tB, Mp, L->K, L->N, Mp, L->g, L->N, NULL, NULL, NULL);
-        }
-        if (!e) e = ork_mlp_colsum(st, dcur, NULL, Mp, L->N, L->gb, q->colpart);
-        if (!e && l > 0) {
-            /* dP_{l-1} = (dP_l W_l^T) * gelu'(pre_{l-1}) */
-            e = ork_mlp_gemm(st, 2, dcur, L->N, L->wb, L->N, Mp, L->K, L->N, NULL, L->K, NULL, q->pre[l - 1], dnext);
-            void *t = dcur;
-            dcur = dnext;
-            dnext = t;
-        }
+        e = ork_mlp_gemm_mid(st, 2, q->dpre[l], L->N, L->wb, L->N, Mp, L->K, L->N, NULL, L->K, NULL, q->pre[l - 1],
+                             q->dpre[l - 1], q->dpre_t[l - 1], ldt);
     }
-    if (!e && loss) {
-        float s = 0.0f;
-        e = (int)hipMemcpyAsync(&s, q->scal, 4, hipMemcpyDeviceToHost, st);
-        if (!e) e = (int)hipStreamSynchronize(st);
-        *loss = s / (float)rows;
+    const void *xt[MLP_MAX_LAYERS], *dt[MLP_MAX_LAYERS], *cols[MLP_MAX_LAYERS + 1];
+    const float *scale[MLP_MAX_LAYERS + 1];
+    float *gw[MLP_MAX_LAYERS], *gc[MLP_MAX_LAYERS + 1];
+    int K[MLP_MAX_LAYERS];
+    for (int l = 0; l < nl; ++l) {
+        xt[l] = q->in_t[l];
+        dt[l] = q->dpre_t[l];
+        gw[l] = q->L[l].g;
+        K[l] = q->L[l].K;
+        cols[l] = q->dpre[l];
+        scale[l] = NULL;
+        gc[l] = q->L[l].gb;
     }
+    cols[nl] = q->act[nl - 1];
+    scale[nl] = q->dy;
+    gc[nl] = q->g_out;
+    /* dW_l = X_l^T dP_l */
+    if (!e) e = ork_mlp_weight_grads(st, nl, xt, dt, gw, K, H, Mp, ldt, SPLITK_MAX);
+    if (!e) e = ork_mlp_colsums(st, nl + 1, cols, scale, gc, Mp, H, q->colpart, q->sq, q->dy, q->scal);
     return e;
 }
 
 int orkan_mlp_train_step(orkan_mlp_t *q, int batch, const float *x, const float *target, float lr, float *loss) {
     if (!q || batch <= 0 || batch > q->max_batch) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    const int Mp = pad_rows(batch);
-    int e = stage_input(q, x, batch, Mp);
-    if (!e) e = backward(q, batch, target, loss);
+    int e = stage_input(q, x, batch, pad_rows(batch), 1);
+    if (!e) e = backward(q, batch, target);
     if (e) return e;
     q->step += 1;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float c1 = 1.0f - powf(b1, (float)q->step), c2 = 1.0f - powf(b2, (float)q->step);
-    for (int l = 0; l < q->nl && !e; ++l) {
-        layer_t *L = &q->L[l];
-        e = ork_mlp_adam(st, L->w, L->g, L->m, L->v, (long)L->K * L->N, L->N, lr, b1, b2, eps, c1, c2, L->wb, L->wtb,
-                         L->K);
-        if (!e) e = ork_mlp_adam(st, L->b, L->gb, L->mb, L->vb, L->N, L->N, lr, b1, b2, eps, c1, c2, NULL, NULL, 1);
-    }
-    if (!e) e = ork_mlp_adam(st, q->w_out, q->g_out, q->m_out, q->v_out, q->hidden, q->hidden, lr, b1, b2, eps, c1,
-                             c2, NULL, NULL, 1);
-    if (!e) {
-        float gb = 0.0f;
-        e = (int)hipMemcpyAsync(&gb, q->gb_out_d, 4, hipMemcpyDeviceToHost, st);
-        if (!e) e = (int)hipStreamSynchronize(st);
-        q->mb_out = b1 * q->mb_out + (1 - b1) * gb;
-        q->vb_out = b2 * q->vb_out + (1 - b2) * gb * gb;
-        q->b_out -= lr * (q->mb_out / c1) / (sqrtf(q->vb_out / c2) + eps);
-    }
-    return e;
+    e = adam(q, 1, lr, b1, b2, eps, c1, c2);
+    float s[2] = {0.0f, 0.0f};
+    if (!e) e = (int)hipMemcpyAsync(s, q->scal, sizeof(s), hipMemcpyDeviceToHost, st);
+    if (!e) e = (int)hipStreamSynchronize(st);
+    if (e) return e;
+    const float gb = s[1];
+    q->mb_out = b1 * q->mb_out + (1 - b1) * gb;
+    q->vb_out = b2 * q->vb_out + (1 - b2) * gb * gb;
+    q->b_out -= lr * (q->mb_out / c1) / (sqrtf(q->vb_out / c2) + eps);
+    if (loss) *loss = s[0] / (float)batch;
+    return 0;
 }
 
 /* gradients without an update (for checking against a CPU computation) */
@@ -346,16 +353,19 @@ int orkan_mlp_grads(orkan_mlp_t *q, int batch, const float *x, const float *targ
                     float *const *db, float *dw_out, float *db_out, float *loss) {
     if (!q || batch <= 0 || batch > q->max_batch) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    int e = stage_input(q, x, batch, pad_rows(batch));
-    if (!e) e = backward(q, batch, target, loss);
+    int e = stage_input(q, x, batch, pad_rows(batch), 1);
+    if (!e) e = backward(q, batch, target);
     for (int l = 0; l < q->nl && !e; ++l) {
         if (dW && dW[l]) e |= (int)hipMemcpyAsync(dW[l], q->L[l].g, (size_t)q->L[l].K * q->L[l].N * 4,
                                                    hipMemcpyDeviceToHost, st);
         if (db && db[l]) e |= (int)hipMemcpyAsync(db[l], q->L[l].gb, (size_t)q->L[l].N * 4, hipMemcpyDeviceToHost, st);
     }
     if (!e && dw_out) e = (int)hipMemcpyAsync(dw_out, q->g_out, (size_t)q->hidden * 4, hipMemcpyDeviceToHost, st);
-    if (!e && db_out) e = (int)hipMemcpyAsync(db_out, q->gb_out_d, 4, hipMemcpyDeviceToHost, st);
+    float s[2] = {0.0f, 0.0f};
+    if (!e) e = (int)hipMemcpyAsync(s, q->scal, sizeof(s), hipMemcpyDeviceToHost, st);
     if (!e) e = (int)hipStreamSynchronize(st);
+    if (!e && db_out) *db_out = s[1];
+    if (!e && loss) *loss = s[0] / (float)batch;
     return e;
 }
 

@@ -155,3 +155,29 @@ def test_forward_candidates_matches_forward(ncand, max_batch):
     lib.orkan_dev_free(dang)
     lib.orkan_dev_free(ydev)
     m.close()
+
+
+@pytest.mark.parametrize("rows,hidden,layers", [(1, 128, 1), (127, 128, 2), (129, 256, 3), (384, 512, 4), (1024, 384, 2)])
+def test_gradients_at_tile_edges(rows, hidden, layers):
+    """One row, one row to each side of the padding, an odd number of 128-row panels (the batch then is one slice of
+    the weight gradients), 1 to 4 layers, and a width that is no power of two.  Bounds as in
+    test_forward_backward_match_oracle: bf16 rounding of activations and gradients (2^-9 per value)."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(rows + hidden)
+    W, b, wo, bo = mlp_np.init_params(rng, 128, hidden, layers)
+    W, wo = [w.astype(np.float32) for w in W], wo.astype(np.float32)
+    b = [(0.1 * rng.standard_normal(hidden)).astype(np.float32) for _ in b]
+    m = surrogate.Mlp(lib, hidden=hidden, layers=layers, max_batch=rows)
+    m.set_weights(W, b, wo, 0.25)
+    x = rng.standard_normal((rows, 128)).astype(np.float32)
+    t = rng.standard_normal(rows).astype(np.float32)
+    params = ([w.astype(np.float64) for w in W], [v.astype(np.float64) for v in b], wo.astype(np.float64), 0.25)
+    loss, (dW, db, dwo, dbo) = m.grads(x, t)
+    lref, (rW, rb, rwo, rbo) = mlp_np.loss_and_grads(params, x.astype(np.float64), t.astype(np.float64), exact=False)
+    assert abs(loss - lref) <= 1e-2 * max(lref, 1e-3)
+    for l in range(layers):
+        assert np.linalg.norm(dW[l] - rW[l]) <= 2e-2 * np.linalg.norm(rW[l]), l
+        assert np.linalg.norm(db[l] - rb[l]) <= 2e-2 * np.linalg.norm(rb[l]), l
+    assert np.linalg.norm(dwo - rwo) <= 2e-2 * np.linalg.norm(rwo)
+    assert abs(dbo - rbo) <= 1e-2 * max(1.0, abs(rbo))
+    m.close()
