@@ -30,6 +30,10 @@ int ork_mlp_colsums(void *stream, int count, const void *const *a, const float *
 int ork_mlp_first_layer_graph(void *stream, const float *gf, int ng, const void *w, int N, float *u);
 int ork_mlp_first_layer_rows(void *stream, const float *angles, int na, long r0, int rows, int Mp, const float *u,
                              const void *wa, const float *bias, int N, void *act);
+int ork_mlp_screen_ok(int na, int hidden, int nl);
+int ork_mlp_screen(void *stream, const float *gf, int ng, const void *w0, const void *const *wt, void *wpk, float *u,
+                   const float *const *bias, int nl, int H, const float *w_out, float b_out, const float *angles,
+                   long ncand, float *y);
 int ork_mlp_adam_all(void *stream, int count, float *const *w, const float *const *g, float *const *m, float *const *v,
                      void *const *wb, void *const *wtb, const int *rows, const int *cols, float lr, float b1, float b2,
                      float eps, float c1, float c2);
@@ -63,6 +67,7 @@ struct orkan_mlp {
     float *scal;                /* sum of squared errors, d loss / d b_out */
     float *colpart;             /* (nl + 1) x 64 x hidden partial column sums */
     float *gf_dev, *u1;         /* screening: graph features [in_dim], their layer-1 share [hidden] */
+    void *wpk;                  /* screening: the later layers' weights in fragment order */
     long step;
 };
 
@@ -119,6 +124,7 @@ orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch
     q->colpart = dmalloc((size_t)(nhidden + 1) * 64 * H * 4, &err);
     q->gf_dev = dmalloc((size_t)in_dim * 4, &err);
     q->u1 = dmalloc(H * 4, &err);
+    if (ork_mlp_screen_ok(8, hidden, nhidden)) q->wpk = dmalloc((size_t)(nhidden - 1) * H * H * 2, &err);
     if (err) {
         orkan_mlp_destroy(q);
         return NULL;
@@ -148,7 +154,7 @@ void orkan_mlp_destroy(orkan_mlp_t *q) {
             if (p[i]) (void)hipFree(p[i]);
     }
     void *p[] = {q->w_out, q->g_out, q->m_out, q->v_out, q->x32, q->x16, q->y, q->dy, q->sq, q->tgt, q->scal,
-                 q->colpart, q->gf_dev, q->u1};
+                 q->colpart, q->gf_dev, q->u1, q->wpk};
     for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
         if (p[i]) (void)hipFree(p[i]);
     free(q);
@@ -255,10 +261,10 @@ int orkan_mlp_forward(orkan_mlp_t *q, int batch, const float *x, float *y) {
     return (int)hipStreamSynchronize(st);
 }
 
-/* Screening: rows r = 0..ncand-1 are [gf (ng floats), angles_dev[r] (in_dim - ng floats)].
- * The graph features' share of layer 1 is computed once (first_layer_graph); each
- * chunk then builds layer 1's activations from the angles alone and runs the
- * remaining layers.  y_dev receives ncand predictions. */
+/* Screening: rows r = 0..ncand-1 are [gf (ng floats), angles_dev[r] (in_dim - ng floats)]; y_dev receives ncand
+ * predictions.  The graph features' share of layer 1 is computed once.  8 angles (p = 4) and a width of 128, 256 or 512
+ * run through every layer in one kernel (k_screen.hip: a tile of activations and two workgroups fit a CU's LDS, the
+ * accumulators its registers); other shapes go layer by layer, in chunks of max_batch rows.  Both give the same bits. */
 int orkan_mlp_forward_candidates(orkan_mlp_t *q, const float *gf_host, int ng, const float *angles_dev, long ncand,
                                  float *y_dev) {
     if (!q || ng <= 0 || ng >= q->in_dim || ncand < 0) return (int)hipErrorInvalidValue;
@@ -266,6 +272,18 @@ int orkan_mlp_forward_candidates(orkan_mlp_t *q, const float *gf_host, int ng, c
     const int na = q->in_dim - ng, H = q->hidden;
     const layer_t *L0 = &q->L[0];
     int e = (int)hipMemcpyAsync(q->gf_dev, gf_host, (size_t)ng * 4, hipMemcpyHostToDevice, st);
+    if (!e && ork_mlp_screen_ok(na, H, q->nl)) {
+        const void *wt[MLP_MAX_LAYERS];
+        const float *bias[MLP_MAX_LAYERS];
+        for (int l = 0; l < q->nl; ++l) {
+            bias[l] = q->L[l].b;
+            if (l) wt[l - 1] = q->L[l].wtb;
+        }
+        e = ork_mlp_screen(st, q->gf_dev, ng, L0->wb, wt, q->wpk, q->u1, bias, q->nl, H, q->w_out, q->b_out, angles_dev,
+                           ncand, y_dev);
+        if (!e) e = (int)hipStreamSynchronize(st);
+        return e;
+    }
     if (!e) e = ork_mlp_first_layer_graph(st, q->gf_dev, ng, L0->wb, H, q->u1);
     for (long r0 = 0; r0 < ncand && !e; r0 += q->max_batch) {
         const int rows = (int)(ncand - r0 < q->max_batch ? ncand - r0 : q->max_batch);

@@ -181,3 +181,34 @@ def test_gradients_at_tile_edges(rows, hidden, layers):
     assert np.linalg.norm(dwo - rwo) <= 2e-2 * np.linalg.norm(rwo)
     assert abs(dbo - rbo) <= 1e-2 * max(1.0, abs(rbo))
     m.close()
+
+
+@pytest.mark.parametrize("hidden,layers", [(128, 1), (128, 3), (256, 2), (512, 3), (512, 4), (384, 3)])
+@pytest.mark.parametrize("ncand", [1, 63, 65, 1000])
+def test_screening_equals_the_assembled_rows(hidden, layers, ncand):
+    """Every width and depth of the one-kernel screening forward (and a width it leaves to the layer kernels), at and
+    beside its 64-row tiles, against the CPU oracle on the assembled rows; nothing written past the last candidate.
+    Bound as in test_forward_candidates_matches_forward."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(hidden + layers + ncand)
+    W, b, wo, bo = mlp_np.init_params(rng, 128, hidden, layers)
+    W, wo = [w.astype(np.float32) for w in W], wo.astype(np.float32)
+    b = [(0.1 * rng.standard_normal(hidden)).astype(np.float32) for _ in b]
+    m = surrogate.Mlp(lib, hidden=hidden, layers=layers, max_batch=256)
+    m.set_weights(W, b, wo, 0.25)
+    gf = surrogate.graph_features(rng.uniform(0, 1, 60))
+    ang = rng.uniform(0, 1, (ncand, 8)).astype(np.float32)
+    x = np.concatenate([np.broadcast_to(gf, (ncand, 120)), ang], 1).astype(np.float32)
+    params = ([w.astype(np.float64) for w in W], [v.astype(np.float64) for v in b], wo.astype(np.float64), 0.25)
+    y_ref, _, _ = mlp_np.forward(params, x.astype(np.float64), exact=False)
+    dang = upload(lib, ang)
+    guard = np.full(ncand + 1, 12345.0, np.float32)
+    ydev = upload(lib, guard)
+    m.forward_candidates(gf, dang, ncand, ydev)
+    y = np.empty(ncand + 1, np.float32)
+    assert lib.orkan_copy_to_host(y.ctypes.data, ydev, y.nbytes) == 0
+    assert y[ncand] == 12345.0
+    assert np.abs(y[:ncand] - y_ref).max() <= 2e-3 * max(1.0, np.abs(y_ref).max())
+    for p in (dang, ydev):
+        lib.orkan_dev_free(p)
+    m.close()
