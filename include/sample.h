@@ -25,8 +25,9 @@ typedef struct {
 /* S (caller-allocated, K x K column-major, K = channels[lstar].n_ops) = the sample matrix at the
  * channel of 0-based index lstar.  iota: a PURE complex128 state, CONSUMED (it ends holding
  * K_{lstar-1} ... K_1 |iota>; pass a copy to keep it).  obs: 2^n doubles (host or device).
- * workspace_bytes caps the state vectors the call holds besides iota: two for the linear
- * combinations and 2B leaves (B = the leaf block, at most 64), so at least 4 x 16 x 2^n bytes.
+ * workspace_bytes caps the state vectors the call holds besides iota: 2B leaves (B = the leaf block,
+ * at most 64; B where it holds every leaf) and, for the linear combinations, two vectors or as many
+ * pairs, at most B, as the rest of the cap allows: at least 4 x 16 x 2^n bytes.
  * Both triangles are filled, S_ba = conj(S_ab) exactly, the diagonal is real.  The result does not
  * depend on the block size.  Returns QS_OK, QS_ERR_NULL, QS_ERR_TYPE (iota not PURE complex128),
  * QS_ERR_PARAM (lstar out of range, a channel without operations or, other than at lstar, without

@@ -97,3 +97,56 @@ def test_sample_matrix_against_brute_force(sizes, lstar):
     assert np.all(np.diag(S_big).imag == 0.0)
     assert np.abs(pre - pre_want).max() <= 1e-12                # iota consumed: holds the prefix
     del keep
+
+
+@pytest.mark.parametrize("n", [1, 3, 4, 7, 10])
+@pytest.mark.parametrize("K,others", [(1, (1,)), (2, (3,)), (16, (2, 1)), (17, (2,)), (33, (4, 2)), (64, (2,)),
+                                      (65, (3,)), (81, (1,))])
+def test_sample_matrix_at_tile_and_block_edges(n, K, others):
+    """Leaf counts at and beside the 16-vector tiles and the 64-leaf block, combinations of 1 to 4 operations, states
+    below and at the product's 16-amplitude step; every workspace from the smallest to one that holds all leaves and
+    their scratch gives the same bits.  Bound: sums of 2^n products of amplitudes whose norms multiply to `scale`, every
+    gate and product rounded at 2^-53 a few times: 1e-12 of the scale."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(1000 * n + K)
+    names = [("rx", True), ("ry", True), ("rz", True), ("h", False), ("x", False)]
+    sizes = [others[0], K] + list(others)
+    table, chans, keep = [], [], []
+    for l, m in enumerate(sizes):
+        cbs, mats = [], []
+        for _ in range(m):
+            name, ang = names[rng.integers(len(names))]
+            q, th = int(rng.integers(n)), float(rng.uniform(0, 6)) if ang else None
+            fn = getattr(lib, name)
+            cbs.append(_ffi.QOP(lambda st, fn=fn, a=((q,) if th is None else (q, th)): fn(st, *a)))
+            mats.append(gate_full(name, (q,), n, th or 0.0))
+        w = (rng.standard_normal(m) + 1j * rng.standard_normal(m)) / np.sqrt(m)
+        arr, wa = (_ffi.QOP * m)(*cbs), np.ascontiguousarray(w, dtype=np.complex128)
+        keep += [cbs, arr, wa]
+        table.append(_ffi.AnsatzChannelT(m, arr, wa.ctypes.data))
+        chans.append((None, None, mats, w))
+    tab = (_ffi.AnsatzChannelT * len(table))(*table)
+    psi0, obs = random_psi(n, rng), rng.uniform(-1, 1, 1 << n)
+    psi = sum(wm * (U @ psi0) for U, wm in zip(chans[0][2], chans[0][3]))
+    leaves = []
+    for U in chans[1][2]:
+        v = U @ psi
+        for c in chans[2:]:
+            v = sum(wm * (A @ v) for A, wm in zip(c[2], c[3]))
+        leaves.append(v)
+    M = np.array(leaves)
+    want = (M.conj() * obs) @ M.T
+    got = []
+    vec = 16 << n
+    for budget in (4 * vec, 7 * vec, (2 * K + 3) * vec, 1 << 28):
+        st = _ffi.StateT(PURE, None, 0)
+        lib.state_init(C.byref(st), n, None)
+        assert lib.orkan_state_upload(C.byref(st), psi0.ctypes.data) == 0
+        S = np.zeros((K, K), np.complex128)
+        assert lib.sample_matrix(C.byref(st), obs.ctypes.data, tab, len(sizes), 1, budget, S.ctypes.data) == 0
+        lib.state_free(C.byref(st))
+        got.append(S.T.copy())      # column-major
+    scale = max(1.0, np.abs(want).max())
+    assert np.abs(got[0] - want).max() <= 1e-12 * scale
+    assert all(np.array_equal(g, got[0]) for g in got[1:])
+    assert np.array_equal(got[0], got[0].conj().T) and not np.diagonal(got[0]).imag.any()
