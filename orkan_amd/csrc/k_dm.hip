@@ -387,6 +387,145 @@ __global__ __launch_bounds__(DM_THREADS) void dm_group_kernel(S *__restrict__ rh
     }
 }
 
+// ---- two-qubit superoperators and unitaries on groups of 32 x 32 entries -------------------------------
+// The groups, their ownership and the arithmetic are those of dm_group_kernel; the shape is another.  Four waves share
+// a group.  Each thread loads its 4 entries at once (one after the other before); every wave then holds all 64 blocks of
+// 4 x 4, one per lane, and forms one row of each result, so no wave is idle and no block's 16 results wait for one lane.
+// Group tiles have 64, 256 or 1024 entries (LB 3, 4, 5), so which tile a run of 64 entries belongs to, where that tile
+// lies and whether it is stored or read from its mirror are the same for all lanes: scalar work, and a lane adds one
+// offset of its own.  The superoperator's 256 entries come as scalar operands (scalar loads of a 4 KB array: rho is not
+// aliased), where LDS broadcasts cost a 16 B read per complex product.
+// 12 qubits, tiled: 48 us per channel_2q (76 through dm_group_kernel), 43 us per two_from_mat (95), against 42 for the
+// entries read and written once; 13 qubits 180-213 us (305-350) and 174-212 (358-417) against 166; 8 qubits 5.5 us (7.4)
+// and 5.7 (10).  One wave per group: channel_2q 64 us on 12 qubits, 10-12 on 8; two waves 57 and 8.4.
+// Groups smaller than 32 x 32 (states below 5 qubits, small storage tiles) stay with dm_group_kernel.
+struct PairOp {
+    int lbit[2];    // LDS coordinate bit of gate argument j
+    int srt[2];     // ... ascending
+    cd m[16];       // DENSE: 4x4 row-major
+};
+constexpr int PAIR_W = 4;   // waves per group
+
+template <typename S, int LAYOUT, int OP, int LB, int NTA>
+__global__ __launch_bounds__(64 * PAIR_W) void dm_pair_kernel(S *__restrict__ rho, DmPlan p, PairOp op,
+                                                     const cd *__restrict__ s2) {
+    constexpr int G = LW_MAX - LB, NT = 1 << G, B = 1 << LB, W = PAIR_W, PER = W_MAX * W_MAX / 64 / W;
+    __shared__ cd lds[W_MAX * LDS_STRIDE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    u64 R, C;
+    group_rc(p, blockIdx.x, R, C);
+    R = __builtin_amdgcn_readfirstlane((unsigned)R);   // group indexes are below 2^31
+    C = __builtin_amdgcn_readfirstlane((unsigned)C);
+    const u64 TRb = ins0k(R, p.gpos, G), TCb = ins0k(C, p.gpos, G);
+    const bool diag_group = R == C;
+    // entry u of the lane, of the group's 16 runs of 64 entries the run wave + W u: its group tile (ti, tj), its slow and
+    // fast position in the tile
+    constexpr int USH = 2 * LB - 6;
+    const auto slow = [&](int u) { return (lane >> LB) + (((wave + W * u) & ((1 << USH) - 1)) << (6 - LB)); };
+    const auto ti = [&](int u) { return ((wave + W * u) >> USH) >> G; };
+    const auto tj = [&](int u) { return ((wave + W * u) >> USH) & (NT - 1); };
+    const int fast = lane & (B - 1);
+    // offset of entry (slow, fast) of the stored virtual tile (TR, TC)
+    const auto offset = [&](u64 TR, u64 TC, int sl) -> u64 {
+        if constexpr (LAYOUT == ORK_TILED) {
+            return tiled_off(p.L, TR * B, TC * B) + (u64)(unsigned)((sl << p.L) + fast);
+        } else {
+            // column c0 + sl starts sl (2 dim - 2 c0 + 1 - sl) / 2 entries after column c0; its diagonal is row c0 + sl
+            const u64 c0 = TC * B, d = 2 * p.dim - 2 * c0 + 1;
+            return packed_off(p.dim, TR * B, c0) + (((u64)(unsigned)sl * (d - (unsigned)sl)) >> 1) + (u64)fast - (u64)sl;
+        }
+    };
+
+    S raw[PER];
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = ti(u), j = tj(u);
+        const u64 TR = TRb | spread_bits(i, p.gpos, G), TC = TCb | spread_bits(j, p.gpos, G);
+        // a tile that is not stored is read from its mirror (TC, TR), in that tile's memory order
+        const bool st = tile_stored<LAYOUT>(p, TR, TC);
+        raw[u] = ldr<NTA>(rho + offset(st ? TR : TC, st ? TC : TR, slow(u)));
+    }
+    if constexpr (sizeof(S) == 8) {
+#pragma unroll
+        for (int u = 0; u < PER; ++u) hold(raw[u]);
+    }
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = ti(u), j = tj(u);
+        const u64 TR = TRb | spread_bits(i, p.gpos, G), TC = TCb | spread_bits(j, p.gpos, G);
+        const int sr = LAYOUT == ORK_TILED ? slow(u) : fast, sc = LAYOUT == ORK_TILED ? fast : slow(u);
+        const cd v = to_cd(raw[u]);
+        if (tile_stored<LAYOUT>(p, TR, TC)) {
+            if (LAYOUT == ORK_PACKED && TR == TC) {
+                // a diagonal tile holds its lower half only
+                if (sr >= sc) lds[(i * B + sr) * LDS_STRIDE + j * B + sc] = v;
+                if (sr > sc) lds[(i * B + sc) * LDS_STRIDE + j * B + sr] = cconj(v);
+            } else {
+                lds[(i * B + sr) * LDS_STRIDE + j * B + sc] = v;
+            }
+        } else {
+            lds[(i * B + sc) * LDS_STRIDE + j * B + sr] = cconj(v);
+        }
+    }
+    __syncthreads();
+
+    // lane: block (lane >> 3, lane & 7)
+    const int x0 = (int)ins0k((u64)(lane >> 3), op.srt, 2), y0 = (int)ins0k((u64)(lane & 7), op.srt, 2);
+    int xo[4], yo[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        xo[a] = (x0 | (int)spread_bits(a, op.lbit, 2)) * LDS_STRIDE;
+        yo[a] = y0 | (int)spread_bits(a, op.lbit, 2);
+    }
+    cd v[16];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) v[a * 4 + c] = lds[xo[a] + yo[c]];
+    __syncthreads();
+    // wave w: row w of every block's result
+    const int xr = (x0 | (int)spread_bits(wave, op.lbit, 2)) * LDS_STRIDE;
+    if constexpr (OP == ORK_DM_SOP2) {
+        const cd *__restrict__ sw = s2 + wave * 64;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            cd o = cmk(0.0, 0.0);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) cfma(o, sw[a * 16 + j], v[j]);
+            lds[xr + yo[a]] = o;
+        }
+    } else {
+        // U rho by rows, then . U^dagger by columns
+        const cd *u = op.m + wave * 4;
+        cd t[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            t[c] = cmk(0.0, 0.0);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) cfma(t[c], u[b], v[b * 4 + c]);
+        }
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            cd o = cmk(0.0, 0.0);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) cfma(o, t[b], cconj(op.m[a * 4 + b]));
+            lds[xr + yo[a]] = o;
+        }
+    }
+    __syncthreads();
+
+#pragma unroll
+    for (int u = 0; u < PER; ++u) {
+        const int i = ti(u), j = tj(u);
+        const u64 TR = TRb | spread_bits(i, p.gpos, G), TC = TCb | spread_bits(j, p.gpos, G);
+        const int sl = slow(u), sr = LAYOUT == ORK_TILED ? sl : fast, sc = LAYOUT == ORK_TILED ? fast : sl;
+        if (tile_stored<LAYOUT>(p, TR, TC) && !(LAYOUT == ORK_PACKED && TR == TC && sr < sc))
+            stx<NTA>(rho + offset(TR, TC, sl), lds[(i * B + sr) * LDS_STRIDE + j * B + sc]);
+        if (!diag_group && tile_stored<LAYOUT>(p, TC, TR))
+            stx<NTA>(rho + offset(TC, TR, sl), cconj(lds[(i * B + sc) * LDS_STRIDE + j * B + sr]));
+    }
+}
+
 // ---- tiled layout, 1-qubit superoperator, streamed ---------------------------------------
 // The quad (r0, r1) x (c0, c1), r1 = r0 | 2^q, c1 = c0 | 2^q, goes from HBM to
 // registers and back with no LDS round trip wherever its four entries are
@@ -1729,6 +1868,45 @@ int launch_group(hipStream_t st, void *rho, DmPlan p, int opk, const DmOp &op) {
     return 0;
 }
 
+template <typename S, int LAYOUT, int OP, int LB>
+void launch_pair_lb(hipStream_t st, void *rho, const DmPlan &p, const PairOp &op, const cd *s2, bool nt) {
+    const unsigned grid = (unsigned)p.ngroups;
+    if (nt) dm_pair_kernel<S, LAYOUT, OP, LB, 1><<<grid, 64 * PAIR_W, 0, st>>>((S *)rho, p, op, s2);
+    else dm_pair_kernel<S, LAYOUT, OP, LB, 0><<<grid, 64 * PAIR_W, 0, st>>>((S *)rho, p, op, s2);
+}
+
+// two-qubit SOP2 and DENSE on groups of 32 x 32 entries; order and nontemporal accesses as the tile groups
+bool pair_ok(const DmPlan &p, int opk, int k) {
+    return k == 2 && (opk == ORK_DM_SOP2 || opk == ORK_DM_DENSE) && p.LW == LW_MAX && p.LB >= 3 &&
+           p.ngroups <= ((u64)1 << 30);
+}
+template <typename S, int LAYOUT>
+int launch_pair_op(hipStream_t st, void *rho, DmPlan p, int opk, const DmOp &op) {
+    const Shape sh = g_group_shape[LAYOUT == ORK_TILED ? 1 : 0];
+    p.xcd = sh.xcd;
+    p.col = sh.col;
+    const u64 tl = p.dim >> p.L;
+    const bool nt = LAYOUT == ORK_TILED && sh.nt && ((u64)sizeof(S) << p.LB) >= 128 &&
+                    ((tl * (tl + 1) / 2) << (2 * p.L)) * sizeof(S) >= ork_nt_min_bytes();
+    PairOp po;
+    for (int j = 0; j < 2; ++j) {
+        po.lbit[j] = op.lbit[j];
+        po.srt[j] = op.srt[j];
+    }
+    for (int i = 0; i < 16; ++i) po.m[i] = op.m[i];
+#define ORK_PAIR_LAUNCH(OPC)                                                             \
+    do {                                                                                 \
+        if (p.LB == 5) launch_pair_lb<S, LAYOUT, OPC, 5>(st, rho, p, po, op.s2, nt);     \
+        else if (p.LB == 4) launch_pair_lb<S, LAYOUT, OPC, 4>(st, rho, p, po, op.s2, nt); \
+        else launch_pair_lb<S, LAYOUT, OPC, 3>(st, rho, p, po, op.s2, nt);               \
+    } while (0)
+    if (opk == ORK_DM_SOP2) ORK_PAIR_LAUNCH(ORK_DM_SOP2);
+    else ORK_PAIR_LAUNCH(ORK_DM_DENSE);
+#undef ORK_PAIR_LAUNCH
+    ORK_LAUNCH_CHECK();
+    return 0;
+}
+
 // streamed tiled superoperator; shape [q < L, q >= L].  A later sweep of every target (h on 14 qubits)
 // moved the complex128 defaults to XCD runs of 32 workgroups under an 80 KB cap for in-tile targets 3-4
 // (6.74 against 6.58 TB/s) and a 64 KB cap for the split tile quads (6.36 against 6.23).  Measured on a 14-qubit density matrix
@@ -2269,6 +2447,13 @@ extern "C" int ork_dm_group(void *stream, int prec, int layout, int log_tile, vo
         log_tile >= 1)
         return prec == ORK_F32 ? launch_stream<float2>(st, rho, log_tile, n, m->qs[0], op)
                                : launch_stream<double2>(st, rho, log_tile, n, m->qs[0], op);
+    if (pair_ok(p, opk, k)) {
+        if (prec == ORK_F32)
+            return layout == ORK_PACKED ? launch_pair_op<float2, ORK_PACKED>(st, rho, p, opk, op)
+                                        : launch_pair_op<float2, ORK_TILED>(st, rho, p, opk, op);
+        return layout == ORK_PACKED ? launch_pair_op<double2, ORK_PACKED>(st, rho, p, opk, op)
+                                    : launch_pair_op<double2, ORK_TILED>(st, rho, p, opk, op);
+    }
     if (prec == ORK_F32)
         return layout == ORK_PACKED ? launch_group<float2, ORK_PACKED>(st, rho, p, opk, op)
                                     : launch_group<float2, ORK_TILED>(st, rho, p, opk, op);

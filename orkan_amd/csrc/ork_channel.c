@@ -14,6 +14,7 @@
 #include "orkan_backend.h"
 
 #include <string.h>
+#include <hip/hip_runtime_api.h>
 
 #define CV(cond, msg) ORK_VALIDATE("channel", cond, msg)
 
@@ -86,10 +87,20 @@ void channel_2q(state_t *state, const superop_t *sop, qubit_t q1, qubit_t q2) {
     m.k = 2;
     m.qs[0] = q1;
     m.qs[1] = q2;
+    /* a host superoperator goes to the device as a launch's arguments: a staged copy made the host wait for the
+     * stream in every call */
     ork_lock();
-    const double *S = ork_dev_doubles((const double *)sop->data, 2 * 256);
-    const int e = ork_dm_group(ork_dev()->stream, ork_prec(state), ork_layout(state), LOG_TILE_DIM, state->data,
-                               state->qubits, ORK_DM_SOP2, &m, S);
+    ork_dev_t *d = ork_dev();
+    const double *S = (const double *)sop->data;
+    int e = 0;
+    if (!ork_is_dev_ptr(S)) {
+        if (!d->sop2) d->sop2 = ork_mem_get(2 * 256 * sizeof(double));
+        e = d->sop2 ? ork_put256(d->stream, d->sop2, S) : (int)hipErrorOutOfMemory;
+        S = d->sop2;
+    }
+    if (!e)
+        e = ork_dm_group(d->stream, ork_prec(state), ork_layout(state), LOG_TILE_DIM, state->data, state->qubits,
+                         ORK_DM_SOP2, &m, S);
     ork_unlock();
     ORK_HIP("channel_2q", e);
 }

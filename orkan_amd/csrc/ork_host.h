@@ -40,6 +40,7 @@ typedef struct {
     size_t stage_bytes;
     void *phase;           /* exp_diag per-index phases */
     size_t phase_bytes;
+    double *sop2;          /* channel_2q's superoperator: 256 complex */
     int noalloc_err;       /* result of ork_noalloc_setup() on this device */
 } ork_dev_t;
 

@@ -58,6 +58,8 @@ typedef struct {
 } ork_mono_t;
 
 int ork_fill(void *stream, int prec, void *data_dev, uint64_t len, double re, double im);
+/* dst_dev[0..256) = src (256 complex in host memory, free again on return) through kernel arguments */
+int ork_put256(void *stream, void *dst_dev, const double *src);
 int ork_fill_tiled_corner(void *stream, int prec, void *data_dev, int n, int log_tile, double v);
 
 int ork_sv_1q(void *stream, int prec, void *psi_dev, int n, int q, int op, const double *coef);
