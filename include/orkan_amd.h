@@ -168,9 +168,9 @@ int orkan_set_launch_shape(int kernel, int flags, int lds_bytes);
  * Batched QAOA evaluation.  One evaluation is the reference call sequence
  *   state_plus(PURE, n); p x { exp_diag(C, gamma_l); rx(q, 2 beta_l) for q = 0..n-1 }; mean(C)
  * for a graph's cost diagonal C (2^n doubles).  All evaluations of one call
- * run in a single persistent kernel launch replayed from a hipGraph; states of
- * up to 2^LT amplitudes stay in LDS, larger ones (n <= 2 LT) stream through HBM
- * in p + 1 LDS-tiled sweeps.
+ * run together; states of up to 2^LT amplitudes stay on the chip, larger ones
+ * (n <= 2 LT) stream through HBM in p + 1 tiled sweeps, each one launch over
+ * every tile of every state.
  * ---------------------------------------------------------------------------------------------- */
 typedef struct orkan_qaoa orkan_qaoa_t;
 
@@ -182,7 +182,8 @@ void orkan_qaoa_destroy(orkan_qaoa_t *q);
  * (row e, first p[e] used); out[e] = <C> after the circuit.  0 on success. */
 int orkan_qaoa_eval(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma,
                     const double *beta, double *out);
-/* launch configuration: LDS tile 2^lt amplitudes (10..13), workgroup size, workgroups per CU (0: max) */
+/* launch configuration: tile of 2^lt amplitudes (10..13), workgroup size, workgroups per CU (0: as many as run best).
+ * lt 12 with 256 threads holds the tile in registers, every other shape in LDS. */
 int orkan_qaoa_set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu);
 int orkan_qaoa_get_config(const orkan_qaoa_t *q, int *lt, int *threads, int *grid);
 /* time every candidate configuration on this evaluation list and keep the fastest */

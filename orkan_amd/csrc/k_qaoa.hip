@@ -1,5 +1,5 @@
 // k_qaoa.hip -- batched QAOA evaluation: thousands of (graph, angles) circuits
-// of uneven qubit counts in one persistent launch.
+// of uneven qubit counts in a few launches for all of them together.
 //
 // One evaluation is the reference's own QAOA call sequence:
 //   state_plus(PURE, n); p x { exp_diag(C, gamma); rx(q, 2 beta) for q = 0..n-1 };
@@ -11,15 +11,19 @@
 // of those calls to rounding (the rx of one layer act on distinct qubits and
 // commute; states in HBM apply them in another order than 0..n-1).
 //
-// Execution: every workgroup of the persistent grid pulls evaluations from an
-// atomic counter (largest first) and runs each one start to finish, so no
-// workgroup ever waits for another.  A state of n <= LT qubits lives in LDS for
-// the whole circuit.  A larger state (n <= 2 LT) lives in HBM and is swept in
-// LDS tiles of 2^LT amplitudes, alternating contiguous tiles and tiles gathered
-// at stride 2^LT; each sweep finishes the previous layer's rx on the qubits the
+// Execution: a state of n <= LT qubits stays on the chip for the whole circuit. A
+// larger state (n <= 2 LT) lives in HBM and is swept in tiles of 2^LT
+// amplitudes, alternating contiguous tiles and tiles gathered at stride 2^LT;
+// each sweep finishes the previous layer's rx on the qubits the
 // previous sweep could not reach and runs the next layer's exp_diag and rx on
 // every qubit it holds: p + 1 sweeps for p layers instead of p (n + 1) gate
 // passes; the last sweep reduces sum_x C(x) |psi_x|^2.
+//
+// Two forms. qaoa_sweep and qaoa_one_tile, the default: tiles of 2^12 amplitudes
+// in registers, one launch per sweep with a workgroup for every tile of every
+// evaluation. qaoa_persistent, the other shapes and phases of 2^50 and more: tiles in
+// LDS, the workgroups of one launch pull evaluations from an atomic counter
+// (largest first) and run each one start to finish.
 #include "k_common.hpp"
 
 namespace {
@@ -310,6 +314,388 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
     }
 }
 
+// ---- tiles of 2^12 amplitudes in registers -----------------------------------------------------------
+// qaoa_persistent keeps its tile in LDS and takes it through registers and back for every three qubits and for the
+// phases: nine round trips per layer of a 20-qubit state, 288 B of LDS traffic per amplitude, half of its cycles bank
+// conflicts, and that was its time.  Here a workgroup of 256 threads holds the tile in registers, 16 amplitudes per
+// thread, in one of three layouts:
+//   layout 0: e = u | t << 4                     (register index u = tile bits 0-3)
+//   layout 1: e = (t & 15) | u << 4 | (t >> 4) << 8   (bits 4-7)
+//   layout 2: e = t | u << 8                     (bits 8-11)
+// An rx on four qubits, a phase, a load or a store happens in a layout without LDS; a change of layout moves the real
+// parts, then the imaginary parts, through one padded array of 2^12 doubles (34 KB: four workgroups per CU), written and
+// read without bank conflicts (one spare slot per 16).  A sweep of a 17- to 20-qubit state changes layout three times: 96
+// B per amplitude.
+//
+// The sweeps are those of qaoa_persistent (k = 0..p, alternating contiguous and gathered tiles).  Sweep k finishes layer
+// k - 1 on tile bits ls..11 and runs layer k's phase and rx on every tile bit; the rx of one layer commute, so a sweep
+// visits the layouts in the order that needs fewest changes: 1 (load, finish bits 4-7), 0 (finish bits 0-3, only where
+// ls < 4), 2 (finish bits 8-11, phase, rx), 0 (rx), 1 (rx, store); with ls >= 8 it starts in layout 2.
+// A launch is one sweep k over all tiles of all states that have it, so a single large state fills the chip as well as a
+// thousand do: with a workgroup per evaluation one state of 18 qubits took 2180 us, now 99; 64 of 16 qubits 632 and 209;
+// six of 21 to 24 qubits 185 and 5.2 ms; 300 of 4 to 11 qubits (qaoa_one_tile) 231 and 213.  4096 evaluations of 10 to 20
+// qubits and 1 to 8 layers: 29.0 ms a call, some 3 of them on the host, against 38.8 with the best shape of qaoa_persistent
+// and 33.8 with these tiles and a workgroup per evaluation.  It is bound by memory: 140 GB of amplitudes and cost
+// diagonal in runs of 256 and 128 B take 26 ms with everything else left out, the rest alone 14.  Nontemporal accesses gain
+// nothing.
+constexpr int RT_BITS = 12, RT_THREADS = 256;
+constexpr int RT_BATCH = 4;   // phases whose loads and sincos go together
+
+// a value that is the same in every lane, as a scalar: what is loaded by a computed index counts as per-lane otherwise, and
+// with it every branch and address that depends on it
+__device__ __forceinline__ int uni(int x) { return __builtin_amdgcn_readfirstlane(x); }
+__device__ __forceinline__ u64 uni(u64 x) {
+    return (u64)(unsigned)uni((int)(unsigned)(x >> 32)) << 32 | (unsigned)uni((int)(unsigned)x);
+}
+__device__ __forceinline__ double uni(double x) { return __longlong_as_double((long long)uni((u64)__double_as_longlong(x))); }
+
+// rx without its scalar factor in one form: c I - i s X = c (I - i u X) with u = s / c where |c| >= |s|, else
+// -i s X (I - i u X) with u = -c / s.  The X flips every qubit of the layer; it commutes with every later rx, so the
+// register version leaves it out and reads C at the complemented index from then on (RxFlip.flip).
+struct RxFlip {
+    double u;
+    bool flip;
+    __device__ RxFlip(double c, double s) {
+        flip = fabs(c) < fabs(s);
+        u = flip ? -c / s : s / c;
+    }
+};
+// the thread's 16 amplitudes: two arrays, so that either half can change layout by itself
+struct Amps {
+    double re[16], im[16];
+};
+// sin and cos of x for |x| < 2^50: reduction to [-pi/4, pi/4] by the nearest multiple k of pi/2 with pi/2 as the sum of two
+// doubles (x - k P1 is exact in one fma: a multiple of 2^-52 below 1; the second fma rounds once; the sum is off by k
+// 1.5e-33), then Taylor's series to x^17 / 17! and x^18 / 18!, whose next terms are below 2^-60 there.  Off by at most 2^-52.6
+// (checked against 50 digits).  The library's sincos carries a reduction for any argument, whose registers did not fit
+// beside 16 amplitudes.
+__device__ __forceinline__ void sincos_bounded(double x, double &s, double &c) {
+    const double kd = fma(x, 0.63661977236758138, 6755399441055744.0);   // k + 1.5 2^52: k in the low bits
+    const int q = (int)(unsigned)(unsigned long long)__double_as_longlong(kd);
+    const double k = kd - 6755399441055744.0;
+    double r = fma(-k, 1.5707963267948966, x);
+    r = fma(-k, 6.123233995736766e-17, r);
+    const double z = r * r;
+    double a = 2.8114572543455206e-15;
+    a = fma(a, z, -7.647163731819816e-13);
+    a = fma(a, z, 1.6059043836821613e-10);
+    a = fma(a, z, -2.505210838544172e-08);
+    a = fma(a, z, 2.7557319223985893e-06);
+    a = fma(a, z, -0.0001984126984126984);
+    a = fma(a, z, 0.008333333333333333);
+    a = fma(a, z, -0.16666666666666666);
+    const double sn = fma(a * z, r, r);
+    double b = -1.5619206968586225e-16;
+    b = fma(b, z, 4.779477332387385e-14);
+    b = fma(b, z, -1.1470745597729725e-11);
+    b = fma(b, z, 2.08767569878681e-09);
+    b = fma(b, z, -2.755731922398589e-07);
+    b = fma(b, z, 2.48015873015873e-05);
+    b = fma(b, z, -0.001388888888888889);
+    b = fma(b, z, 0.041666666666666664);
+    b = fma(b, z, -0.5);
+    const double cs = fma(b, z, 1.0);
+    const double s0 = q & 1 ? cs : sn, c0 = q & 1 ? sn : cs;
+    s = q & 2 ? -s0 : s0;
+    c = (q + 1) & 2 ? -c0 : c0;
+}
+
+// I - i u X on the register bits of `mask`; u = 0 leaves a bit as it is, so that no branch splits the registers' lives
+__device__ __forceinline__ void rx4(Amps &v, unsigned mask, double u) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        __builtin_amdgcn_sched_barrier(0);
+        const double uk = (mask >> k) & 1 ? u : 0.0;
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (!((j >> k) & 1)) {
+                const int i = j | (1 << k);
+                const double ar = v.re[j], ai = v.im[j], br = v.re[i], bi = v.im[i];
+                v.re[j] = fma(uk, bi, ar);
+                v.im[j] = fma(-uk, br, ai);
+                v.re[i] = fma(uk, ai, br);
+                v.im[i] = fma(-uk, ar, bi);
+            }
+    }
+}
+
+// tile element of register u: lay_base + u * lay_step; its slot in LDS: lay_slot + u * lay_slot_step (one spare slot per 16
+// elements; in layout 0 the 16 elements of a thread are one such group)
+template <int LAY> __device__ __forceinline__ int lay_base(int t) {
+    return LAY == 0 ? t << 4 : LAY == 1 ? (t & 15) | (t >> 4) << 8 : t;
+}
+template <int LAY> __device__ __forceinline__ int lay_slot(int t) {
+    const int e = lay_base<LAY>(t);
+    return e + (e >> 4);
+}
+constexpr int lay_step(int lay) { return lay == 0 ? 1 : lay == 1 ? 16 : 256; }
+constexpr int lay_slot_step(int lay) { return lay == 0 ? 1 : lay == 1 ? 17 : 272; }
+
+template <int FROM, int TO>
+__device__ __forceinline__ void change_layout(Amps &v, double *lds) {
+    constexpr int ws = lay_slot_step(FROM), rs = lay_slot_step(TO);
+    double *w = lds + lay_slot<FROM>(threadIdx.x);
+    const double *r = lds + lay_slot<TO>(threadIdx.x);
+#pragma unroll
+    for (int u = 0; u < 16; ++u) w[u * ws] = v.re[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v.re[u] = r[u * rs];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) w[u * ws] = v.im[u];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < 16; ++u) v.im[u] = r[u * rs];
+    __syncthreads();
+}
+
+// Memory index of a tile element: f(x) = (x >> ls) << 12 | (x & (2^ls - 1)) past the chunk's own offset in a gathered tile,
+// x itself in a contiguous one.  f acts on bits and a thread's and a register's share of x have no bit in common, so the
+// two shares join by xor, also through a further map that is linear over bits.
+struct TileMap {
+    unsigned chunk;   // offset of the tile's element 0
+    int ls;           // 12: contiguous
+    __device__ __forceinline__ unsigned f(unsigned x) const { return (x >> ls) << RT_BITS | (x & ((1u << ls) - 1)); }
+    template <int LAY> __device__ __forceinline__ unsigned reg(int u) const { return chunk | f((unsigned)(u * lay_step(LAY))); }
+};
+// Byte offset of an amplitude in a state slot: blocks of 16 real parts and 16 imaginary parts (256 B, the run of a gathered
+// tile of 20 qubits), and the blocks of each 2^12 amplitudes in an order that turns with the bits above: in index order the
+// 2^(n - 12) runs of a gathered tile lie 64 KB apart, on few of the memory channels (4 to 6 % of the whole batch).
+__device__ __forceinline__ unsigned slot_off(unsigned x) {
+    const unsigned y = x ^ ((x >> 8) & 0xff0u);
+    return (y >> 4) << 8 | (y & 15u) << 3;
+}
+// An array as a buffer resource: an access adds a thread's and a scalar byte offset to it in one instruction.  (Through
+// pointers the compiler kept a 64-bit address per register and access alive across the sweep, over 100 VGPRs.) 
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+typedef __amdgpu_buffer_rsrc_t Buf;
+__device__ __forceinline__ Buf buffer(const void *p, u64 bytes) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, (int)(unsigned)bytes, 0x00020000);
+}
+__device__ __forceinline__ double load8(Buf b, unsigned off) {
+    return __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(b, (int)off, 0, 0));
+}
+template <int LAY> __device__ __forceinline__ void load_amps(Amps &v, Buf s, const TileMap &m, unsigned off) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int x = (int)(off ^ slot_off(m.reg<LAY>(u)));
+        v.re[u] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(s, x, 0, 0));
+        v.im[u] = __builtin_bit_cast(double, __builtin_amdgcn_raw_buffer_load_b64(s, x + 128, 0, 0));
+    }
+}
+template <int LAY> __device__ __forceinline__ void store_amps(const Amps &v, Buf s, const TileMap &m, unsigned off) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        const int x = (int)(off ^ slot_off(m.reg<LAY>(u)));
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v.re[u]), s, x, 0, 0);
+        __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(v2u, v.im[u]), s, x + 128, 0, 0);
+    }
+}
+
+// the cost diagonal, read at the complemented index while `flip` is set
+struct Diag {
+    Buf b;
+    unsigned last;   // 2^n - 1
+    bool flip;
+    template <int LAY> __device__ __forceinline__ double at(const TileMap &m, int u, unsigned off) const {
+        return load8(b, (off ^ m.reg<LAY>(u) ^ (flip ? last : 0u)) * 8);
+    }
+    // states of at most one tile, whose elements past 2^n do not exist: 0 there
+    template <int LAY> __device__ __forceinline__ double at_small(int u, unsigned off) const {
+        const unsigned x = off | (unsigned)(u * lay_step(LAY));
+        return x <= last ? load8(b, (x ^ (flip ? last : 0u)) * 8) : 0.0;
+    }
+};
+
+// the phases of the thread's 16 amplitudes in layout LAY
+template <int LAY, int SMALL>
+__device__ __forceinline__ void phase16(Amps &v, const Diag &C, const TileMap &m, unsigned off, double g) {
+#pragma unroll
+    for (int u0 = 0; u0 < 16; u0 += RT_BATCH) {
+        double cv[RT_BATCH];
+#pragma unroll
+        for (int u = 0; u < RT_BATCH; ++u) cv[u] = SMALL ? C.at_small<LAY>(u0 + u, off) : C.at<LAY>(m, u0 + u, off);
+#pragma unroll
+        for (int u = 0; u < RT_BATCH; ++u) {
+            if (u == 0) __builtin_amdgcn_sched_barrier(0);
+            double s, c;
+            sincos_bounded(cv[u] * g, s, c);
+            const double x = v.re[u0 + u], y = v.im[u0 + u];
+            v.re[u0 + u] = fma(c, x, s * y);
+            v.im[u0 + u] = fma(c, y, -(s * x));
+        }
+    }
+}
+template <int LAY, int SMALL>
+__device__ __forceinline__ double mean16(const Amps &v, const Diag &C, const TileMap &m, unsigned off) {
+    double acc = 0.0;
+#pragma unroll
+    for (int u0 = 0; u0 < 16; u0 += 8) {
+        double cv[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) cv[u] = SMALL ? C.at_small<LAY>(u0 + u, off) : C.at<LAY>(m, u0 + u, off);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) acc += cv[u] * (v.re[u0 + u] * v.re[u0 + u] + v.im[u0 + u] * v.im[u0 + u]);
+    }
+    return acc;
+}
+
+// product over layers of the squared modulus the scaled rx leave out, once per qubit
+__device__ double rx_scale(const double *ang, int p, int n) {
+    double scale = 1.0;
+    for (int l = 0; l < p; ++l) {
+        const double c = ang[3 * l + 1], s = ang[3 * l + 2];
+        const double f2 = fabs(c) < fabs(s) ? s * s : c * c;
+        for (int q = 0; q < n; ++q) scale *= f2;
+    }
+    return scale;
+}
+
+// an evaluation of a launch
+struct QaoaRec {
+    u64 diag_off;    // of C in the diagonal arena (doubles)
+    u64 tile;        // of its first tile in the state slots (tiles of 2^12 amplitudes)
+    int angle_off;   // of its per-layer (gamma, cos beta, sin beta)
+    int p, n, out;   // layers, qubits, place of its result
+};
+
+// states of at most one tile: a workgroup runs the whole circuit
+__global__ __launch_bounds__(RT_THREADS, 3) void qaoa_one_tile(const QaoaRec *__restrict__ recs,
+                                                              const double *__restrict__ angles,
+                                                              const double *__restrict__ diag, double *__restrict__ out) {
+    __shared__ double lds[(1 << RT_BITS) + (1 << RT_BITS) / 16];
+    __shared__ double red[RT_THREADS / 64];
+    const int t = threadIdx.x;
+    const QaoaRec r = recs[blockIdx.x];
+    const int n = r.n, p = r.p;
+    const double *ang = angles + r.angle_off;
+    Diag C{buffer(diag + r.diag_off, (u64)8 << n), (1u << n) - 1, false};
+    // layouts 2 and 1 take turns in holding the phase, 0 in between.  Amplitudes past 2^n are 0 and stay 0 (their bits carry
+    // no rx)
+    const TileMap m{0, RT_BITS};
+    const unsigned b0 = n >= 4 ? 15u : (1u << n) - 1, b1 = n >= 8 ? 15u : n > 4 ? (1u << (n - 4)) - 1 : 0u,
+                   b2 = n > 8 ? (1u << (n - 8)) - 1 : 0u;
+    const double amp = 1.0 / sqrt((double)(1u << n));
+    Amps v;
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        v.re[u] = (t | u << 8) < (1 << n) ? amp : 0.0;
+        v.im[u] = 0.0;
+    }
+    for (int l = 0; l < p; ++l) {
+        const double g = uni(ang[3 * l]);
+        const RxFlip rx(uni(ang[3 * l + 1]), uni(ang[3 * l + 2]));
+        if (l & 1) {
+            phase16<1, 1>(v, C, m, (unsigned)lay_base<1>(t), g);
+            rx4(v, b1, rx.u);
+            change_layout<1, 0>(v, lds);
+            rx4(v, b0, rx.u);
+            change_layout<0, 2>(v, lds);
+            rx4(v, b2, rx.u);
+        } else {
+            phase16<2, 1>(v, C, m, (unsigned)t, g);
+            rx4(v, b2, rx.u);
+            change_layout<2, 0>(v, lds);
+            rx4(v, b0, rx.u);
+            change_layout<0, 1>(v, lds);
+            rx4(v, b1, rx.u);
+        }
+        C.flip ^= rx.flip;
+    }
+    const double acc = p & 1 ? mean16<1, 1>(v, C, m, (unsigned)lay_base<1>(t)) : mean16<2, 1>(v, C, m, (unsigned)t);
+    const double tot = block_sum<RT_THREADS>(acc, red);
+    if (t == 0) out[r.out] = tot * rx_scale(ang, p, n);
+}
+
+// One sweep k of every larger state that has it (p >= k): a workgroup per tile.  The evaluations are sorted by qubits, then
+// by layers, both descending, so the tiles of a sweep are a few runs of equal 2^(n - 12).
+constexpr int RT_CLASSES = 12;   // 13 to 24 qubits
+struct SweepArgs {
+    const QaoaRec *recs;
+    const double *angles, *diag;
+    double2 *states;
+    double *part;                     // per tile of the slots: its share of the mean
+    int k, nclass;
+    unsigned first[RT_CLASSES + 1];   // first workgroup of each class
+    int rec[RT_CLASSES], n[RT_CLASSES];
+};
+
+__global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
+    __shared__ double lds[(1 << RT_BITS) + (1 << RT_BITS) / 16];
+    __shared__ double red[RT_THREADS / 64];
+    const int t = threadIdx.x, k = A.k;
+    int c = 0;
+    while (c + 1 < A.nclass && blockIdx.x >= A.first[c + 1]) ++c;
+    const int n = A.n[c];
+    const unsigned b = blockIdx.x - A.first[c], ch = b & ((1u << (n - RT_BITS)) - 1);
+    const QaoaRec r = A.recs[A.rec[c] + (int)(b >> (n - RT_BITS))];
+    const double *ang = A.angles + r.angle_off;
+    const bool gathered = k & 1, last = k == r.p;
+    // the flips of the layers before k
+    bool flip = false;
+    for (int l = 0; l < k; ++l) flip ^= fabs(uni(ang[3 * l + 1])) < fabs(uni(ang[3 * l + 2]));
+    const Diag C{buffer(A.diag + r.diag_off, (u64)8 << n), (1u << n) - 1, flip};
+    const double g = last ? 0.0 : uni(ang[3 * k]);
+    const RxFlip rx(last ? 1.0 : uni(ang[3 * k + 1]), last ? 0.0 : uni(ang[3 * k + 2]));
+    const RxFlip rxp(k ? uni(ang[3 * k - 2]) : 1.0, k ? uni(ang[3 * k - 1]) : 0.0);
+    const int ls = 2 * RT_BITS - n;
+    // layer k - 1 is left to finish on tile bits ls..11, by layout
+    const unsigned f0 = ls < 4 ? 15u & (15u << ls) : 0u;
+    const unsigned f1 = ls < 8 ? 15u & (15u << (ls > 4 ? ls - 4 : 0)) : 0u;
+    const unsigned f2 = 15u & (15u << (ls > 8 ? ls - 8 : 0));
+    const TileMap m{ch << (gathered ? ls : RT_BITS), gathered ? ls : RT_BITS};
+    const unsigned off2 = m.f((unsigned)t), soff1 = slot_off(m.f((unsigned)lay_base<1>(t))), soff2 = slot_off(off2);
+    const Buf S = buffer(A.states + (r.tile << RT_BITS), (u64)16 << n);
+    Amps v;
+    if (k == 0) {
+        const double amp = 1.0 / sqrt((double)(1u << n));
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            v.re[u] = amp;
+            v.im[u] = 0.0;
+        }
+    } else {
+        if (f1) {
+            load_amps<1>(v, S, m, soff1);
+            rx4(v, f1, rxp.u);
+            if (f0) {
+                change_layout<1, 0>(v, lds);
+                rx4(v, f0, rxp.u);
+                change_layout<0, 2>(v, lds);
+            } else {
+                change_layout<1, 2>(v, lds);
+            }
+        } else {
+            load_amps<2>(v, S, m, soff2);
+        }
+        rx4(v, f2, rxp.u);
+    }
+    if (last) {
+        const double tot = block_sum<RT_THREADS>(mean16<2, 0>(v, C, m, off2), red);
+        if (t == 0) A.part[r.tile + ch] = tot;
+        return;
+    }
+    phase16<2, 0>(v, C, m, off2, g);
+    rx4(v, 15u, rx.u);
+    change_layout<2, 0>(v, lds);
+    rx4(v, 15u, rx.u);
+    change_layout<0, 1>(v, lds);
+    rx4(v, 15u, rx.u);
+    store_amps<1>(v, S, m, soff1);
+}
+
+// the tiles' shares of each mean, in a fixed order
+__global__ __launch_bounds__(256) void qaoa_finish(const QaoaRec *__restrict__ recs, const double *__restrict__ angles,
+                                                   const double *__restrict__ part, double *__restrict__ out) {
+    __shared__ double red[4];
+    const QaoaRec r = recs[blockIdx.x];
+    double acc = 0.0;
+    for (int i = threadIdx.x; i < 1 << (r.n - RT_BITS); i += 256) acc += part[r.tile + (u64)i];
+    const double tot = block_sum<256>(acc, red);
+    if (threadIdx.x == 0) out[r.out] = tot * rx_scale(angles + r.angle_off, r.p, r.n);
+}
+
 __global__ void reset_counter(unsigned *c) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0u;
 }
@@ -324,6 +710,27 @@ __global__ __launch_bounds__(256) void maxcut_diag_kernel(double *__restrict__ o
     for (int k = 0; k < ne; ++k)
         if (((x >> ei[k]) ^ (x >> ej[k])) & 1) acc += w[k];
     out[x] = acc;
+}
+
+// cmax[g] = the largest |C| of graph g, infinity if any is not finite
+__global__ __launch_bounds__(256) void diag_max_kernel(const QaoaGraph *__restrict__ graphs, const double *__restrict__ diag,
+                                                       double *__restrict__ cmax) {
+    __shared__ double red[256];
+    const QaoaGraph g = graphs[blockIdx.x];
+    const double *C = diag + g.diag_off;
+    double m = 0.0;
+#pragma unroll 4
+    for (u64 x = threadIdx.x; x < ((u64)1 << g.n); x += 256) {
+        const double a = fabs(C[x]);
+        m = fmax(m, a <= 1.7976931348623157e308 ? a : __builtin_huge_val());
+    }
+    red[threadIdx.x] = m;
+    __syncthreads();
+    for (int h = 128; h; h >>= 1) {
+        if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) cmax[blockIdx.x] = red[0];
 }
 
 template <int LT, int THREADS>
@@ -356,19 +763,75 @@ extern "C" int ork_qaoa_launch(void *stream, int lt, int threads, int grid, cons
 #define ORK_QCASE(L, TH) if (lt == L && threads == TH) return launch_qaoa<L, TH>(st, a, grid);
     ORK_QCASE(10, 256) ORK_QCASE(10, 512) ORK_QCASE(10, 1024)
     ORK_QCASE(11, 256) ORK_QCASE(11, 512) ORK_QCASE(11, 1024)
-    ORK_QCASE(12, 256) ORK_QCASE(12, 512) ORK_QCASE(12, 1024)
+    ORK_QCASE(12, 512) ORK_QCASE(12, 1024)
     ORK_QCASE(13, 512) ORK_QCASE(13, 1024)
 #undef ORK_QCASE
     return (int)hipErrorInvalidValue;
 }
 
+// recs: `count` QaoaRec on the device, sorted by qubits, then by layers, both descending; n and p: their qubits and layers on
+// the host; the states of more than 12 qubits have their tiles in `states`, one partial sum per tile in `part`
+extern "C" int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, const int *p, int count, const double *angles,
+                               const double *diag, void *states, double *part, double *out) {
+    hipStream_t st = (hipStream_t)stream;
+    const QaoaRec *r = (const QaoaRec *)recs;
+    int large = 0, pmax = 0;
+    while (large < count && n[large] > RT_BITS) {
+        if (n[large] > 2 * RT_BITS) return (int)hipErrorInvalidValue;
+        if (p[large] > pmax) pmax = p[large];
+        ++large;
+    }
+    if (count > large) {
+        qaoa_one_tile<<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
+        ORK_LAUNCH_CHECK();
+    }
+    for (int k = 0; k <= pmax && large; ++k) {
+        SweepArgs A;
+        A.recs = r;
+        A.angles = angles;
+        A.diag = diag;
+        A.states = (double2 *)states;
+        A.part = part;
+        A.k = k;
+        A.nclass = 0;
+        unsigned blocks = 0;
+        for (int i = 0; i < large;) {
+            int m = 0, j = i;
+            for (; j < large && n[j] == n[i]; ++j) m += p[j] >= k;   // the first m of the class
+            if (m) {
+                A.first[A.nclass] = blocks;
+                A.rec[A.nclass] = i;
+                A.n[A.nclass++] = n[i];
+                blocks += (unsigned)m << (n[i] - RT_BITS);
+            }
+            i = j;
+        }
+        A.first[A.nclass] = blocks;
+        qaoa_sweep<<<blocks, RT_THREADS, 0, st>>>(A);
+        ORK_LAUNCH_CHECK();
+    }
+    if (large) {
+        qaoa_finish<<<large, 256, 0, st>>>(r, angles, part, out);
+        ORK_LAUNCH_CHECK();
+    }
+    return 0;
+}
+
+extern "C" int ork_qaoa_diag_max(void *stream, int ngraphs, const void *graphs, const double *diag, double *cmax) {
+    diag_max_kernel<<<ngraphs, 256, 0, (hipStream_t)stream>>>((const QaoaGraph *)graphs, diag, cmax);
+    ORK_LAUNCH_CHECK();
+    return 0;
+}
+
 extern "C" int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu) {
     hipError_t e = hipErrorInvalidValue;
+    if (lt == RT_BITS && threads == RT_THREADS)
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_sweep, RT_THREADS, 0);
 #define ORK_QOCC(L, TH) \
     if (lt == L && threads == TH) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_persistent<L, TH>, TH, 0);
     ORK_QOCC(10, 256) ORK_QOCC(10, 512) ORK_QOCC(10, 1024)
     ORK_QOCC(11, 256) ORK_QOCC(11, 512) ORK_QOCC(11, 1024)
-    ORK_QOCC(12, 256) ORK_QOCC(12, 512) ORK_QOCC(12, 1024)
+    ORK_QOCC(12, 512) ORK_QOCC(12, 1024)
     ORK_QOCC(13, 512) ORK_QOCC(13, 1024)
 #undef ORK_QOCC
     return (int)e;

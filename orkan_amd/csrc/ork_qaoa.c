@@ -1,8 +1,9 @@
 /*
  * ork_qaoa.c -- host side of the batched QAOA launcher: device arenas for the
- * cost diagonals, the evaluation list and the per-workgroup state scratch; a
- * hipGraph holding the counter reset and the persistent kernel; and the
- * autotuner that picks the LDS tile and workgroup size.
+ * cost diagonals, the evaluation list and the state scratch; the launches of the
+ * register kernels, one per sweep over every evaluation (12, 256: the default);
+ * for the LDS shapes a hipGraph holding the counter reset and the persistent
+ * kernel; and the autotuner that picks among them.
  *
  * No reference counterpart: the reference evaluates one circuit per call
  * sequence (state_plus, exp_diag, rx, mean).  Each evaluation here computes
@@ -18,10 +19,14 @@ int ork_qaoa_launch(void *stream, int lt, int threads, int grid, const void *eva
                     const int *nevals, const void *graphs, const double *angles, const double *diag, void *states,
                     uint64_t slot_elems, double *out, unsigned *counter);
 int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu);
+int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, const int *p, int count, const double *angles,
+                    const double *diag, void *states, double *part, double *out);
+int ork_qaoa_diag_max(void *stream, int ngraphs, const void *graphs, const double *diag, double *cmax);
 int ork_maxcut_diag(void *stream, double *out, int n, int ne, const int *ei, const int *ej, const double *w);
 
 typedef struct { int graph, p, angle_off, pad; } q_eval_t;
 typedef struct { uint64_t diag_off, state_off; int n, pad; } q_graph_t;
+typedef struct { uint64_t diag_off, tile; int angle_off, p, n, out; } q_rec_t;
 
 struct orkan_qaoa {
     int ngraphs, max_evals, max_p, nmax;
@@ -40,6 +45,14 @@ struct orkan_qaoa {
      * threads' gates and reductions use, and replayed on the library stream */
     hipStream_t capture_stream;
     int nevals_h;          /* host source of the nevals_d upload */
+    double *cmax_h;        /* per graph: largest |C| */
+    /* the register kernels' list: records sorted by qubits, then layers, both descending */
+    q_rec_t *recs_h;
+    void *recs_d;
+    int *n_h, *p_h, *start_h, nstaged;
+    int states_short;      /* the device had no memory for all the scratch asked for */
+    size_t room;           /* tiles per round of launches, as the staged records number them */
+    int wide;              /* the staged list holds a phase too large for the register kernel's sincos */
     hipGraph_t graph;
     hipGraphExec_t exec;
     int graph_ok;
@@ -56,23 +69,19 @@ static int cus(void) {
     return n;
 }
 
-static int ensure_states(orkan_qaoa_t *q) {
-    /* scratch for states larger than the LDS tile: one slot of 2^nmax per workgroup */
-    size_t need = 16;
-    if (q->nmax > q->lt) need = (size_t)q->grid * ((size_t)1 << q->nmax) * 16;
-    if (q->states_bytes >= need) return 0;
-    if (q->states_d) {
-        (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
-        (void)hipFree(q->states_d);
-    }
-    q->states_d = NULL;
-    q->states_bytes = 0;
-    int e = (int)hipMalloc(&q->states_d, need);
-    if (e) return e;
-    q->states_bytes = need;
-    q->graph_ok = 0;
-    return 0;
-}
+/* the register kernels (2^12 amplitudes per workgroup of 256 threads) take phases gamma C up to this; larger ones, and ones
+ * that are not finite, run through the LDS kernel, whose sincos reduces any argument */
+#define REG_LT 12
+#define REG_THREADS 256
+#define REG_PHASE_MAX 1125899906842624.0   /* 2^50 */
+#define WIDE_THREADS 512
+#define TILE_BYTES ((size_t)16 << REG_LT)
+/* state slots of the register kernels: evaluations beyond them go in further rounds of launches. 4096 evaluations of 10 to
+ * 20 qubits: 29.0 ms with 64 or 128 MB, which the last-level cache can hold from one sweep to the next, 29.6 with 256 MB
+ * to 16 GB */
+#define SWEEP_BYTES ((size_t)128 << 20)
+
+static int is_reg(const orkan_qaoa_t *q) { return q->lt == REG_LT && q->threads == REG_THREADS; }
 
 static void drop_graph(orkan_qaoa_t *q) {
     if (q->graph_ok) {
@@ -82,6 +91,60 @@ static void drop_graph(orkan_qaoa_t *q) {
     q->graph_ok = 0;
 }
 
+/* The state scratch of the current configuration (and, for it, of the staged list). The LDS kernels need a slot of 2^nmax
+ * for each workgroup. The register kernels take what there is: a slot for each evaluation up to SWEEP_BYTES and 8 B per
+ * tile for the partial sums, halved while memory is short down to one slot of the largest state. */
+static int ensure_states(orkan_qaoa_t *q) {
+    const size_t slot = (size_t)16 << q->nmax;
+    size_t need = 16, least;
+    if (is_reg(q)) {
+        least = (q->nmax > REG_LT ? slot + slot / TILE_BYTES * sizeof(double) : 0) + 16;
+        if (q->nmax > REG_LT) {
+            size_t all = 0;
+            for (int g = 0; g < q->ngraphs; ++g)
+                if (q->graphs_h[g].n > REG_LT) all += (size_t)16 << q->graphs_h[g].n;
+            const size_t rounds = ((size_t)q->max_evals + q->ngraphs - 1) / q->ngraphs;
+            need = all > SWEEP_BYTES / rounds ? SWEEP_BYTES : all * rounds;
+            if (need / slot > (size_t)q->max_evals) need = (size_t)q->max_evals * slot;
+            if (need < slot) need = slot;
+            need += need / TILE_BYTES * sizeof(double) + 16;
+            /* qaoa_persistent takes lists with phases beyond REG_PHASE_MAX */
+            const size_t slots = q->max_evals < cus() ? (size_t)q->max_evals : (size_t)cus();
+            if (q->wide && need < slots * slot) need = slots * slot;
+        }
+    } else {
+        if (q->nmax > q->lt) need = (size_t)q->grid * slot;
+        least = need;
+    }
+    if (q->states_bytes >= need || (q->states_bytes >= least && q->states_short)) return 0;
+    if (q->states_d) {
+        (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
+        (void)hipFree(q->states_d);
+    }
+    q->states_d = NULL;
+    q->states_bytes = 0;
+    q->states_short = 0;
+    drop_graph(q);
+    int e = (int)hipMalloc(&q->states_d, need);
+    while (e && need / 2 >= least) {
+        (void)hipGetLastError();
+        need /= 2;
+        q->states_short = 1;
+        e = (int)hipMalloc(&q->states_d, need);
+    }
+    if (e) {
+        q->states_d = NULL;
+        return e;
+    }
+    q->states_bytes = need;
+    return 0;
+}
+
+/* tiles of the register kernels that the state scratch holds, their partial sums behind them */
+static size_t tile_room(const orkan_qaoa_t *q) {
+    return q->states_bytes < 16 ? 0 : (q->states_bytes - 16) / (TILE_BYTES + sizeof(double));
+}
+
 /* caller holds ork_lock (the state scratch may be freed and the graph dropped) */
 static int set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu) {
     if (2 * lt < q->nmax) return (int)hipErrorInvalidValue;     /* pass B needs n <= 2 LT */
@@ -89,11 +152,13 @@ static int set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu) {
     int e = ork_qaoa_occupancy(lt, threads, &occ);
     if (e) return e;
     if (occ <= 0) return (int)hipErrorInvalidConfiguration;
-    if (blocks_per_cu <= 0 || blocks_per_cu > occ) blocks_per_cu = occ;
+    if (blocks_per_cu <= 0) blocks_per_cu = occ;
+    if (blocks_per_cu > occ) blocks_per_cu = occ;
     drop_graph(q);
     q->lt = lt;
     q->threads = threads;
     q->grid = cus() * blocks_per_cu;
+    if (q->grid > q->max_evals) q->grid = q->max_evals;   /* a workgroup takes at least one evaluation */
     return ensure_states(q);
 }
 
@@ -119,7 +184,14 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     q->evals_h = calloc((size_t)max_evals, sizeof(q_eval_t));
     q->order_h = calloc((size_t)max_evals, sizeof(int));
     q->angles_h = calloc((size_t)max_evals * max_p * 3, sizeof(double));
-    if (!q->graphs_h || !q->evals_h || !q->order_h || !q->angles_h) goto fail;
+    q->cmax_h = calloc((size_t)ngraphs, sizeof(double));
+    q->recs_h = calloc((size_t)max_evals, sizeof(q_rec_t));
+    q->n_h = calloc((size_t)max_evals, sizeof(int));
+    q->p_h = calloc((size_t)max_evals, sizeof(int));
+    q->start_h = calloc((size_t)27 * (max_p + 1) + 1, sizeof(int));
+    if (!q->graphs_h || !q->evals_h || !q->order_h || !q->angles_h || !q->cmax_h || !q->recs_h || !q->n_h || !q->p_h ||
+        !q->start_h)
+        goto fail;
     if (hipStreamCreateWithFlags(&q->capture_stream, hipStreamNonBlocking) != hipSuccess) {
         q->capture_stream = NULL;
         goto fail;
@@ -142,19 +214,29 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
         hipSuccess)
         goto fail;
     if (hipMalloc(&q->evals_d, (size_t)max_evals * sizeof(q_eval_t)) != hipSuccess) goto fail;
+    if (hipMalloc(&q->recs_d, (size_t)max_evals * sizeof(q_rec_t)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->order_d, (size_t)max_evals * sizeof(int)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->nevals_d, sizeof(int)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->angles_d, (size_t)max_evals * max_p * 3 * sizeof(double)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->out_d, (size_t)max_evals * sizeof(double)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->counter_d, sizeof(unsigned)) != hipSuccess) goto fail;
-    if (hipStreamSynchronize(st) != hipSuccess) goto fail;
     {
-        /* default tile: 4096 amplitudes (64 KB of LDS), 512 threads; 8192 when the
-         * largest state needs it */
-        int lt = 12;
+        double *cmax = ork_mem_get((size_t)ngraphs * sizeof(double));
+        const int bad = !cmax || ork_qaoa_diag_max(st, ngraphs, q->graphs_d, q->diag_d, cmax) ||
+                        hipMemcpyAsync(q->cmax_h, cmax, (size_t)ngraphs * sizeof(double), hipMemcpyDeviceToHost, st) !=
+                            hipSuccess;
+        if (hipStreamSynchronize(st) != hipSuccess || bad) {
+            ork_mem_put(cmax);
+            goto fail;
+        }
+        ork_mem_put(cmax);
+    }
+    {
+        /* default: 4096 amplitudes in the registers of 256 threads; 8192 in LDS when the largest state needs it */
+        int lt = REG_LT;
         while (2 * lt < q->nmax) ++lt;
         ork_lock();
-        const int e = set_config(q, lt, lt >= 13 ? 1024 : 512, 0);
+        const int e = set_config(q, lt, lt >= 13 ? 1024 : REG_THREADS, 0);
         ork_unlock();
         if (e) goto fail;
     }
@@ -169,13 +251,18 @@ void orkan_qaoa_destroy(orkan_qaoa_t *q) {
     (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
     drop_graph(q);
     void *bufs[] = {q->graphs_d, q->diag_d, q->evals_d, q->order_d, q->nevals_d,
-                    q->angles_d, q->out_d, q->counter_d, q->states_d};
+                    q->angles_d, q->out_d, q->counter_d, q->states_d, q->recs_d};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i)
         if (bufs[i]) (void)hipFree(bufs[i]);
     free(q->graphs_h);
     free(q->evals_h);
     free(q->order_h);
     free(q->angles_h);
+    free(q->cmax_h);
+    free(q->recs_h);
+    free(q->n_h);
+    free(q->p_h);
+    free(q->start_h);
     if (q->capture_stream) (void)hipStreamDestroy(q->capture_stream);
     free(q);
 }
@@ -211,10 +298,45 @@ static int by_cost_desc(const void *a, const void *b) {
     return *(const int *)a - *(const int *)b;
 }
 
-/* upload the evaluation list; angles: rows of max_p gammas and betas */
-static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma,
-                 const double *beta) {
+/* the register kernels' records: a counting sort by qubits, then layers, both descending */
+static void sort_recs(orkan_qaoa_t *q, int nevals) {
+    const int stride = q->max_p + 1, nkeys = 27 * stride;
+    memset(q->start_h, 0, ((size_t)nkeys + 1) * sizeof(int));
+    for (int e = 0; e < nevals; ++e) {
+        const q_eval_t *ev = &q->evals_h[e];
+        const int key = (26 - q->graphs_h[ev->graph].n) * stride + (q->max_p - ev->p);
+        ++q->start_h[key + 1];
+    }
+    for (int k = 0; k < nkeys; ++k) q->start_h[k + 1] += q->start_h[k];
+    for (int e = 0; e < nevals; ++e) {
+        const q_eval_t *ev = &q->evals_h[e];
+        const int n = q->graphs_h[ev->graph].n;
+        const int at = q->start_h[(26 - n) * stride + (q->max_p - ev->p)]++;
+        const q_rec_t r = {q->graphs_h[ev->graph].diag_off, 0, ev->angle_off, ev->p, n, e};
+        q->recs_h[at] = r;
+        q->n_h[at] = n;
+        q->p_h[at] = ev->p;
+    }
+}
+
+/* the number of records from `at` on whose states fit the scratch together */
+static int next_round(const orkan_qaoa_t *q, int at) {
+    size_t used = 0;
+    int i = at;
+    for (; i < q->nstaged; ++i) {
+        const size_t tiles = q->n_h[i] > REG_LT ? (size_t)1 << (q->n_h[i] - REG_LT) : 0;
+        if (used + tiles > q->room || used + tiles > ((size_t)1 << 31) - 1) break;
+        used += tiles;
+    }
+    return i - at;
+}
+
+/* upload the evaluation list; angles: rows of max_p gammas and betas.  any_shape: for every kernel, not only the one the
+ * configuration and the list's phases call for */
+static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma, const double *beta,
+                 int any_shape) {
     if (nevals < 0 || nevals > q->max_evals) return (int)hipErrorInvalidValue;
+    q->wide = 0;
     for (int e = 0; e < nevals; ++e) {
         if (graph[e] < 0 || graph[e] >= q->ngraphs || p[e] < 1 || p[e] > q->max_p) return (int)hipErrorInvalidValue;
         q->evals_h[e].graph = graph[e];
@@ -223,30 +345,69 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
         for (int l = 0; l < p[e]; ++l) {
             /* rx(q, 2 beta): the reference evaluates cos(theta / 2) and sin(theta / 2) */
             const double theta = 2.0 * beta[(size_t)e * q->max_p + l];
-            q->angles_h[(size_t)e * q->max_p * 3 + 3 * l] = gamma[(size_t)e * q->max_p + l];
+            const double gl = gamma[(size_t)e * q->max_p + l];
+            q->angles_h[(size_t)e * q->max_p * 3 + 3 * l] = gl;
+            if (!(fabs(gl) * q->cmax_h[graph[e]] < REG_PHASE_MAX)) q->wide = 1;
             q->angles_h[(size_t)e * q->max_p * 3 + 3 * l + 1] = cos(theta / 2.0);
             q->angles_h[(size_t)e * q->max_p * 3 + 3 * l + 2] = sin(theta / 2.0);
         }
         q->order_h[e] = e;
     }
-    g_sort_q = q;
-    qsort(q->order_h, (size_t)nevals, sizeof(int), by_cost_desc);
+    q->nstaged = nevals;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    int e = 0;
-    if (nevals > 0) {
-        e |= (int)hipMemcpyAsync(q->evals_d, q->evals_h, (size_t)nevals * sizeof(q_eval_t), hipMemcpyHostToDevice, st);
-        e |= (int)hipMemcpyAsync(q->order_d, q->order_h, (size_t)nevals * sizeof(int), hipMemcpyHostToDevice, st);
+    int e = ensure_states(q);
+    if (e) return e;
+    if (nevals > 0)
         e |= (int)hipMemcpyAsync(q->angles_d, q->angles_h, (size_t)nevals * q->max_p * 3 * sizeof(double),
                                  hipMemcpyHostToDevice, st);
+    if (nevals > 0 && (any_shape || (is_reg(q) && !q->wide))) {
+        sort_recs(q, nevals);
+        /* every round numbers its tiles from 0 */
+        q->room = tile_room(q);
+        for (int at = 0, m; at < nevals && (m = next_round(q, at)) > 0; at += m) {
+            uint64_t tile = 0;
+            for (int i = at; i < at + m; ++i) {
+                q->recs_h[i].tile = tile;
+                if (q->n_h[i] > REG_LT) tile += (uint64_t)1 << (q->n_h[i] - REG_LT);
+            }
+        }
+        e |= (int)hipMemcpyAsync(q->recs_d, q->recs_h, (size_t)nevals * sizeof(q_rec_t), hipMemcpyHostToDevice, st);
     }
-    q->nevals_h = nevals;
-    e |= (int)hipMemcpyAsync(q->nevals_d, &q->nevals_h, sizeof(int), hipMemcpyHostToDevice, st);
+    if (any_shape || !is_reg(q) || q->wide) {
+        g_sort_q = q;
+        qsort(q->order_h, (size_t)nevals, sizeof(int), by_cost_desc);
+        if (nevals > 0) {
+            e |= (int)hipMemcpyAsync(q->evals_d, q->evals_h, (size_t)nevals * sizeof(q_eval_t), hipMemcpyHostToDevice, st);
+            e |= (int)hipMemcpyAsync(q->order_d, q->order_h, (size_t)nevals * sizeof(int), hipMemcpyHostToDevice, st);
+        }
+        q->nevals_h = nevals;
+        e |= (int)hipMemcpyAsync(q->nevals_d, &q->nevals_h, sizeof(int), hipMemcpyHostToDevice, st);
+    }
     e |= (int)hipStreamSynchronize(st);
     return e;
 }
 
 /* caller holds ork_lock */
 int orkan_qaoa_launch_staged(orkan_qaoa_t *q) {
+    if (is_reg(q)) {
+        void *st = ork_dev()->stream;
+        if (q->wide) {
+            const size_t slots = q->nmax > REG_LT ? q->states_bytes / ((size_t)16 << q->nmax) : (size_t)cus();
+            const int grid = slots < (size_t)cus() ? (int)slots : cus();
+            return ork_qaoa_launch(st, REG_LT, WIDE_THREADS, grid, q->evals_d, q->order_d, q->nevals_d, q->graphs_d,
+                                   q->angles_d, q->diag_d, q->states_d, ((uint64_t)1 << q->nmax), q->out_d, q->counter_d);
+        }
+        for (int at = 0; at < q->nstaged;) {
+            const int m = next_round(q, at);
+            if (m == 0) return (int)hipErrorInvalidValue;
+            const int e = ork_qaoa_sweeps(st, (const q_rec_t *)q->recs_d + at, q->n_h + at, q->p_h + at, m, q->angles_d,
+                                          q->diag_d, q->states_d, (double *)((char *)q->states_d + q->room * TILE_BYTES),
+                                          q->out_d);
+            if (e) return e;
+            at += m;
+        }
+        return 0;
+    }
     if (!q->graph_ok) {
         int e = capture(q);
         if (e) return e;
@@ -258,7 +419,7 @@ int orkan_qaoa_eval(orkan_qaoa_t *q, int nevals, const int *graph, const int *p,
                     const double *beta, double *out) {
     if (!q) return (int)hipErrorInvalidValue;
     ork_lock();
-    int e = stage(q, nevals, graph, p, gamma, beta);
+    int e = stage(q, nevals, graph, p, gamma, beta, 0);
     if (!e) e = orkan_qaoa_launch_staged(q);
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     if (!e && nevals > 0 && out)
@@ -294,7 +455,9 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
     }
     /* the whole search holds the library lock: staging, every reconfiguration and launch */
     ork_lock();
-    int e = stage(q, nevals, graph, p, gamma, beta);
+    /* the register kernels' records number tiles of the scratch: it has its size for them first */
+    if (2 * REG_LT >= q->nmax) (void)set_config(q, REG_LT, REG_THREADS, 0);
+    int e = stage(q, nevals, graph, p, gamma, beta, 1);
     if (e) {
         ork_unlock();
         (void)hipEventDestroy(a);

@@ -118,3 +118,48 @@ def test_full_4096_batch_sample():
         i = inst[k]
         want = oracle_eval(orc, i["n"], batch.maxcut_diag(i["n"], i["edges"], i["w"]), i["p"], i["gamma"], i["beta"])
         assert abs(got[k] - want) <= 1e-12, (k, i["n"], i["p"], got[k], want)
+
+
+@pytest.mark.parametrize("lo,hi", [(1, 8), (9, 13), (14, 17), (18, 20), (21, 22)])
+@pytest.mark.parametrize("flips", [False, True])
+def test_register_tiles(lo, hi, flips):
+    """The register kernel at every qubit count of its range: states of one tile, with and without empty registers, and
+    every split of the tile bits between contiguous and gathered tiles; 1 to 4 layers (both layouts a one-tile state may
+    end in), mixers of |cos| >= |sin| only and of both forms (where the cost diagonal is read complemented)."""
+    lib = orkan_amd.load(5)
+    orc = engines.oracle(5)
+    rng = np.random.default_rng(lo + flips)
+    ns, ps = [], []
+    for n in range(lo, hi + 1):
+        for p in ((1, 2, 3, 4) if n < 18 else (2, 3) if n < 21 else (2,)):
+            ns.append(n)
+            ps.append(p)
+    diags = [rng.uniform(-3, 5, 1 << n) for n in ns]
+    gam = [rng.uniform(0, np.pi, p) for p in ps]
+    bet = [rng.uniform(0, np.pi, p) if flips else rng.uniform(-0.7, 0.7, p) for p in ps]
+    b = batch.QaoaBatch(lib, ns, diags, max_evals=len(ns), max_p=4)
+    assert b.config()["lt"] == 12 and b.config()["threads"] == 256
+    got = b.eval(list(range(len(ns))), ps, gam, bet)
+    assert np.array_equal(got, b.eval(list(range(len(ns))), ps, gam, bet))
+    for k, n in enumerate(ns):
+        want = oracle_eval(orc, n, diags[k], ps[k], gam[k], bet[k])
+        assert abs(got[k] - want) <= 1e-12, (n, ps[k], got[k], want)
+    b.close()
+
+
+@pytest.mark.parametrize("big", [3e15, 1e300, np.inf, np.nan])
+def test_phases_beyond_the_register_kernel(big):
+    """A phase of 2^50 or more, or one that is not finite, takes the whole list through the LDS kernel: the bits of that
+    kernel's own shape, NaN where a phase has no value."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(7)
+    ns = [6, 13, 14]
+    diags = [rng.uniform(0, 2, 1 << n) for n in ns]
+    diags[1][5] = big
+    args = ([0, 1, 2], [2, 2, 1], [rng.uniform(0.5, 1, 2) for _ in ns], [rng.uniform(0, 3, 2) for _ in ns])
+    b = batch.QaoaBatch(lib, ns, diags, max_evals=3, max_p=2)
+    got = b.eval(*args)
+    b.set_config(12, 512)
+    assert np.array_equal(got, b.eval(*args), equal_nan=True)
+    assert np.isfinite(got[[0, 2]]).all() and (np.isfinite(big) or np.isnan(got[1]))
+    b.close()
