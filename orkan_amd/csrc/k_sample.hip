@@ -4,6 +4,7 @@
 #include "k_common.hpp"
 
 typedef double d4 __attribute__((ext_vector_type(4)));
+typedef double d2 __attribute__((ext_vector_type(2)));
 
 namespace {
 
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(SM_THREADS) void block_partial_kernel(const double2
     const u64 x0 = (u64)blockIdx.x * chunk;
     // thread: row tid / 16 of each 16, amplitude tid % 16; rows past the end repeat the last vector
     const int lr = tid >> 4, lx = tid & 15;
-    cd v[SIDES][NT];
+    d2 v[SIDES][NT];   // a vector type: as structs the compiler kept them in scratch memory
     double o = 0.0;
     const auto load = [&](u64 xs) {
         const u64 x = xs + lx;
@@ -88,9 +89,9 @@ __global__ __launch_bounds__(SM_THREADS) void block_partial_kernel(const double2
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             const int r = t * 16 + lr;
-            v[0][t] = P[(u64)(r < na ? r : na - 1) * stride + xc];
-            if (!SAME) v[SIDES - 1][t] = Q[(u64)(r < nb ? r : nb - 1) * stride + xc];
-            if (GUARD && !in) v[0][t] = v[SIDES - 1][t] = cmk(0.0, 0.0);
+            v[0][t] = *(const d2 *)&P[(u64)(r < na ? r : na - 1) * stride + xc];
+            if (!SAME) v[SIDES - 1][t] = *(const d2 *)&Q[(u64)(r < nb ? r : nb - 1) * stride + xc];
+            if (GUARD && !in) v[0][t] = v[SIDES - 1][t] = d2{0.0, 0.0};
         }
     };
     const auto stage = [&](int buf) {
@@ -98,7 +99,7 @@ __global__ __launch_bounds__(SM_THREADS) void block_partial_kernel(const double2
 #pragma unroll
         for (int t = 0; t < NT; ++t)
 #pragma unroll
-            for (int h = 0; h < SIDES; ++h) lds[buf][h][(t * 16 + lr) * SM_ROW + lx] = v[h][t];
+            for (int h = 0; h < SIDES; ++h) lds[buf][h][(t * 16 + lr) * SM_ROW + lx] = cmk(v[h][t].x, v[h][t].y);
     };
     d4 re[NT], im[NT];
 #pragma unroll
