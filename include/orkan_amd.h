@@ -127,7 +127,8 @@ double orkan_event_ms(int a, int b);      /* elapsed ms between two recorded eve
  * launch shape and tuning choice above back to the built-in defaults (flags and lds_bytes unused),
  * 15 / 16: as 6 / 7 for complex64 storage (kernels 6 and 7 then apply to complex128 only),
  * 17: tile and workgroup size of the orkan_layer_1q sweeps (flags only: 0 2^12 amplitudes / 256
- * threads, 1 2^12 / 512, the default, 2 2^11 / 256, 3 2^11 / 512)), 18: as 9 for complex64 storage
+ * threads, 1 2^12 / 512, the default, from 21 qubits on with the tile in the registers of 256
+ * threads, 2 2^11 / 256, 3 2^11 / 512)), 18: as 9 for complex64 storage
  * (kernel 9 then applies to complex128 only), 19: statevector exp_diag (flags bits 0-1: log2 of the
  * amplitudes per thread, 0..2, bit 2: the shape of complex64 states, else of complex128 ones;
  * lds_bytes as below), 20: permutation / phase kernels (cx, cz, swap, ...) on complex64 states

@@ -25,6 +25,7 @@
 // LDS, the workgroups of one launch pull evaluations from an atomic counter
 // (largest first) and run each one start to finish.
 #include "k_common.hpp"
+#include "k_tile.hpp"
 
 namespace {
 
@@ -317,15 +318,9 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 // ---- tiles of 2^12 amplitudes in registers -----------------------------------------------------------
 // qaoa_persistent keeps its tile in LDS and takes it through registers and back for every three qubits and for the
 // phases: nine round trips per layer of a 20-qubit state, 288 B of LDS traffic per amplitude, half of its cycles bank
-// conflicts, and that was its time.  Here a workgroup of 256 threads holds the tile in registers, 16 amplitudes per
-// thread, in one of three layouts:
-//   layout 0: e = u | t << 4                     (register index u = tile bits 0-3)
-//   layout 1: e = (t & 15) | u << 4 | (t >> 4) << 8   (bits 4-7)
-//   layout 2: e = t | u << 8                     (bits 8-11)
-// An rx on four qubits, a phase, a load or a store happens in a layout without LDS; a change of layout moves the real
-// parts, then the imaginary parts, through one padded array of 2^12 doubles (34 KB: four workgroups per CU), written and
-// read without bank conflicts (one spare slot per 16).  A sweep of a 17- to 20-qubit state changes layout three times: 96
-// B per amplitude.
+// conflicts, and that was its time.  Here a workgroup of 256 threads holds the tile in registers (k_tile.hpp): an rx on
+// four qubits, a phase, a load or a store happens in one of the three layouts without LDS, and a sweep of a 17- to 20-qubit
+// state changes layout three times: 96 B of LDS traffic per amplitude.
 //
 // The sweeps are those of qaoa_persistent (k = 0..p, alternating contiguous and gathered tiles).  Sweep k finishes layer
 // k - 1 on tile bits ls..11 and runs layer k's phase and rx on every tile bit; the rx of one layer commute, so a sweep
@@ -338,7 +333,6 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 // and 33.8 with these tiles and a workgroup per evaluation.  It is bound by memory: 140 GB of amplitudes and cost
 // diagonal in runs of 256 and 128 B take 26 ms with everything else left out, the rest alone 14.  Nontemporal accesses gain
 // nothing.
-constexpr int RT_BITS = 12, RT_THREADS = 256;
 constexpr int RT_BATCH = 4;   // phases whose loads and sincos go together
 
 // a value that is the same in every lane, as a scalar: what is loaded by a computed index counts as per-lane otherwise, and
@@ -359,10 +353,6 @@ struct RxFlip {
         flip = fabs(c) < fabs(s);
         u = flip ? -c / s : s / c;
     }
-};
-// the thread's 16 amplitudes: two arrays, so that either half can change layout by itself
-struct Amps {
-    double re[16], im[16];
 };
 // sin and cos of x for |x| < 2^50: reduction to [-pi/4, pi/4] by the nearest multiple k of pi/2 with pi/2 as the sum of two
 // doubles (x - k P1 is exact in one fma: a multiple of 2^-52 below 1; the second fma rounds once; the sum is off by k
@@ -417,37 +407,6 @@ __device__ __forceinline__ void rx4(Amps &v, unsigned mask, double u) {
                 v.im[i] = fma(-uk, ar, bi);
             }
     }
-}
-
-// tile element of register u: lay_base + u * lay_step; its slot in LDS: lay_slot + u * lay_slot_step (one spare slot per 16
-// elements; in layout 0 the 16 elements of a thread are one such group)
-template <int LAY> __device__ __forceinline__ int lay_base(int t) {
-    return LAY == 0 ? t << 4 : LAY == 1 ? (t & 15) | (t >> 4) << 8 : t;
-}
-template <int LAY> __device__ __forceinline__ int lay_slot(int t) {
-    const int e = lay_base<LAY>(t);
-    return e + (e >> 4);
-}
-constexpr int lay_step(int lay) { return lay == 0 ? 1 : lay == 1 ? 16 : 256; }
-constexpr int lay_slot_step(int lay) { return lay == 0 ? 1 : lay == 1 ? 17 : 272; }
-
-template <int FROM, int TO>
-__device__ __forceinline__ void change_layout(Amps &v, double *lds) {
-    constexpr int ws = lay_slot_step(FROM), rs = lay_slot_step(TO);
-    double *w = lds + lay_slot<FROM>(threadIdx.x);
-    const double *r = lds + lay_slot<TO>(threadIdx.x);
-#pragma unroll
-    for (int u = 0; u < 16; ++u) w[u * ws] = v.re[u];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 16; ++u) v.re[u] = r[u * rs];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 16; ++u) w[u * ws] = v.im[u];
-    __syncthreads();
-#pragma unroll
-    for (int u = 0; u < 16; ++u) v.im[u] = r[u * rs];
-    __syncthreads();
 }
 
 // Memory index of a tile element: f(x) = (x >> ls) << 12 | (x & (2^ls - 1)) past the chunk's own offset in a gathered tile,
@@ -564,7 +523,7 @@ struct QaoaRec {
 __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_one_tile(const QaoaRec *__restrict__ recs,
                                                               const double *__restrict__ angles,
                                                               const double *__restrict__ diag, double *__restrict__ out) {
-    __shared__ double lds[(1 << RT_BITS) + (1 << RT_BITS) / 16];
+    __shared__ double lds[RT_SLOTS];
     __shared__ double red[RT_THREADS / 64];
     const int t = threadIdx.x;
     const QaoaRec r = recs[blockIdx.x];
@@ -622,7 +581,7 @@ struct SweepArgs {
 };
 
 __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
-    __shared__ double lds[(1 << RT_BITS) + (1 << RT_BITS) / 16];
+    __shared__ double lds[RT_SLOTS];
     __shared__ double red[RT_THREADS / 64];
     const int t = threadIdx.x, k = A.k;
     int c = 0;

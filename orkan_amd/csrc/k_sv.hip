@@ -7,6 +7,7 @@
 // memory traffic is the HBM stream every gate needs: the touched amplitudes are
 // read once and written once, 16 B per complex128 amplitude.
 #include "k_common.hpp"
+#include "k_tile.hpp"
 
 namespace {
 
@@ -807,9 +808,118 @@ __global__ __launch_bounds__(THREADS) void sv_layer_kernel(S *__restrict__ psi, 
 #undef LIDX
 }
 
-// tile bits and workgroup size of the layer sweeps: 0 (12, 256), 1 (12, 512), 2 (11, 256), 3 (11, 512).
-// Measured on 2^28 amplitudes: 8.2 / 4.9 / 10.0 / 15.3 ms per layer (complex128), 7.2 / 4.1 / 9.1 / 14.6
-// (complex64): 512 threads hold the tile's 8 amplitudes each, the register-resident path.
+// The same sweep with the tile of 2^12 amplitudes in registers (k_tile.hpp).  PASS 0: the contiguous tile,
+// qubits 0-11 in three layouts; PASS 1: a run of 2^r amplitudes, 4 <= r < 8, matrices on tile bits r..11 in two layouts;
+// PASS 2: r >= 8, one layout, no LDS.  The qubits above 11 go in equal shares, so the runs are 0.5 to 4 KB and each thread
+// has 16 loads in flight in four workgroups per CU; the LDS kernel moves 256 B runs, its last sweep a tile of as few as 32
+// amplitudes per workgroup, and every three qubits go through LDS.  Bound by memory: n = 25 (512 MB) 566 us, three sweeps
+// at 5.7 TB/s, against 857; n = 21 43 against 210, n = 23 158 against 391, n = 28 4.78 ms against 4.85 (complex64: 364
+// against 711, 48 / 220, 101 / 381, 3.28 / 3.97).  Below 2^21 amplitudes a launch is one round of workgroups and waits on
+// a single thread's chain, twice as long here as with 512 threads: n = 20 30 us against 25, n = 16 15 against 14.
+constexpr int LAYER_TILE_MIN = 21;
+struct TileLayerArgs {
+    double m[RT_BITS][8];   // per tile bit: m00, m01, m10, m11 (re, im), row-major
+    int r, lo;              // low run bits, global bit of tile bit r
+    unsigned mask;          // tile bits that carry a matrix
+};
+
+__device__ __forceinline__ void mats4(Amps &v, const double (*m)[8], unsigned mask) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        if (!((mask >> k) & 1)) continue;
+        const double *c = m[k];
+        const double ar = c[0], ai = c[1], br = c[2], bi = c[3], cr = c[4], ci = c[5], dr = c[6], di = c[7];
+#pragma unroll
+        for (int j = 0; j < 16; ++j)
+            if (!((j >> k) & 1)) {
+                const int i = j | (1 << k);
+                const double xr = v.re[j], xi = v.im[j], yr = v.re[i], yi = v.im[i];
+                v.re[j] = fma(-bi, yi, fma(br, yr, fma(ar, xr, -(ai * xi))));
+                v.im[j] = fma(bi, yr, fma(br, yi, fma(ar, xi, ai * xr)));
+                v.re[i] = fma(-di, yi, fma(dr, yr, fma(cr, xr, -(ci * xi))));
+                v.im[i] = fma(di, yr, fma(dr, yi, fma(cr, xi, ci * xr)));
+            }
+    }
+}
+
+template <typename S, int NT, int PASS>
+__global__ __launch_bounds__(RT_THREADS, 4) void sv_layer_tile_kernel(S *__restrict__ psi, TileLayerArgs a) {
+    __shared__ double lds[PASS == 2 ? 1 : RT_SLOTS];
+    constexpr int OUT = PASS == 2 ? 2 : 1;
+    const int tid = threadIdx.x;
+    const u64 t = blockIdx.x;
+    const int midb = a.lo - a.r;
+    const u64 base = (t & (((u64)1 << midb) - 1)) << a.r | (t >> midb) << (a.lo + RT_BITS - a.r);
+    const auto at = [&](int e) { return (u64)(e & ((1 << a.r) - 1)) | (u64)(e >> a.r) << a.lo; };
+    Amps v;
+    {
+        const S *p = psi + (base | at(lay_base<2>(tid)));
+        S raw[16];
+#pragma unroll
+        for (int u = 0; u < 16; ++u) raw[u] = ldr<NT>(p + at(u * lay_step(2)));
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const cd x = to_cd(raw[u]);
+            v.re[u] = x.x;
+            v.im[u] = x.y;
+        }
+    }
+    mats4(v, a.m + 8, a.mask >> 8);
+    if (PASS == 0) {
+        change_layout<2, 0>(v, lds);
+        mats4(v, a.m, a.mask);
+        change_layout<0, 1>(v, lds);
+        mats4(v, a.m + 4, a.mask >> 4);
+    }
+    if (PASS == 1) {
+        change_layout<2, 1>(v, lds);
+        mats4(v, a.m + 4, a.mask >> 4);
+    }
+    // the stores' addresses are formed anew: kept from the loads, they spill
+    int wid = tid;
+    asm volatile("" : "+v"(wid));
+    S *p = psi + (base | at(lay_base<OUT>(wid)));
+#pragma unroll
+    for (int u = 0; u < 16; ++u) stx<NT>(p + at(u * lay_step(OUT)), cmk(v.re[u], v.im[u]));
+}
+
+template <typename S>
+int sv_layer_tiles(hipStream_t st, S *psi, int n, bool nt, const double *mats) {
+    const unsigned grid = 1u << (n - RT_BITS);
+    TileLayerArgs a{};
+    a.r = a.lo = RT_BITS;
+    a.mask = (1u << RT_BITS) - 1;
+    for (int q = 0; q < RT_BITS; ++q)
+        for (int i = 0; i < 8; ++i) a.m[q][i] = mats[8 * q + i];
+    if (nt) sv_layer_tile_kernel<S, 1, 0><<<grid, RT_THREADS, 0, st>>>(psi, a);
+    else sv_layer_tile_kernel<S, 0, 0><<<grid, RT_THREADS, 0, st>>>(psi, a);
+    ORK_LAUNCH_CHECK();
+    // the qubits above in equal shares of at most 8, so that the runs are as long as they can be
+    const int left = n - RT_BITS, sweeps = (left + 7) / 8;
+    for (int k = 0, lo = RT_BITS; k < sweeps; ++k) {
+        const int g = (left * (k + 1)) / sweeps - (left * k) / sweeps;
+        TileLayerArgs b{};
+        b.r = RT_BITS - g;
+        b.lo = lo;
+        b.mask = ((1u << g) - 1) << b.r;
+        for (int j = 0; j < g; ++j)
+            for (int i = 0; i < 8; ++i) b.m[b.r + j][i] = mats[8 * (lo + j) + i];
+        if (g <= 4) {
+            if (nt) sv_layer_tile_kernel<S, 1, 2><<<grid, RT_THREADS, 0, st>>>(psi, b);
+            else sv_layer_tile_kernel<S, 0, 2><<<grid, RT_THREADS, 0, st>>>(psi, b);
+        } else {
+            if (nt) sv_layer_tile_kernel<S, 1, 1><<<grid, RT_THREADS, 0, st>>>(psi, b);
+            else sv_layer_tile_kernel<S, 0, 1><<<grid, RT_THREADS, 0, st>>>(psi, b);
+        }
+        ORK_LAUNCH_CHECK();
+        lo += g;
+    }
+    return 0;
+}
+
+// tile bits and workgroup size of the layer sweeps: 0 (12, 256), 1 (12, 512; from LAYER_TILE_MIN qubits on the register
+// tiles), 2 (11, 256), 3 (11, 512).  Measured on 2^28 amplitudes with tiles in LDS: 8.2 / 4.9 / 10.0 / 15.3 ms per layer
+// (complex128), 7.2 / 4.1 / 9.1 / 14.6 (complex64): 512 threads hold 8 amplitudes each, loaded and stored without LDS.
 constexpr int kLayerVariant = 1;
 static int g_layer_variant = kLayerVariant;
 
@@ -824,6 +934,7 @@ template <typename S>
 int sv_layer(hipStream_t st, void *psi, int n, const double *mats) {
     const bool nt = !(g_nt_off & 1) && ((u64)sizeof(S) << n) >= g_nt_min_bytes;
     const int v = g_layer_variant, LTv = v >= 2 ? 11 : 12;
+    if (v == 1 && n >= LAYER_TILE_MIN) return sv_layer_tiles<S>(st, (S *)psi, n, nt, mats);
     auto launch = [&](const LayerArgs &a) {
         switch (v) {
         case 1: launch_layer<S, 12, 512>(st, psi, n, nt, a); break;

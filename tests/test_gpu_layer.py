@@ -8,6 +8,7 @@ import pytest
 
 import engines
 import orkan_amd
+from orkan_amd._ffi import StateT
 from linalg_np import MIXED_TILED, PURE
 
 pytestmark = pytest.mark.gpu
@@ -130,3 +131,38 @@ def test_layer_errors(eng):
     dm = eng.plus(MIXED_TILED, 4)
     assert api.orkan_layer_1q(C.byref(dm), m.ctypes.data) == -4   # QS_ERR_TYPE: pure states only
     eng.free(dm)
+
+
+@pytest.mark.parametrize("n,f32", [(21, 0), (21, 1), (22, 0), (24, 1), (25, 0), (27, 1)])
+def test_layer_register_tiles(eng, n, f32):
+    """The sweeps with tiles in registers, from their smallest size on: shares of 4 and 5, 5 and 5, 6 and 6, 6 and 7, 7 and
+    8 qubits above the contiguous tile's 12 (the last two with nontemporal accesses).  The state is a product of
+    n different qubit states, so the result is the product of the transformed ones.  A 2x2 product is off by at most 4
+    roundings of a pair's norm, a factor of the reference by 2: together less than 27 x 6 x 1.1e-16 of the state's norm of
+    1; complex64 storage adds 6e-8 of it at the start and per sweep (unitaries keep what was added before)."""
+    rng = np.random.default_rng(n)
+    mats = _unitaries(rng, n)
+    qubits = rng.standard_normal((n, 2)) + 1j * rng.standard_normal((n, 2))
+    qubits /= np.linalg.norm(qubits, axis=1)[:, None]
+
+    def product(vs):
+        out = np.ones(1, np.complex128)
+        for v in vs:
+            out = (v[:, None] * out[None, :]).reshape(-1)
+        return out
+
+    st = eng.new(PURE, n, product(qubits))
+    if f32:
+        s32 = eng.api.orkan_state_convert(C.byref(st), 1)
+        eng.free(st)
+        st = s32
+    m = _colmajor(mats)
+    assert eng.api.orkan_layer_1q(C.byref(st), m.ctypes.data) == 0
+    if f32:
+        back = eng.api.orkan_state_convert(C.byref(st), 0)
+        eng.free(st)
+        st = back
+    got = eng.read(st)
+    eng.free(st)
+    ref = product([mq @ v for mq, v in zip(mats, qubits)])
+    assert np.linalg.norm(got - ref) <= (4 * 6e-8 if f32 else 1e-13)
