@@ -24,6 +24,7 @@
 // src/gate/tiled/gate_tiled_h.c:28-225, src/channel/channel_tiled.c:52-185,
 // src/gate/tiled/gate_tiled_2q.c:3).
 #include "k_common.hpp"
+#include "k_reduce.hpp"
 
 namespace {
 
@@ -1739,43 +1740,15 @@ __global__ __launch_bounds__(DM_THREADS) void sincos_kernel(double2 *__restrict_
 }
 
 // ---- mean: sum_x obs[x] Re rho_xx ---------------------------------------------------------
-constexpr int RED_BLOCKS = 2048;   // same partials layout as the statevector reductions
-
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
-}
+static_assert(RED_THREADS == DM_THREADS, "put_partial's workgroups");
 
 template <typename S, int LAYOUT>
 __global__ __launch_bounds__(DM_THREADS) void dm_mean_kernel(const S *__restrict__ rho, DmPlan p,
                                                              const double *__restrict__ obs, double *__restrict__ part) {
-    __shared__ double red[DM_THREADS / 64];
-    double acc = 0.0;
+    double acc[1] = {0.0};
     for (u64 x = (u64)blockIdx.x * DM_THREADS + threadIdx.x; x < p.dim; x += (u64)gridDim.x * DM_THREADS)
-        acc += obs[x] * ldc(rho + elem_off<LAYOUT>(p, x, x)).x;
-    acc = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int i = 0; i < DM_THREADS / 64; ++i) s += red[i];
-        part[blockIdx.x] = s;
-    }
-}
-
-__global__ __launch_bounds__(DM_THREADS) void dm_finish_kernel(double *__restrict__ part, int nblk) {
-    __shared__ double red[DM_THREADS / 64];
-    double acc = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += DM_THREADS) acc += part[b];
-    acc = wave_sum(acc);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double s = 0.0;
-        for (int i = 0; i < DM_THREADS / 64; ++i) s += red[i];
-        part[RED_BLOCKS] = s;
-    }
+        acc[0] += obs[x] * ldc(rho + elem_off<LAYOUT>(p, x, x)).x;
+    put_partial<1>(acc, part);
 }
 
 // ---- host-side planning -------------------------------------------------------------------
@@ -2516,9 +2489,8 @@ extern "C" int ork_dm_mean(void *stream, int prec, int layout, int log_tile, con
         else dm_mean_kernel<double2, ORK_TILED><<<(unsigned)nb, DM_THREADS, 0, st>>>((const double2 *)rho, p, obs, part);
     }
     ORK_LAUNCH_CHECK();
-    dm_finish_kernel<<<1, DM_THREADS, 0, st>>>(part, (int)nb);
-    ORK_LAUNCH_CHECK();
-    hipError_t e = hipMemcpyAsync(out, part + RED_BLOCKS, sizeof(double), hipMemcpyDeviceToHost, st);
+    const hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) return (int)e;
-    return (int)hipStreamSynchronize(st);
+    add_partials<1>(part, (int)nb, out);
+    return 0;
 }

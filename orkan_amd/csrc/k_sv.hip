@@ -7,14 +7,13 @@
 // memory traffic is the HBM stream every gate needs: the touched amplitudes are
 // read once and written once, 16 B per complex128 amplitude.
 #include "k_common.hpp"
+#include "k_reduce.hpp"
 #include "k_tile.hpp"
 
 namespace {
 
 constexpr int SV_THREADS = 256;
 constexpr int SV_UNROLL = 2;      // bases per thread in the permutation kernel (doubled for complex64)
-constexpr int RED_THREADS = 256;
-constexpr int RED_BLOCKS = 2048;  // room for first-stage partials; their count depends only on the size and shape
 
 struct Coef {
     double v[8];
@@ -476,33 +475,6 @@ __global__ __launch_bounds__(SV_THREADS) void sv_exp_diag_kernel(S *__restrict__
 }
 
 // ---- reductions ---------------------------------------------------------------------------
-__device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
-}
-
-// block-wide sum of NV values; result valid in thread 0
-template <int NV>
-__device__ __forceinline__ void block_sum(double (&v)[NV]) {
-    __shared__ double red[NV][RED_THREADS / 64];
-    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        v[i] = wave_sum(v[i]);
-        if (lane == 0) red[i][wv] = v[i];
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            double s = 0.0;
-            for (int w = 0; w < RED_THREADS / 64; ++w) s += red[i][w];
-            v[i] = s;
-        }
-    }
-}
-
 // U independent accumulators per thread: x, x + G, ..., x + (U-1)G (G = grid stride) are loaded
 // together, so each thread keeps U loads in flight; they are added in that fixed order.
 template <int U>
@@ -534,8 +506,7 @@ __global__ __launch_bounds__(RED_THREADS) void sv_mean_kernel(const S *__restric
         for (int u = 0; u < U; ++u) a4[u] += o[u] * (a[u].x * a[u].x + a[u].y * a[u].y);
     }
     double acc[1] = {sum_fixed<U>(a4)};
-    block_sum<1>(acc);
-    if (threadIdx.x == 0) part[blockIdx.x] = acc[0];
+    put_partial<1>(acc, part);
 }
 
 template <typename S, int NT, int U>
@@ -564,26 +535,7 @@ __global__ __launch_bounds__(RED_THREADS) void sv_matel_kernel(const S *__restri
         }
     }
     double acc[2] = {sum_fixed<U>(re4), sum_fixed<U>(im4)};
-    block_sum<2>(acc);
-    if (threadIdx.x == 0) {
-        part[2 * blockIdx.x] = acc[0];
-        part[2 * blockIdx.x + 1] = acc[1];
-    }
-}
-
-// second stage: nv interleaved sums over nblk partials, written after the partials
-template <int NV>
-__global__ __launch_bounds__(RED_THREADS) void finish_kernel(double *__restrict__ part, int nblk) {
-    double acc[NV];
-#pragma unroll
-    for (int i = 0; i < NV; ++i) acc[i] = 0.0;
-    for (int b = threadIdx.x; b < nblk; b += RED_THREADS)
-#pragma unroll
-        for (int i = 0; i < NV; ++i) acc[i] += part[NV * b + i];
-    block_sum<NV>(acc);
-    if (threadIdx.x == 0)
-#pragma unroll
-        for (int i = 0; i < NV; ++i) part[NV * RED_BLOCKS + i] = acc[i];
+    put_partial<2>(acc, part);
 }
 
 template <typename S, int OP, int U, int XCD, int NT>
@@ -973,7 +925,7 @@ int sv_layer(hipStream_t st, void *psi, int n, const double *mats) {
 }  // namespace
 
 // ---- C ABI --------------------------------------------------------------------------------
-extern "C" uint64_t ork_partials_len(void) { return 2 * RED_BLOCKS + 2; }
+extern "C" uint64_t ork_partials_len(void) { return 2 * RED_BLOCKS; }
 
 // mats: n x 8 doubles, the row-major 2x2 matrix of each qubit (re, im interleaved)
 extern "C" int ork_sv_layer(void *stream, int prec, void *psi, int n, const double *mats) {
@@ -1312,11 +1264,10 @@ extern "C" int ork_sv_mean(void *stream, int prec, const void *psi, int n, const
         else launch_mean<double2, 0>(st, nb, psi, obs, dim, part);
     }
     ORK_LAUNCH_CHECK();
-    finish_kernel<1><<<1, RED_THREADS, 0, st>>>(part, nb);
-    ORK_LAUNCH_CHECK();
-    hipError_t e = hipMemcpyAsync(out, part + RED_BLOCKS, sizeof(double), hipMemcpyDeviceToHost, st);
+    const hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) return (int)e;
-    return (int)hipStreamSynchronize(st);
+    add_partials<1>(part, nb, out);
+    return 0;
 }
 
 extern "C" int ork_sv_matel(void *stream, int prec, const void *bra, const void *ket, int n, const double *obs,
@@ -1333,9 +1284,8 @@ extern "C" int ork_sv_matel(void *stream, int prec, const void *bra, const void 
         else launch_matel<double2, 0>(st, nb, bra, ket, obs, dim, part);
     }
     ORK_LAUNCH_CHECK();
-    finish_kernel<2><<<1, RED_THREADS, 0, st>>>(part, nb);
-    ORK_LAUNCH_CHECK();
-    hipError_t e = hipMemcpyAsync(out, part + 2 * RED_BLOCKS, 2 * sizeof(double), hipMemcpyDeviceToHost, st);
+    const hipError_t e = hipStreamSynchronize(st);
     if (e != hipSuccess) return (int)e;
-    return (int)hipStreamSynchronize(st);
+    add_partials<2>(part, nb, out);
+    return 0;
 }

@@ -35,7 +35,7 @@ void ork_hip_fail(const char *where, int err);
 
 typedef struct {
     void *stream;
-    double *partials;      /* reduction partial sums */
+    double *partials;      /* reduction partial sums, pinned host memory */
     void *stage;           /* device copy of a caller's obs / diag array */
     size_t stage_bytes;
     void *phase;           /* exp_diag per-index phases */

@@ -67,10 +67,12 @@ int ork_sv_1q(void *stream, int prec, void *psi_dev, int n, int q, int op, const
 int ork_sv_layer(void *stream, int prec, void *psi_dev, int n, const double *mats);
 int ork_sv_mono(void *stream, int prec, void *psi_dev, int n, const ork_mono_t *m);
 int ork_sv_exp_diag(void *stream, int prec, void *psi_dev, int n, const double *diag_dev, double t);
+/* the reductions: `partials` (ork_partials_len() doubles of pinned host memory) is scratch of one call at a time; the
+ * call returns when *out holds the sum */
 int ork_sv_mean(void *stream, int prec, const void *psi_dev, int n, const double *obs_dev,
-                double *partials_dev, double *out_host);
+                double *partials, double *out);
 int ork_sv_matel(void *stream, int prec, const void *bra_dev, const void *ket_dev, int n,
-                 const double *obs_dev, double *partials_dev, double *out_host);
+                 const double *obs_dev, double *partials, double *out);
 
 /* rho -> op(rho) on the packed or tiled layout */
 int ork_dm_group(void *stream, int prec, int layout, int log_tile, void *rho_dev, int n,
@@ -82,7 +84,7 @@ int ork_dm_phase(void *stream, int prec, int layout, int log_tile, void *rho_dev
 int ork_dm_exp_diag(void *stream, int prec, int layout, int log_tile, void *rho_dev, int n,
                     const double *diag_dev, double t, void *phase_dev);
 int ork_dm_mean(void *stream, int prec, int layout, int log_tile, const void *rho_dev, int n,
-                const double *obs_dev, double *partials_dev, double *out_host);
+                const double *obs_dev, double *partials, double *out);
 
 /* Allocation-free exp_diag: the phase scratch of a density matrix is a fixed device array of
  * 2^ORK_NOALLOC_MAX_QUBITS complex128 (k_noalloc.hip).  ork_noalloc_setup takes that array's
@@ -111,7 +113,7 @@ void ork_dm_reset_shapes(void);
 void ork_sv_reset_tuning(void);
 void ork_mlp_gemm_reset(void);
 
-/* number of doubles the *_mean / matel launchers need in partials_dev */
+/* number of doubles the *_mean / matel launchers need in partials */
 uint64_t ork_partials_len(void);
 
 /* dst (packed or tiled, len stored entries) <- the logical density matrix of src (pure: |psi><psi|,

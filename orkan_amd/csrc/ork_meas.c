@@ -1,8 +1,8 @@
 /*
- * ork_meas.c -- mean and matel_diag: two-stage deterministic reductions on the
- * device (per-workgroup partial sums in a fixed order, then one workgroup),
- * validated like src/meas/meas.c:23-74.  `obs` may be a host array (staged into
- * HBM) or a device array from orkan_dev_alloc (used in place).
+ * ork_meas.c -- mean and matel_diag: deterministic reductions (per-workgroup
+ * partial sums on the device, added on the host in a fixed order), validated
+ * like src/meas/meas.c:23-74.  `obs` may be a host array (staged into HBM) or a
+ * device array from orkan_dev_alloc (used in place).
  */
 #include "ork_host.h"
 #include "orkan_backend.h"

@@ -37,7 +37,8 @@ ork_dev_t *ork_dev(void) {
             hipStream_t st;
             ORK_HIP("hipStreamCreateWithFlags", hipStreamCreateWithFlags(&st, hipStreamNonBlocking));
             d->stream = (void *)st;
-            ORK_HIP("hipMalloc(partials)", hipMalloc((void **)&d->partials, ork_partials_len() * sizeof(double)));
+            ORK_HIP("hipHostMalloc(partials)", hipHostMalloc((void **)&d->partials, ork_partials_len() * sizeof(double),
+                                                             hipHostMallocDefault));
             /* device address of the allocation-free exp_diag's scratch array on this device; a failure
              * leaves it unset, and only orkan_exp_diag_noalloc reports it */
             d->noalloc_err = ork_noalloc_setup();

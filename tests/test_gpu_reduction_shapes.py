@@ -58,3 +58,46 @@ def test_reduction_shapes_match_oracle(n, fp32):
         assert dev.api.orkan_set_launch_shape(RESET_HOOK, 0, 0) == 0
         dev.free(a)
         dev.free(b)
+
+
+def test_alternating_sizes_and_threads():
+    """Every call's partial sums share one host buffer: values of one workgroup (n <= 11, 8 for a density matrix), two,
+    the most, and again, from one thread and from four at once, are those of the first call to the bit and the sums of
+    numpy to 2^n roundings of terms below 1 in all (n 1.1e-16 for pairwise sums, taken as 1e-13)."""
+    import threading
+
+    from linalg_np import MIXED_PACKED, MIXED_TILED
+    dev = engines.DeviceEngine(orkan_amd.lib_path(5), 5)
+    work = []
+    for kind, n in ((PURE, 1), (PURE, 11), (PURE, 12), (PURE, 13), (PURE, 19), (PURE, 20), (MIXED_TILED, 8),
+                    (MIXED_PACKED, 9), (MIXED_PACKED, 10)):
+        g = wl.rng(900 + n)
+        obs = g.uniform(-1, 1, 1 << n)
+        if kind == PURE:
+            psi = g.standard_normal(1 << n) + 1j * g.standard_normal(1 << n)
+            psi /= np.linalg.norm(psi)
+            st, ref = dev.new(kind, n, psi), float(np.sum(obs * np.abs(psi) ** 2))
+        else:
+            st, ref = dev.plus(kind, n), float(np.sum(obs)) / (1 << n)
+        work.append((st, obs, ref))
+    first = [dev.mean(st, obs) for st, obs, _ in work]
+    for got, (_, _, ref) in zip(first, work):
+        assert abs(got - ref) <= 1e-13
+    wrong = []
+
+    def run(seed):
+        order = np.random.default_rng(seed).permutation(np.repeat(np.arange(len(work)), 5))
+        for i in order:
+            got = dev.mean(work[i][0], work[i][1])
+            if got != first[i]:
+                wrong.append((int(i), got, first[i]))
+
+    run(0)
+    threads = [threading.Thread(target=run, args=(k,)) for k in range(1, 5)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not wrong, wrong[:3]
+    for st, _, _ in work:
+        dev.free(st)
