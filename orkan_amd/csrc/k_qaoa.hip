@@ -17,7 +17,8 @@
 // each sweep finishes the previous layer's rx on the qubits the
 // previous sweep could not reach and runs the next layer's exp_diag and rx on
 // every qubit it holds: p + 1 sweeps for p layers instead of p (n + 1) gate
-// passes; the last sweep reduces sum_x C(x) |psi_x|^2.
+// passes; the last sweep reduces sum_x C(x) |psi_x|^2.  Where C(x) = C(~x), half of a state larger than a tile
+// stands for all of it.
 //
 // Two forms. qaoa_sweep and qaoa_one_tile, the default: tiles of 2^12 amplitudes
 // in registers, one launch per sweep with a workgroup for every tile of every
@@ -327,13 +328,22 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 // visits the layouts in the order that needs fewest changes: 1 (load, finish bits 4-7), 0 (finish bits 0-3, only where
 // ls < 4), 2 (finish bits 8-11, phase, rx), 0 (rx), 1 (rx, store); with ls >= 8 it starts in layout 2.
 // A launch is one sweep k over all tiles of all states that have it, so a single large state fills the chip as well as a
-// thousand do: with a workgroup per evaluation one state of 18 qubits took 2180 us, now 99; 64 of 16 qubits 632 and 209;
-// six of 21 to 24 qubits 185 and 5.2 ms; 300 of 4 to 11 qubits (qaoa_one_tile) 231 and 213.  4096 evaluations of 10 to 20
-// qubits and 1 to 8 layers: 29.0 ms a call, some 3 of them on the host, against 38.8 with the best shape of qaoa_persistent
-// and 33.8 with these tiles and a workgroup per evaluation.  It is bound by memory: 140 GB of amplitudes and cost
+// thousand do: with a workgroup per evaluation one state of 18 qubits took 2180 us, now 99; 300 of 4 to 11 qubits
+// (qaoa_one_tile) 231 and 213; with SYM = 0, 64 of 16 qubits 632 and 209, six of 21 to 24 qubits 185 and 5.2 ms, 4096
+// evaluations of 10 to 20 qubits and 1 to 8 layers 38.8 and 29.0 ms a call.  Memory bounds it: 140 GB of amplitudes and cost
 // diagonal in runs of 256 and 128 B take 26 ms with everything else left out, the rest alone 14.  Nontemporal accesses gain
 // nothing.
-constexpr int RT_BATCH = 4;   // phases whose loads and sincos go together
+//
+// SYM = 1: half of the state, for a cost with C(x) = C(~x) (any sum of pair terms: MaxCut).  |+>, the phases and the rx all
+// keep psi(x) = psi(~x), so m = n - 1 bits y name an amplitude: y_i = x_i ^ x_(n-1) for i < 12, y_i = x_i ^ x_v for i >= 12,
+// with v the qubit of bit vb < 5.  The X of qubits i < n - 1 other than v flips y_i alone.  The X of qubit n - 1 flips y_0 to y_11,
+// all inside a contiguous tile; that of v flips y_vb and y_12 to y_(m-1), all inside a gathered tile, whose low run holds bit vb.
+// So either sweep still reaches what the other leaves: the contiguous one bits 0-11 without vb and qubit n - 1, the gathered
+// one its tile's bits without vb and qubit v; the two wide flips ride on a change of layout (change_layout_flip).  The state
+// of x_(n-1) = 0 has C(y) at y, with bits 12.. complemented where y_vb = 1: in runs of 2^vb, 128 B up to 20 qubits.  The
+// product of a layer's X over all qubits is 1 here, so RxFlip.flip is not needed.  Half the bytes and the work:
+// 4096 evaluations of 10 to 20 qubits 29.0 -> 16.8 ms a call (3 of them on the host), 64 of 16 qubits 212 -> 163 us, 700 of 12
+// to 17 1.57 -> 1.04 ms, six of 21 to 24 5.5 -> 2.0 ms, one of 18 99 us both ways.
 
 // a value that is the same in every lane, as a scalar: what is loaded by a computed index counts as per-lane otherwise, and
 // with it every branch and address that depends on it
@@ -467,8 +477,8 @@ struct Diag {
     }
 };
 
-// the phases of the thread's 16 amplitudes in layout LAY
-template <int LAY, int SMALL>
+// the phases of the thread's 16 amplitudes in layout LAY, RT_BATCH loads and sincos at a time
+template <int LAY, int SMALL, int RT_BATCH = 4>
 __device__ __forceinline__ void phase16(Amps &v, const Diag &C, const TileMap &m, unsigned off, double g) {
 #pragma unroll
     for (int u0 = 0; u0 < 16; u0 += RT_BATCH) {
@@ -516,18 +526,20 @@ struct QaoaRec {
     u64 diag_off;    // of C in the diagonal arena (doubles)
     u64 tile;        // of its first tile in the state slots (tiles of 2^12 amplitudes)
     int angle_off;   // of its per-layer (gamma, cos beta, sin beta)
-    int p, n, out;   // layers, qubits, place of its result
+    int p, n, m;     // layers, qubits, bits of the stored index: n, or n - 1 (SYM)
+    int out, pad;    // place of its result
 };
 
 // states of at most one tile: a workgroup runs the whole circuit
-__global__ __launch_bounds__(RT_THREADS, 3) void qaoa_one_tile(const QaoaRec *__restrict__ recs,
+template <int SYM>
+__global__ __launch_bounds__(RT_THREADS, SYM ? 2 : 3) void qaoa_one_tile(const QaoaRec *__restrict__ recs,
                                                               const double *__restrict__ angles,
                                                               const double *__restrict__ diag, double *__restrict__ out) {
     __shared__ double lds[RT_SLOTS];
     __shared__ double red[RT_THREADS / 64];
     const int t = threadIdx.x;
     const QaoaRec r = recs[blockIdx.x];
-    const int n = r.n, p = r.p;
+    const int n = uni(r.m), p = uni(r.p);
     const double *ang = angles + r.angle_off;
     Diag C{buffer(diag + r.diag_off, (u64)8 << n), (1u << n) - 1, false};
     // layouts 2 and 1 take turns in holding the phase, 0 in between.  Amplitudes past 2^n are 0 and stay 0 (their bits carry
@@ -548,28 +560,30 @@ __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_one_tile(const QaoaRec *__
         if (l & 1) {
             phase16<1, 1>(v, C, m, (unsigned)lay_base<1>(t), g);
             rx4(v, b1, rx.u);
-            change_layout<1, 0>(v, lds);
+            if (SYM) change_layout_flip<1, 0>(v, lds, C.last, rx.u);
+            else change_layout<1, 0>(v, lds);
             rx4(v, b0, rx.u);
             change_layout<0, 2>(v, lds);
             rx4(v, b2, rx.u);
         } else {
             phase16<2, 1>(v, C, m, (unsigned)t, g);
             rx4(v, b2, rx.u);
-            change_layout<2, 0>(v, lds);
+            if (SYM) change_layout_flip<2, 0>(v, lds, C.last, rx.u);
+            else change_layout<2, 0>(v, lds);
             rx4(v, b0, rx.u);
             change_layout<0, 1>(v, lds);
             rx4(v, b1, rx.u);
         }
-        C.flip ^= rx.flip;
+        if (!SYM) C.flip ^= rx.flip;
     }
     const double acc = p & 1 ? mean16<1, 1>(v, C, m, (unsigned)lay_base<1>(t)) : mean16<2, 1>(v, C, m, (unsigned)t);
     const double tot = block_sum<RT_THREADS>(acc, red);
-    if (t == 0) out[r.out] = tot * rx_scale(ang, p, n);
+    if (t == 0) out[r.out] = tot * rx_scale(ang, p, r.n);
 }
 
 // One sweep k of every larger state that has it (p >= k): a workgroup per tile.  The evaluations are sorted by qubits, then
 // by layers, both descending, so the tiles of a sweep are a few runs of equal 2^(n - 12).
-constexpr int RT_CLASSES = 12;   // 13 to 24 qubits
+constexpr int RT_CLASSES = 12;   // 13 to 24 index bits
 struct SweepArgs {
     const QaoaRec *recs;
     const double *angles, *diag;
@@ -577,9 +591,10 @@ struct SweepArgs {
     double *part;                     // per tile of the slots: its share of the mean
     int k, nclass;
     unsigned first[RT_CLASSES + 1];   // first workgroup of each class
-    int rec[RT_CLASSES], n[RT_CLASSES];
+    int rec[RT_CLASSES], n[RT_CLASSES];   // first record and index bits of each
 };
 
+template <int SYM>
 __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
     __shared__ double lds[RT_SLOTS];
     __shared__ double red[RT_THREADS / 64];
@@ -590,10 +605,10 @@ __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
     const unsigned b = blockIdx.x - A.first[c], ch = b & ((1u << (n - RT_BITS)) - 1);
     const QaoaRec r = A.recs[A.rec[c] + (int)(b >> (n - RT_BITS))];
     const double *ang = A.angles + r.angle_off;
-    const bool gathered = k & 1, last = k == r.p;
+    const bool gathered = k & 1, last = k == uni(r.p);
     // the flips of the layers before k
     bool flip = false;
-    for (int l = 0; l < k; ++l) flip ^= fabs(uni(ang[3 * l + 1])) < fabs(uni(ang[3 * l + 2]));
+    for (int l = 0; !SYM && l < k; ++l) flip ^= fabs(uni(ang[3 * l + 1])) < fabs(uni(ang[3 * l + 2]));
     const Diag C{buffer(A.diag + r.diag_off, (u64)8 << n), (1u << n) - 1, flip};
     const double g = last ? 0.0 : uni(ang[3 * k]);
     const RxFlip rx(last ? 1.0 : uni(ang[3 * k + 1]), last ? 0.0 : uni(ang[3 * k + 2]));
@@ -606,6 +621,12 @@ __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
     const TileMap m{ch << (gathered ? ls : RT_BITS), gathered ? ls : RT_BITS};
     const unsigned off2 = m.f((unsigned)t), soff1 = slot_off(m.f((unsigned)lay_base<1>(t))), soff2 = slot_off(off2);
     const Buf S = buffer(A.states + (r.tile << RT_BITS), (u64)16 << n);
+    // SYM: the bit of qubit v; the tile bits that the X of qubit n - 1 or v, whichever is in reach, flips; the place in
+    // the diagonal
+    const int vb = ls < 5 ? ls - 1 : 4;
+    const unsigned all = SYM ? (RT_SIZE - 1) & ~(1u << vb) : RT_SIZE - 1;
+    const unsigned cross = gathered ? (RT_SIZE - 1) & (~0u << ls | 1u << vb) : RT_SIZE - 1;
+    const unsigned coff2 = SYM && (off2 >> vb & 1) ? off2 ^ (C.last & ~(RT_SIZE - 1)) : off2;
     Amps v;
     if (k == 0) {
         const double amp = 1.0 / sqrt((double)(1u << n));
@@ -621,27 +642,40 @@ __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
             if (f0) {
                 change_layout<1, 0>(v, lds);
                 rx4(v, f0, rxp.u);
-                change_layout<0, 2>(v, lds);
+                if (SYM) change_layout_flip<0, 2>(v, lds, cross, rxp.u);
+                else change_layout<0, 2>(v, lds);
             } else {
-                change_layout<1, 2>(v, lds);
+                if (SYM) change_layout_flip<1, 2>(v, lds, cross, rxp.u);
+                else change_layout<1, 2>(v, lds);
             }
         } else {
             load_amps<2>(v, S, m, soff2);
+            if (SYM) change_layout_flip<2, 2>(v, lds, cross, rxp.u);
         }
         rx4(v, f2, rxp.u);
     }
-    if (last) {
-        const double tot = block_sum<RT_THREADS>(mean16<2, 0>(v, C, m, off2), red);
-        if (t == 0) A.part[r.tile + ch] = tot;
-        return;
+    double acc = 0.0;
+    if (!last) {
+        phase16<2, 0, SYM ? 2 : 4>(v, C, m, coff2, g);   // 4 spill beside change_layout_flip
+        rx4(v, 15u, rx.u);
+        if (SYM) change_layout_flip<2, 0>(v, lds, cross, rx.u);
+        else change_layout<2, 0>(v, lds);
+        rx4(v, all & 15u, rx.u);
+        change_layout<0, 1>(v, lds);
+        rx4(v, all >> 4 & 15u, rx.u);
+        // formed anew: kept from the loads it spills
+        int t1 = t;
+        asm volatile("" : "+v"(t1));
+        store_amps<1>(v, S, m, slot_off(m.f((unsigned)lay_base<1>(t1))));
+    } else {
+        acc = mean16<2, 0>(v, C, m, coff2);
     }
-    phase16<2, 0>(v, C, m, off2, g);
-    rx4(v, 15u, rx.u);
-    change_layout<2, 0>(v, lds);
-    rx4(v, 15u, rx.u);
-    change_layout<0, 1>(v, lds);
-    rx4(v, 15u, rx.u);
-    store_amps<1>(v, S, m, soff1);
+    // apart from the branch above: with a divergent branch inside, the compiler keeps the amplitudes of one side alive
+    // across the other
+    if (last) {
+        const double tot = block_sum<RT_THREADS>(acc, red);
+        if (t == 0) A.part[r.tile + ch] = tot;
+    }
 }
 
 // the tiles' shares of each mean, in a fixed order
@@ -650,7 +684,7 @@ __global__ __launch_bounds__(256) void qaoa_finish(const QaoaRec *__restrict__ r
     __shared__ double red[4];
     const QaoaRec r = recs[blockIdx.x];
     double acc = 0.0;
-    for (int i = threadIdx.x; i < 1 << (r.n - RT_BITS); i += 256) acc += part[r.tile + (u64)i];
+    for (int i = threadIdx.x; i < 1 << (r.m - RT_BITS); i += 256) acc += part[r.tile + (u64)i];
     const double tot = block_sum<256>(acc, red);
     if (threadIdx.x == 0) out[r.out] = tot * rx_scale(angles + r.angle_off, r.p, r.n);
 }
@@ -671,25 +705,35 @@ __global__ __launch_bounds__(256) void maxcut_diag_kernel(double *__restrict__ o
     out[x] = acc;
 }
 
-// cmax[g] = the largest |C| of graph g, infinity if any is not finite
-__global__ __launch_bounds__(256) void diag_max_kernel(const QaoaGraph *__restrict__ graphs, const double *__restrict__ diag,
-                                                       double *__restrict__ cmax) {
+// info[2 g] = the largest |C| of graph g, infinity if any is not finite; info[2 g + 1] = 1 if C(x) = C(~x) for every x, else 0
+__global__ __launch_bounds__(256) void diag_info_kernel(const QaoaGraph *__restrict__ graphs, const double *__restrict__ diag,
+                                                        double *__restrict__ info) {
     __shared__ double red[256];
+    __shared__ int differ;
     const QaoaGraph g = graphs[blockIdx.x];
     const double *C = diag + g.diag_off;
+    const u64 N = (u64)1 << g.n;
     double m = 0.0;
+    bool diff = false;
+    if (threadIdx.x == 0) differ = 0;
+    __syncthreads();
 #pragma unroll 4
-    for (u64 x = threadIdx.x; x < ((u64)1 << g.n); x += 256) {
-        const double a = fabs(C[x]);
-        m = fmax(m, a <= 1.7976931348623157e308 ? a : __builtin_huge_val());
+    for (u64 x = threadIdx.x; x < N / 2; x += 256) {
+        const double a = C[x], b = C[N - 1 - x], h = fmax(fabs(a), fabs(b));
+        diff |= !(a == b);
+        m = fmax(m, fabs(a) <= 1.7976931348623157e308 && fabs(b) <= 1.7976931348623157e308 ? h : __builtin_huge_val());
     }
+    if (diff) differ = 1;
     red[threadIdx.x] = m;
     __syncthreads();
     for (int h = 128; h; h >>= 1) {
         if ((int)threadIdx.x < h) red[threadIdx.x] = fmax(red[threadIdx.x], red[threadIdx.x + h]);
         __syncthreads();
     }
-    if (threadIdx.x == 0) cmax[blockIdx.x] = red[0];
+    if (threadIdx.x == 0) {
+        info[2 * blockIdx.x] = red[0];
+        info[2 * blockIdx.x + 1] = differ ? 0.0 : 1.0;
+    }
 }
 
 template <int LT, int THREADS>
@@ -728,10 +772,11 @@ extern "C" int ork_qaoa_launch(void *stream, int lt, int threads, int grid, cons
     return (int)hipErrorInvalidValue;
 }
 
-// recs: `count` QaoaRec on the device, sorted by qubits, then by layers, both descending; n and p: their qubits and layers on
-// the host; the states of more than 12 qubits have their tiles in `states`, one partial sum per tile in `part`
-extern "C" int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, const int *p, int count, const double *angles,
-                               const double *diag, void *states, double *part, double *out) {
+// recs: `count` QaoaRec on the device, all of one form (sym), sorted by index bits, then by layers, both descending; n and p:
+// their index bits and layers on the host; the states of more than 12 bits have their tiles in `states`, one partial sum per
+// tile in `part`
+extern "C" int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const int *n, const int *p, int count,
+                               const double *angles, const double *diag, void *states, double *part, double *out) {
     hipStream_t st = (hipStream_t)stream;
     const QaoaRec *r = (const QaoaRec *)recs;
     int large = 0, pmax = 0;
@@ -741,7 +786,8 @@ extern "C" int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, con
         ++large;
     }
     if (count > large) {
-        qaoa_one_tile<<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
+        if (sym) qaoa_one_tile<1><<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
+        else qaoa_one_tile<0><<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
         ORK_LAUNCH_CHECK();
     }
     for (int k = 0; k <= pmax && large; ++k) {
@@ -766,7 +812,8 @@ extern "C" int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, con
             i = j;
         }
         A.first[A.nclass] = blocks;
-        qaoa_sweep<<<blocks, RT_THREADS, 0, st>>>(A);
+        if (sym) qaoa_sweep<1><<<blocks, RT_THREADS, 0, st>>>(A);
+        else qaoa_sweep<0><<<blocks, RT_THREADS, 0, st>>>(A);
         ORK_LAUNCH_CHECK();
     }
     if (large) {
@@ -776,8 +823,8 @@ extern "C" int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, con
     return 0;
 }
 
-extern "C" int ork_qaoa_diag_max(void *stream, int ngraphs, const void *graphs, const double *diag, double *cmax) {
-    diag_max_kernel<<<ngraphs, 256, 0, (hipStream_t)stream>>>((const QaoaGraph *)graphs, diag, cmax);
+extern "C" int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs, const double *diag, double *info) {
+    diag_info_kernel<<<ngraphs, 256, 0, (hipStream_t)stream>>>((const QaoaGraph *)graphs, diag, info);
     ORK_LAUNCH_CHECK();
     return 0;
 }
@@ -785,7 +832,7 @@ extern "C" int ork_qaoa_diag_max(void *stream, int ngraphs, const void *graphs, 
 extern "C" int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu) {
     hipError_t e = hipErrorInvalidValue;
     if (lt == RT_BITS && threads == RT_THREADS)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_sweep, RT_THREADS, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_sweep<0>, RT_THREADS, 0);
 #define ORK_QOCC(L, TH) \
     if (lt == L && threads == TH) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_persistent<L, TH>, TH, 0);
     ORK_QOCC(10, 256) ORK_QOCC(10, 512) ORK_QOCC(10, 1024)

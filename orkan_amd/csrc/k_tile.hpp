@@ -11,6 +11,7 @@
 #include "k_common.hpp"
 
 constexpr int RT_BITS = 12, RT_THREADS = 256;
+constexpr unsigned RT_SIZE = 1u << RT_BITS;
 constexpr int RT_SLOTS = 4096 + 256;   // doubles of LDS that change_layout needs
 
 // the thread's 16 amplitudes: two arrays, so that either half can change layout by itself
@@ -45,5 +46,45 @@ __device__ __forceinline__ void change_layout(Amps &v, double *lds) {
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < 16; ++u) v.im[u] = r[u * rs];
+    __syncthreads();
+}
+
+// a change of layout and, on its way, I - i u X on the qubits whose X flips the tile bits of `mask`: each thread reads its
+// new elements and those at the flipped places
+template <int FROM, int TO>
+__device__ __forceinline__ void change_layout_flip(Amps &v, double *lds, unsigned mask, double u) {
+    constexpr int ws = lay_slot_step(FROM), rs = lay_slot_step(TO);
+    constexpr unsigned RB = 15u * lay_step(TO);   // tile bits of the register index
+    __builtin_amdgcn_sched_barrier(0);
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid) : : "memory");
+    const unsigned far = (unsigned)lay_base<TO>(tid) ^ (mask & (RT_SIZE - 1) & ~RB), fu = (mask & RB) / lay_step(TO);
+    double *w = lds + lay_slot<FROM>(tid);
+    const double *r = lds + lay_slot<TO>(tid);
+    // the flipped places' addresses are formed at each use: kept they spill
+    const auto flipped = [&](int k) {
+        unsigned x = far + (far >> 4);
+        asm volatile("" : "+v"(x));
+        return lds[x + ((unsigned)k ^ fu) * rs];
+    };
+    double pre[16];
+#pragma unroll
+    for (int k = 0; k < 16; ++k) w[k * ws] = v.re[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        v.re[k] = r[k * rs];
+        pre[k] = flipped(k);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) w[k * ws] = v.im[k];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < 16; ++k) {
+        if (k % 4 == 0) __builtin_amdgcn_sched_barrier(0);
+        v.re[k] = fma(u, flipped(k), v.re[k]);
+        v.im[k] = fma(-u, pre[k], r[k * rs]);
+    }
     __syncthreads();
 }

@@ -19,14 +19,14 @@ int ork_qaoa_launch(void *stream, int lt, int threads, int grid, const void *eva
                     const int *nevals, const void *graphs, const double *angles, const double *diag, void *states,
                     uint64_t slot_elems, double *out, unsigned *counter);
 int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu);
-int ork_qaoa_sweeps(void *stream, const void *recs, const int *n, const int *p, int count, const double *angles,
+int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const int *n, const int *p, int count, const double *angles,
                     const double *diag, void *states, double *part, double *out);
-int ork_qaoa_diag_max(void *stream, int ngraphs, const void *graphs, const double *diag, double *cmax);
+int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs, const double *diag, double *info);
 int ork_maxcut_diag(void *stream, double *out, int n, int ne, const int *ei, const int *ej, const double *w);
 
 typedef struct { int graph, p, angle_off, pad; } q_eval_t;
 typedef struct { uint64_t diag_off, state_off; int n, pad; } q_graph_t;
-typedef struct { uint64_t diag_off, tile; int angle_off, p, n, out; } q_rec_t;
+typedef struct { uint64_t diag_off, tile; int angle_off, p, n, m, out, pad; } q_rec_t;
 
 struct orkan_qaoa {
     int ngraphs, max_evals, max_p, nmax;
@@ -45,11 +45,12 @@ struct orkan_qaoa {
      * threads' gates and reductions use, and replayed on the library stream */
     hipStream_t capture_stream;
     int nevals_h;          /* host source of the nevals_d upload */
-    double *cmax_h;        /* per graph: largest |C| */
-    /* the register kernels' list: records sorted by qubits, then layers, both descending */
+    double *info_h;        /* per graph: largest |C|; 1 if C(x) = C(~x) for every x, else 0 */
+    /* the register kernels' list: records sorted by form, then index bits, then layers, all descending; n_h: index bits */
     q_rec_t *recs_h;
     void *recs_d;
     int *n_h, *p_h, *start_h, nstaged;
+    unsigned char *sym_h;
     int states_short;      /* the device had no memory for all the scratch asked for */
     size_t room;           /* tiles per round of launches, as the staged records number them */
     int wide;              /* the staged list holds a phase too large for the register kernel's sincos */
@@ -184,12 +185,13 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     q->evals_h = calloc((size_t)max_evals, sizeof(q_eval_t));
     q->order_h = calloc((size_t)max_evals, sizeof(int));
     q->angles_h = calloc((size_t)max_evals * max_p * 3, sizeof(double));
-    q->cmax_h = calloc((size_t)ngraphs, sizeof(double));
+    q->info_h = calloc((size_t)ngraphs * 2, sizeof(double));
+    q->sym_h = calloc((size_t)max_evals, 1);
     q->recs_h = calloc((size_t)max_evals, sizeof(q_rec_t));
     q->n_h = calloc((size_t)max_evals, sizeof(int));
     q->p_h = calloc((size_t)max_evals, sizeof(int));
-    q->start_h = calloc((size_t)27 * (max_p + 1) + 1, sizeof(int));
-    if (!q->graphs_h || !q->evals_h || !q->order_h || !q->angles_h || !q->cmax_h || !q->recs_h || !q->n_h || !q->p_h ||
+    q->start_h = calloc((size_t)2 * 27 * (max_p + 1) + 1, sizeof(int));
+    if (!q->graphs_h || !q->evals_h || !q->order_h || !q->angles_h || !q->info_h || !q->sym_h || !q->recs_h || !q->n_h || !q->p_h ||
         !q->start_h)
         goto fail;
     if (hipStreamCreateWithFlags(&q->capture_stream, hipStreamNonBlocking) != hipSuccess) {
@@ -221,15 +223,15 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     if (hipMalloc((void **)&q->out_d, (size_t)max_evals * sizeof(double)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->counter_d, sizeof(unsigned)) != hipSuccess) goto fail;
     {
-        double *cmax = ork_mem_get((size_t)ngraphs * sizeof(double));
-        const int bad = !cmax || ork_qaoa_diag_max(st, ngraphs, q->graphs_d, q->diag_d, cmax) ||
-                        hipMemcpyAsync(q->cmax_h, cmax, (size_t)ngraphs * sizeof(double), hipMemcpyDeviceToHost, st) !=
+        double *info = ork_mem_get((size_t)ngraphs * 2 * sizeof(double));
+        const int bad = !info || ork_qaoa_diag_info(st, ngraphs, q->graphs_d, q->diag_d, info) ||
+                        hipMemcpyAsync(q->info_h, info, (size_t)ngraphs * 2 * sizeof(double), hipMemcpyDeviceToHost, st) !=
                             hipSuccess;
         if (hipStreamSynchronize(st) != hipSuccess || bad) {
-            ork_mem_put(cmax);
+            ork_mem_put(info);
             goto fail;
         }
-        ork_mem_put(cmax);
+        ork_mem_put(info);
     }
     {
         /* default: 4096 amplitudes in the registers of 256 threads; 8192 in LDS when the largest state needs it */
@@ -258,7 +260,8 @@ void orkan_qaoa_destroy(orkan_qaoa_t *q) {
     free(q->evals_h);
     free(q->order_h);
     free(q->angles_h);
-    free(q->cmax_h);
+    free(q->info_h);
+    free(q->sym_h);
     free(q->recs_h);
     free(q->n_h);
     free(q->p_h);
@@ -298,32 +301,40 @@ static int by_cost_desc(const void *a, const void *b) {
     return *(const int *)a - *(const int *)b;
 }
 
-/* the register kernels' records: a counting sort by qubits, then layers, both descending */
+/* half of the state: a cost with C(x) = C(~x) whose state is larger than a tile.  A tile costs the same whatever part of it
+ * a state fills, and the half's X on the qubit left out takes an exchange more. */
+static int is_sym(const orkan_qaoa_t *q, int graph) {
+    return q->info_h[2 * graph + 1] != 0.0 && q->graphs_h[graph].n > REG_LT;
+}
+
+/* the register kernels' records: a counting sort by form (half states first), index bits and layers, all descending */
+static int rec_key(const orkan_qaoa_t *q, const q_eval_t *ev) {
+    const int sym = is_sym(q, ev->graph);
+    return ((1 - sym) * 27 + 26 - (q->graphs_h[ev->graph].n - sym)) * (q->max_p + 1) + (q->max_p - ev->p);
+}
+
 static void sort_recs(orkan_qaoa_t *q, int nevals) {
-    const int stride = q->max_p + 1, nkeys = 27 * stride;
+    const int nkeys = 2 * 27 * (q->max_p + 1);
     memset(q->start_h, 0, ((size_t)nkeys + 1) * sizeof(int));
-    for (int e = 0; e < nevals; ++e) {
-        const q_eval_t *ev = &q->evals_h[e];
-        const int key = (26 - q->graphs_h[ev->graph].n) * stride + (q->max_p - ev->p);
-        ++q->start_h[key + 1];
-    }
+    for (int e = 0; e < nevals; ++e) ++q->start_h[rec_key(q, &q->evals_h[e]) + 1];
     for (int k = 0; k < nkeys; ++k) q->start_h[k + 1] += q->start_h[k];
     for (int e = 0; e < nevals; ++e) {
         const q_eval_t *ev = &q->evals_h[e];
-        const int n = q->graphs_h[ev->graph].n;
-        const int at = q->start_h[(26 - n) * stride + (q->max_p - ev->p)]++;
-        const q_rec_t r = {q->graphs_h[ev->graph].diag_off, 0, ev->angle_off, ev->p, n, e};
+        const int n = q->graphs_h[ev->graph].n, sym = is_sym(q, ev->graph);
+        const int at = q->start_h[rec_key(q, ev)]++;
+        const q_rec_t r = {q->graphs_h[ev->graph].diag_off, 0, ev->angle_off, ev->p, n, n - sym, e, 0};
         q->recs_h[at] = r;
-        q->n_h[at] = n;
+        q->n_h[at] = n - sym;
         q->p_h[at] = ev->p;
+        q->sym_h[at] = (unsigned char)sym;
     }
 }
 
-/* the number of records from `at` on whose states fit the scratch together */
+/* the number of records from `at` on that are of one form and whose states fit the scratch together */
 static int next_round(const orkan_qaoa_t *q, int at) {
     size_t used = 0;
     int i = at;
-    for (; i < q->nstaged; ++i) {
+    for (; i < q->nstaged && q->sym_h[i] == q->sym_h[at]; ++i) {
         const size_t tiles = q->n_h[i] > REG_LT ? (size_t)1 << (q->n_h[i] - REG_LT) : 0;
         if (used + tiles > q->room || used + tiles > ((size_t)1 << 31) - 1) break;
         used += tiles;
@@ -347,7 +358,7 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
             const double theta = 2.0 * beta[(size_t)e * q->max_p + l];
             const double gl = gamma[(size_t)e * q->max_p + l];
             q->angles_h[(size_t)e * q->max_p * 3 + 3 * l] = gl;
-            if (!(fabs(gl) * q->cmax_h[graph[e]] < REG_PHASE_MAX)) q->wide = 1;
+            if (!(fabs(gl) * q->info_h[2 * graph[e]] < REG_PHASE_MAX)) q->wide = 1;
             q->angles_h[(size_t)e * q->max_p * 3 + 3 * l + 1] = cos(theta / 2.0);
             q->angles_h[(size_t)e * q->max_p * 3 + 3 * l + 2] = sin(theta / 2.0);
         }
@@ -400,7 +411,7 @@ int orkan_qaoa_launch_staged(orkan_qaoa_t *q) {
         for (int at = 0; at < q->nstaged;) {
             const int m = next_round(q, at);
             if (m == 0) return (int)hipErrorInvalidValue;
-            const int e = ork_qaoa_sweeps(st, (const q_rec_t *)q->recs_d + at, q->n_h + at, q->p_h + at, m, q->angles_d,
+            const int e = ork_qaoa_sweeps(st, q->sym_h[at], (const q_rec_t *)q->recs_d + at, q->n_h + at, q->p_h + at, m, q->angles_d,
                                           q->diag_d, q->states_d, (double *)((char *)q->states_d + q->room * TILE_BYTES),
                                           q->out_d);
             if (e) return e;

@@ -147,6 +147,38 @@ def test_register_tiles(lo, hi, flips):
     b.close()
 
 
+@pytest.mark.parametrize("lo,hi", [(1, 8), (9, 13), (14, 17), (18, 20), (21, 24)])
+def test_flip_symmetric_costs(lo, hi):
+    """Costs with C(x) = C(~x) run on half of the state: every qubit count of the range (one tile up to 13 qubits, every
+    place of the bit that the gathered tiles share with the contiguous ones), mixers of both forms, in one list with a
+    cost of each size whose last bit differs in one entry and which must take the general kernels."""
+    lib = orkan_amd.load(5)
+    orc = engines.oracle(5)
+    rng = np.random.default_rng(70 + lo)
+    ns, ps, diags = [], [], []
+    for n in range(lo, hi + 1):
+        for p in ((1, 2, 3, 4) if n < 18 else (2, 3) if n < 21 else (2,)):
+            d = rng.uniform(-3, 5, 1 << n)
+            ns.append(n)
+            ps.append(p)
+            diags.append(d + d[::-1])
+        if n < 21:
+            d = diags[-1].copy()
+            d[0] = np.nextafter(d[0], 9.0)
+            ns.append(n)
+            ps.append(2)
+            diags.append(d)
+    gam = [rng.uniform(0, np.pi, p) for p in ps]
+    bet = [rng.uniform(0, np.pi, p) for p in ps]
+    b = batch.QaoaBatch(lib, ns, diags, max_evals=len(ns), max_p=4)
+    got = b.eval(list(range(len(ns))), ps, gam, bet)
+    assert np.array_equal(got, b.eval(list(range(len(ns))), ps, gam, bet))
+    for k, n in enumerate(ns):
+        want = oracle_eval(orc, n, diags[k], ps[k], gam[k], bet[k])
+        assert abs(got[k] - want) <= 1e-12, (n, ps[k], got[k], want)
+    b.close()
+
+
 @pytest.mark.parametrize("big", [3e15, 1e300, np.inf, np.nan])
 def test_phases_beyond_the_register_kernel(big):
     """A phase of 2^50 or more, or one that is not finite, takes the whole list through the LDS kernel: the bits of that
