@@ -994,15 +994,20 @@ __global__ __launch_bounds__(DM_THREADS) void dm_sop_packed_kernel(S *__restrict
     auto mirror = [&](u64 a, u64 b) {
         return a > b && (a >> q) == (b >> q) && !quad_still<SKIP>(op, ins0(a, q), ins0(b, q));
     };
-    // the block's mirror entries, loaded together with the quads below and staged through LDS
-    // once every load is in flight
-    cd mv[QPT];
-    if (has_mirror) {
+    // the block's mirror entries, loaded together with the quads below, converted and staged through LDS
+    // once every load is in flight (complex64 converted at the load waited for each entry in turn)
+    S mraw[QPT];
+    if (sizeof(S) == 8 || has_mirror) {
 #pragma unroll
         for (int h = 0; h < QPT; ++h) {
             const int t = tid + DM_THREADS * h, x = t / YW, y = y0 + t % YW;   // lanes walk y: rows c1 of column r0(x)
             const u64 a = A * 32 + x, b = Bk * 32 + y;
-            if (mirror(a, b)) mv[h] = ldx<NT == 1>(rho + col_base(D, ins0(a, q)) + ((ins0(b, q) | m) - ins0(a, q)));
+            const bool in = has_mirror && mirror(a, b);
+            // complex64: without a condition, an entry not there reads rho[0]. Inside the condition each entry's
+            // conversion waited for its load: three round trips to memory, now one (cx on 13 qubits, a target next to the
+            // last: 81 -> 75.5 us; h on 9 qubits 5.3 -> 4.7)
+            const S *p = in ? rho + col_base(D, ins0(a, q)) + ((ins0(b, q) | m) - ins0(a, q)) : rho;
+            if (sizeof(S) == 8 || in) mraw[h] = ldr<NT == 1>(p);
         }
     }
     // all quads of a thread in flight: t = tid + 256 h.  Complex64 values are loaded raw for every quad
@@ -1051,6 +1056,8 @@ __global__ __launch_bounds__(DM_THREADS) void dm_sop_packed_kernel(S *__restrict
             for (int h = 0; h < QPT; ++h)
 #pragma unroll
                 for (int j = 0; j < 4; ++j) hold(raw[h][j]);
+#pragma unroll
+            for (int h = 0; h < QPT; ++h) hold(mraw[h]);
         }
 #pragma unroll
         for (int h = 0; h < QPT; ++h)
@@ -1061,7 +1068,7 @@ __global__ __launch_bounds__(DM_THREADS) void dm_sop_packed_kernel(S *__restrict
             for (int h = 0; h < QPT; ++h) {
                 const int t = tid + DM_THREADS * h, x = t / YW, y = y0 + t % YW;
                 const u64 a = A * 32 + x, b = Bk * 32 + y;
-                if (mirror(a, b)) ms[x * LDS_STRIDE + y] = mv[h];
+                if (mirror(a, b)) ms[x * LDS_STRIDE + y] = to_cd(mraw[h]);
             }
             __syncthreads();
         }
@@ -1710,7 +1717,8 @@ __global__ __launch_bounds__(DM_THREADS) void dm_phase_kernel(S *__restrict__ rh
         // e^{-i(d_r - d_c)t} = (cr - i sr)(cc + i sc)   (src/circ/circ_packed.c:54-60)
 #pragma unroll
         for (int j = 0; j < E; ++j)
-            if (chg[j]) f[j] = cmk(pr[j].x * pc[j].x + pr[j].y * pc[j].y, -pr[j].y * pc[j].x + pr[j].x * pc[j].y);
+            if (chg[j])   // explicit fma: the same bits whatever the number of entries per thread
+                f[j] = cmk(fma(pr[j].x, pc[j].x, pr[j].y * pc[j].y), fma(-pr[j].y, pc[j].x, pr[j].x * pc[j].y));
     }
     cd v[E];
 #pragma unroll
@@ -1721,12 +1729,7 @@ __global__ __launch_bounds__(DM_THREADS) void dm_phase_kernel(S *__restrict__ rh
 #pragma unroll
     for (int j = 0; j < E; ++j) {
         if (!act[j]) continue;
-        cd o = v[j];
-        if (chg[j]) {
-            if constexpr (MODE == 0) o = cmul(f[j], v[j]);
-            else o = cmk(f[j].x * v[j].x - f[j].y * v[j].y, f[j].x * v[j].y + f[j].y * v[j].x);
-        }
-        stx<NT>(rho + x0 + (u64)j * DM_THREADS, o);
+        stx<NT>(rho + x0 + (u64)j * DM_THREADS, chg[j] ? cmul(f[j], v[j]) : v[j]);
     }
 }
 
@@ -2168,6 +2171,11 @@ template <typename S, int LAYOUT, int MODE, int NT, int WL>
 void launch_phase_t(hipStream_t st, unsigned grid, int lds, void *rho, const PhasePlan &pp, const PhaseArgs &a,
                     const double2 *cs, int em) {
     constexpr int E = sizeof(S) == 8 ? 8 : 4;
+    if constexpr (!NT && !WL)
+        if (em == 0) {
+            dm_phase_kernel<S, LAYOUT, MODE, 0, 0, 1><<<grid, DM_THREADS, lds, st>>>((S *)rho, pp, a, cs);
+            return;
+        }
     if (em == 4) dm_phase_kernel<S, LAYOUT, MODE, NT, WL, 4 * E><<<grid, DM_THREADS, lds, st>>>((S *)rho, pp, a, cs);
     else if (em == 2) dm_phase_kernel<S, LAYOUT, MODE, NT, WL, 2 * E><<<grid, DM_THREADS, lds, st>>>((S *)rho, pp, a, cs);
     else dm_phase_kernel<S, LAYOUT, MODE, NT, WL, E><<<grid, DM_THREADS, lds, st>>>((S *)rho, pp, a, cs);
@@ -2179,6 +2187,13 @@ void launch_phase_l(hipStream_t st, int layout, unsigned grid, int lds, void *rh
     if (layout == ORK_PACKED) launch_phase_t<S, ORK_PACKED, MODE, NT, WL>(st, grid, lds, rho, pp, a, cs, em);
     else launch_phase_t<S, ORK_TILED, MODE, NT, WL>(st, grid, lds, rho, pp, a, cs, em);
 }
+
+// Below this many workgroups (four per CU) a thread takes one entry instead of 64 B or more of them: the launch is one
+// round of workgroups, whose time is one thread's chain of index decodes (a square root each) and of loads. Complex64,
+// packed: cz on 9 qubits 8.5 us with 8 entries per thread (64 workgroups), 3.4 with one; on 10 qubits 8.6 and 5.8; exp_diag
+// 10.4 and 5.8; complex128 with 4 entries 5.8 and 3.5; from 1024 workgroups on (11 qubits) the entries in flight count.
+// Whole lines and streaming accesses are for states that leave the caches.
+constexpr u64 kPhaseFill = 1024;
 
 template <int MODE>
 int launch_phase(hipStream_t st, int prec, int layout, int L, int n, void *rho, const PhaseArgs &a,
@@ -2194,12 +2209,18 @@ int launch_phase(hipStream_t st, int prec, int layout, int L, int n, void *rho, 
     }
     Shape sh = g_phase_shape[layout == ORK_TILED ? 1 : 0];
     const u64 elem = prec == ORK_F32 ? 8 : 16;
-    const int em = 1 << sh.lp;
-    const u64 per = (prec == ORK_F32 ? 8 : 4) * (u64)em * DM_THREADS;
+    int em = 1 << sh.lp;
+    u64 per = (prec == ORK_F32 ? 8 : 4) * (u64)em * DM_THREADS;
     pp.nchunks = (pp.len + per - 1) / per;
     if (pp.nchunks > 0x7fffffffu) return (int)hipErrorInvalidValue;
     pp.xcd = sh.xcd;
     if (pp.len * elem < ork_nt_min_bytes()) sh.nt = 0;
+    if (!sh.nt && pp.nchunks < kPhaseFill) {
+        em = 0;
+        per = DM_THREADS;
+        pp.nchunks = (pp.len + per - 1) / per;
+        sh.wl = 0;
+    }
     int wl = 0;
     if (MODE == 0) {
         // tiled: the lowest gate qubit decides whether changed entries fill 128 B lines (tile rows are
