@@ -328,9 +328,9 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 // visits the layouts in the order that needs fewest changes: 1 (load, finish bits 4-7), 0 (finish bits 0-3, only where
 // ls < 4), 2 (finish bits 8-11, phase, rx), 0 (rx), 1 (rx, store); with ls >= 8 it starts in layout 2.
 // A launch is one sweep k over all tiles of all states that have it, so a single large state fills the chip as well as a
-// thousand do: with a workgroup per evaluation one state of 18 qubits took 2180 us, now 99; 300 of 4 to 11 qubits
-// (qaoa_one_tile) 231 and 213; with SYM = 0, 64 of 16 qubits 632 and 209, six of 21 to 24 qubits 185 and 5.2 ms, 4096
-// evaluations of 10 to 20 qubits and 1 to 8 layers 38.8 and 29.0 ms a call.  Memory bounds it: 140 GB of amplitudes and cost
+// thousand do: with a workgroup per evaluation one state of 18 qubits took 2180 us, now 77; 300 of 4 to 11 qubits
+// (qaoa_one_tile) 231 and 180; with SYM = 0, 64 of 16 qubits 632 and 187, six of 21 to 24 qubits 185 and 5.2 ms, 4096
+// evaluations of 10 to 20 qubits and 1 to 8 layers 38.8 and 28.2 ms a call.  Memory bounds it: 140 GB of amplitudes and cost
 // diagonal in runs of 256 and 128 B take 26 ms with everything else left out, the rest alone 14.  Nontemporal accesses gain
 // nothing.
 //
@@ -342,8 +342,8 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 // one its tile's bits without vb and qubit v; the two wide flips ride on a change of layout (change_layout_flip).  The state
 // of x_(n-1) = 0 has C(y) at y, with bits 12.. complemented where y_vb = 1: in runs of 2^vb, 128 B up to 20 qubits.  The
 // product of a layer's X over all qubits is 1 here, so RxFlip.flip is not needed.  Half the bytes and the work:
-// 4096 evaluations of 10 to 20 qubits 29.0 -> 16.8 ms a call (3 of them on the host), 64 of 16 qubits 212 -> 163 us, 700 of 12
-// to 17 1.57 -> 1.04 ms, six of 21 to 24 5.5 -> 2.0 ms, one of 18 99 us both ways.
+// 4096 evaluations of 10 to 20 qubits 28.2 -> 16.0 ms a call (2 of them on the host), 64 of 16 qubits 187 -> 140 us, 700 of 12
+// to 17 1.46 -> 0.97 ms, six of 21 to 24 5.4 -> 1.9 ms, one of 18 77 us both ways.
 
 // a value that is the same in every lane, as a scalar: what is loaded by a computed index counts as per-lane otherwise, and
 // with it every branch and address that depends on it
@@ -693,6 +693,22 @@ __global__ void reset_counter(unsigned *c) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0u;
 }
 
+// A call's list from pinned host memory: rows of gamma, then of beta, as the per-layer (gamma, cos beta, sin beta) that the
+// kernels read, and the records.  One launch and no wait in place of two copies from pageable memory (25 to 30 us of every
+// call, one evaluation of 18 qubits 100 -> 77 us); the cosines took the host 0.7 of 16.8 ms for 4096 evaluations.
+__global__ __launch_bounds__(256) void stage_kernel(const double *__restrict__ gb, u64 rows, double *__restrict__ angles,
+                                                    const u64 *__restrict__ recs, u64 words, u64 *__restrict__ dst) {
+    const u64 i = (u64)blockIdx.x * 256 + threadIdx.x;
+    if (i < words) dst[i] = recs[i];
+    if (i >= rows) return;
+    const double theta = 2.0 * gb[rows + i];   // rx(q, 2 beta): the reference evaluates cos(theta / 2) and sin(theta / 2)
+    double s, c;
+    sincos(theta / 2.0, &s, &c);
+    angles[3 * i] = gb[i];
+    angles[3 * i + 1] = c;
+    angles[3 * i + 2] = s;
+}
+
 // C(x) = sum_(i,j) w_ij [x_i != x_j] for one graph
 __global__ __launch_bounds__(256) void maxcut_diag_kernel(double *__restrict__ out, u64 N, int ne,
                                                          const int *__restrict__ ei, const int *__restrict__ ej,
@@ -820,6 +836,16 @@ extern "C" int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const in
         qaoa_finish<<<large, 256, 0, st>>>(r, angles, part, out);
         ORK_LAUNCH_CHECK();
     }
+    return 0;
+}
+
+extern "C" int ork_qaoa_stage(void *stream, const double *gb, uint64_t rows, double *angles, const void *recs, int nrecs,
+                              void *recs_dst) {
+    static_assert(sizeof(QaoaRec) % sizeof(u64) == 0, "copied in words");
+    const u64 words = (u64)nrecs * (sizeof(QaoaRec) / sizeof(u64)), n = rows > words ? rows : words;
+    stage_kernel<<<(unsigned)((n + 255) / 256), 256, 0, (hipStream_t)stream>>>(gb, rows, angles, (const u64 *)recs, words,
+                                                                              (u64 *)recs_dst);
+    ORK_LAUNCH_CHECK();
     return 0;
 }
 

@@ -21,6 +21,7 @@ int ork_qaoa_launch(void *stream, int lt, int threads, int grid, const void *eva
 int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu);
 int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const int *n, const int *p, int count, const double *angles,
                     const double *diag, void *states, double *part, double *out);
+int ork_qaoa_stage(void *stream, const double *gb, uint64_t rows, double *angles, const void *recs, int nrecs, void *recs_dst);
 int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs, const double *diag, double *info);
 int ork_maxcut_diag(void *stream, double *out, int n, int ne, const int *ei, const int *ej, const double *w);
 
@@ -35,7 +36,7 @@ struct orkan_qaoa {
     double *diag_d;
     void *evals_d;
     int *order_d, *nevals_d;
-    double *angles_d, *out_d;
+    double *angles_d;
     unsigned *counter_d;
     void *states_d;
     size_t states_bytes;
@@ -47,7 +48,7 @@ struct orkan_qaoa {
     int nevals_h;          /* host source of the nevals_d upload */
     double *info_h;        /* per graph: largest |C|; 1 if C(x) = C(~x) for every x, else 0 */
     /* the register kernels' list: records sorted by form, then index bits, then layers, all descending; n_h: index bits */
-    q_rec_t *recs_h;
+    q_rec_t *recs_h;       /* pinned */
     void *recs_d;
     int *n_h, *p_h, *start_h, nstaged;
     unsigned char *sym_h;
@@ -60,7 +61,7 @@ struct orkan_qaoa {
     /* host staging */
     q_eval_t *evals_h;
     int *order_h;
-    double *angles_h;
+    double *gb_h, *out_h;  /* pinned: rows of gamma, then of beta; the results */
 };
 
 static int cus(void) {
@@ -184,14 +185,12 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     q->graphs_h = calloc((size_t)ngraphs, sizeof(q_graph_t));
     q->evals_h = calloc((size_t)max_evals, sizeof(q_eval_t));
     q->order_h = calloc((size_t)max_evals, sizeof(int));
-    q->angles_h = calloc((size_t)max_evals * max_p * 3, sizeof(double));
     q->info_h = calloc((size_t)ngraphs * 2, sizeof(double));
     q->sym_h = calloc((size_t)max_evals, 1);
-    q->recs_h = calloc((size_t)max_evals, sizeof(q_rec_t));
     q->n_h = calloc((size_t)max_evals, sizeof(int));
     q->p_h = calloc((size_t)max_evals, sizeof(int));
     q->start_h = calloc((size_t)2 * 27 * (max_p + 1) + 1, sizeof(int));
-    if (!q->graphs_h || !q->evals_h || !q->order_h || !q->angles_h || !q->info_h || !q->sym_h || !q->recs_h || !q->n_h || !q->p_h ||
+    if (!q->graphs_h || !q->evals_h || !q->order_h || !q->info_h || !q->sym_h || !q->n_h || !q->p_h ||
         !q->start_h)
         goto fail;
     if (hipStreamCreateWithFlags(&q->capture_stream, hipStreamNonBlocking) != hipSuccess) {
@@ -220,7 +219,11 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     if (hipMalloc((void **)&q->order_d, (size_t)max_evals * sizeof(int)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->nevals_d, sizeof(int)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->angles_d, (size_t)max_evals * max_p * 3 * sizeof(double)) != hipSuccess) goto fail;
-    if (hipMalloc((void **)&q->out_d, (size_t)max_evals * sizeof(double)) != hipSuccess) goto fail;
+    if (hipHostMalloc((void **)&q->gb_h, (size_t)max_evals * max_p * 2 * sizeof(double), hipHostMallocDefault) !=
+            hipSuccess ||
+        hipHostMalloc((void **)&q->recs_h, (size_t)max_evals * sizeof(q_rec_t), hipHostMallocDefault) != hipSuccess ||
+        hipHostMalloc((void **)&q->out_h, (size_t)max_evals * sizeof(double), hipHostMallocDefault) != hipSuccess)
+        goto fail;
     if (hipMalloc((void **)&q->counter_d, sizeof(unsigned)) != hipSuccess) goto fail;
     {
         double *info = ork_mem_get((size_t)ngraphs * 2 * sizeof(double));
@@ -253,16 +256,17 @@ void orkan_qaoa_destroy(orkan_qaoa_t *q) {
     (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
     drop_graph(q);
     void *bufs[] = {q->graphs_d, q->diag_d, q->evals_d, q->order_d, q->nevals_d,
-                    q->angles_d, q->out_d, q->counter_d, q->states_d, q->recs_d};
+                    q->angles_d, q->counter_d, q->states_d, q->recs_d};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i)
         if (bufs[i]) (void)hipFree(bufs[i]);
+    void *pinned[] = {q->gb_h, q->recs_h, q->out_h};
+    for (size_t i = 0; i < sizeof(pinned) / sizeof(pinned[0]); ++i)
+        if (pinned[i]) (void)hipHostFree(pinned[i]);
     free(q->graphs_h);
     free(q->evals_h);
     free(q->order_h);
-    free(q->angles_h);
     free(q->info_h);
     free(q->sym_h);
-    free(q->recs_h);
     free(q->n_h);
     free(q->p_h);
     free(q->start_h);
@@ -276,7 +280,7 @@ static int capture(orkan_qaoa_t *q) {
     int e = (int)hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal);
     if (e) return e;
     int le = ork_qaoa_launch(st, q->lt, q->threads, q->grid, q->evals_d, q->order_d, q->nevals_d, q->graphs_d,
-                             q->angles_d, q->diag_d, q->states_d, ((uint64_t)1 << q->nmax), q->out_d, q->counter_d);
+                             q->angles_d, q->diag_d, q->states_d, ((uint64_t)1 << q->nmax), q->out_h, q->counter_d);
     e = (int)hipStreamEndCapture(st, &q->graph);
     if (le) return le;
     if (e) return e;
@@ -342,7 +346,7 @@ static int next_round(const orkan_qaoa_t *q, int at) {
     return i - at;
 }
 
-/* upload the evaluation list; angles: rows of max_p gammas and betas.  any_shape: for every kernel, not only the one the
+/* stage the evaluation list; angles: rows of max_p gammas and betas.  any_shape: for every kernel, not only the one the
  * configuration and the list's phases call for */
 static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma, const double *beta,
                  int any_shape) {
@@ -353,24 +357,18 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
         q->evals_h[e].graph = graph[e];
         q->evals_h[e].p = p[e];
         q->evals_h[e].angle_off = e * q->max_p * 3;
-        for (int l = 0; l < p[e]; ++l) {
-            /* rx(q, 2 beta): the reference evaluates cos(theta / 2) and sin(theta / 2) */
-            const double theta = 2.0 * beta[(size_t)e * q->max_p + l];
-            const double gl = gamma[(size_t)e * q->max_p + l];
-            q->angles_h[(size_t)e * q->max_p * 3 + 3 * l] = gl;
-            if (!(fabs(gl) * q->info_h[2 * graph[e]] < REG_PHASE_MAX)) q->wide = 1;
-            q->angles_h[(size_t)e * q->max_p * 3 + 3 * l + 1] = cos(theta / 2.0);
-            q->angles_h[(size_t)e * q->max_p * 3 + 3 * l + 2] = sin(theta / 2.0);
-        }
+        const double *g = gamma + (size_t)e * q->max_p, *b = beta + (size_t)e * q->max_p;
+        memcpy(q->gb_h + (size_t)e * q->max_p, g, (size_t)p[e] * sizeof(double));
+        memcpy(q->gb_h + ((size_t)nevals + e) * q->max_p, b, (size_t)p[e] * sizeof(double));
+        for (int l = 0; l < p[e]; ++l)
+            if (!(fabs(g[l]) * q->info_h[2 * graph[e]] < REG_PHASE_MAX)) q->wide = 1;
         q->order_h[e] = e;
     }
     q->nstaged = nevals;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     int e = ensure_states(q);
     if (e) return e;
-    if (nevals > 0)
-        e |= (int)hipMemcpyAsync(q->angles_d, q->angles_h, (size_t)nevals * q->max_p * 3 * sizeof(double),
-                                 hipMemcpyHostToDevice, st);
+    int nrecs = 0;
     if (nevals > 0 && (any_shape || (is_reg(q) && !q->wide))) {
         sort_recs(q, nevals);
         /* every round numbers its tiles from 0 */
@@ -382,7 +380,11 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
                 if (q->n_h[i] > REG_LT) tile += (uint64_t)1 << (q->n_h[i] - REG_LT);
             }
         }
-        e |= (int)hipMemcpyAsync(q->recs_d, q->recs_h, (size_t)nevals * sizeof(q_rec_t), hipMemcpyHostToDevice, st);
+        nrecs = nevals;
+    }
+    if (nevals > 0) {
+        e = ork_qaoa_stage(st, q->gb_h, (uint64_t)nevals * q->max_p, q->angles_d, q->recs_h, nrecs, q->recs_d);
+        if (e) return e;
     }
     if (any_shape || !is_reg(q) || q->wide) {
         g_sort_q = q;
@@ -393,8 +395,8 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
         }
         q->nevals_h = nevals;
         e |= (int)hipMemcpyAsync(q->nevals_d, &q->nevals_h, sizeof(int), hipMemcpyHostToDevice, st);
+        e |= (int)hipStreamSynchronize(st);
     }
-    e |= (int)hipStreamSynchronize(st);
     return e;
 }
 
@@ -406,14 +408,14 @@ int orkan_qaoa_launch_staged(orkan_qaoa_t *q) {
             const size_t slots = q->nmax > REG_LT ? q->states_bytes / ((size_t)16 << q->nmax) : (size_t)cus();
             const int grid = slots < (size_t)cus() ? (int)slots : cus();
             return ork_qaoa_launch(st, REG_LT, WIDE_THREADS, grid, q->evals_d, q->order_d, q->nevals_d, q->graphs_d,
-                                   q->angles_d, q->diag_d, q->states_d, ((uint64_t)1 << q->nmax), q->out_d, q->counter_d);
+                                   q->angles_d, q->diag_d, q->states_d, ((uint64_t)1 << q->nmax), q->out_h, q->counter_d);
         }
         for (int at = 0; at < q->nstaged;) {
             const int m = next_round(q, at);
             if (m == 0) return (int)hipErrorInvalidValue;
             const int e = ork_qaoa_sweeps(st, q->sym_h[at], (const q_rec_t *)q->recs_d + at, q->n_h + at, q->p_h + at, m, q->angles_d,
                                           q->diag_d, q->states_d, (double *)((char *)q->states_d + q->room * TILE_BYTES),
-                                          q->out_d);
+                                          q->out_h);
             if (e) return e;
             at += m;
         }
@@ -433,9 +435,10 @@ int orkan_qaoa_eval(orkan_qaoa_t *q, int nevals, const int *graph, const int *p,
     int e = stage(q, nevals, graph, p, gamma, beta, 0);
     if (!e) e = orkan_qaoa_launch_staged(q);
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    if (!e && nevals > 0 && out)
-        e = (int)hipMemcpyAsync(out, q->out_d, (size_t)nevals * sizeof(double), hipMemcpyDeviceToHost, st);
-    if (!e) e = (int)hipStreamSynchronize(st);
+    /* also after an error: the next call writes the pinned list again */
+    const int es = (int)hipStreamSynchronize(st);
+    if (!e) e = es;
+    if (!e && nevals > 0 && out) memcpy(out, q->out_h, (size_t)nevals * sizeof(double));
     ork_unlock();
     return e;
 }
