@@ -410,6 +410,8 @@ int orkan_qaoa_launch_staged(orkan_qaoa_t *q) {
             return ork_qaoa_launch(st, REG_LT, WIDE_THREADS, grid, q->evals_d, q->order_d, q->nevals_d, q->graphs_d,
                                    q->angles_d, q->diag_d, q->states_d, ((uint64_t)1 << q->nmax), q->out_h, q->counter_d);
         }
+        /* a configuration set since then may have left less scratch than the records' tiles were numbered for */
+        if (q->room > tile_room(q)) return (int)hipErrorOutOfMemory;
         for (int at = 0; at < q->nstaged;) {
             const int m = next_round(q, at);
             if (m == 0) return (int)hipErrorInvalidValue;
