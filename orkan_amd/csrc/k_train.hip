@@ -151,19 +151,33 @@ __global__ __launch_bounds__(MT) void gemm_nt_mid_kernel(const bf16 *__restrict_
 }
 
 // ---- operand preparation ------------------------------------------------------------------------
-// x (fp32 [rows][K]) -> bf16 x16 [M][K] and its transpose x16t [K][ldt]; rows at and past `rows` are zero.  One 64 x 32
-// tile per workgroup through LDS.
-__global__ __launch_bounds__(256) void stage_input_kernel(const float *__restrict__ x, int rows, int K,
-                                                          bf16 *__restrict__ x16, bf16 *__restrict__ x16t, long ldt) {
+// Rows m_first .. of x (fp32 [rows][K]) -> bf16 x16 [M][K] and its transpose x16t [K][ldt]; rows at and past `rows` are
+// zero.  One 64 x 32 tile per workgroup through LDS.  x may be pinned host memory: a host batch is then read over PCIe
+// once, by this kernel, chunk after chunk behind the host's copies into that memory, and its targets (tgt_src, `rows` of
+// them, may be null) come along.  Bound by PCIe there: 16 B per lane,
+// every load of a thread in flight; 0.5 MB in 14.5 us, 36 GB/s, against 87 us for 2 MB through hipMemcpy.
+__global__ __launch_bounds__(256) void stage_input_kernel(const float *__restrict__ x, int m_first, int rows, int K,
+                                                          bf16 *__restrict__ x16, bf16 *__restrict__ x16t, long ldt,
+                                                          const float *__restrict__ tgt_src, float *__restrict__ tgt) {
     __shared__ bf16 tile[32][64 + 2];
-    const int m0 = blockIdx.x * 64, k0 = blockIdx.y * 32;
+    const int m0 = m_first + blockIdx.x * 64, k0 = blockIdx.y * 32;
+    if (tgt_src && blockIdx.y == 0 && threadIdx.x < 64 && m0 + (int)threadIdx.x < rows)
+        tgt[m0 + threadIdx.x] = tgt_src[m0 + threadIdx.x];
+    float4 f[2];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        const int e = threadIdx.x + u * 256, m = e >> 5, k = e & 31;
-        const long at = (long)(m0 + m) * K + k0 + k;
-        const bf16 v = (bf16)(m0 + m < rows ? x[at] : 0.0f);
-        x16[at] = v;
-        tile[k][m] = v;
+    for (int u = 0; u < 2; ++u) {
+        const int e = threadIdx.x + u * 256, m = m0 + (e >> 3);
+        f[u] = *(const float4 *)(x + (long)(m < rows ? m : rows - 1) * K + k0 + (e & 7) * 4);
+    }
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+        const int e = threadIdx.x + u * 256, m = e >> 3, k = (e & 7) * 4;
+        const bool in = m0 + m < rows;
+        const bf16x4 v = {(bf16)(in ? f[u].x : 0.0f), (bf16)(in ? f[u].y : 0.0f), (bf16)(in ? f[u].z : 0.0f),
+                          (bf16)(in ? f[u].w : 0.0f)};
+        *(bf16x4 *)(x16 + (long)(m0 + m) * K + k0 + k) = v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tile[k + j][m] = v[j];
     }
     __syncthreads();
     if (x16t)
@@ -172,6 +186,31 @@ __global__ __launch_bounds__(256) void stage_input_kernel(const float *__restric
             const int e = threadIdx.x + u * 256, k = e >> 6, m = e & 63;
             x16t[(long)(k0 + k) * ldt + m0 + m] = tile[k][m];
         }
+}
+
+// Arrays one after the other into pinned host memory, 4096 floats per workgroup: one launch and one wait for all the
+// parameters of a network, where a copy into pageable memory waits for each array.
+constexpr int PACK_MAX = 2 * 4 + 1;
+struct PackArgs {
+    const float *src[PACK_MAX];
+    int first[PACK_MAX + 1];   // in float4
+    int count;
+};
+__global__ __launch_bounds__(256) void pack_kernel(PackArgs a, float4 *__restrict__ dst) {
+    float4 f[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int x = min((int)blockIdx.x * 1024 + u * 256 + (int)threadIdx.x, a.first[a.count] - 1);
+        int i = 0;
+#pragma unroll
+        for (int j = 1; j < PACK_MAX; ++j) i += j < a.count && x >= a.first[j];
+        f[u] = ((const float4 *)a.src[i])[x - a.first[i]];
+    }
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int x = (int)blockIdx.x * 1024 + u * 256 + (int)threadIdx.x;
+        if (x < a.first[a.count]) dst[x] = f[u];
+    }
 }
 
 // dPre of the last hidden layer, dpre[m][k] = dy[m] w[k] gelu'(pre[m][k]) (bf16), and its transpose
@@ -357,7 +396,8 @@ __global__ __launch_bounds__(256) void colsums_finish_kernel(ColsumArgs c) {
         for (int off = 32; off > 0; off >>= 1) acc += __shfl_down(acc, off, 64);
         if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = acc;
         __syncthreads();
-        if (threadIdx.x == 0) c.vout[w] = red[0] + red[1] + red[2] + red[3];
+        if (threadIdx.x == 0)   // pinned host memory
+            __hip_atomic_store(c.vout + w, red[0] + red[1] + red[2] + red[3], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         __syncthreads();
     }
 }
@@ -438,11 +478,33 @@ extern "C" int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, c
     return 0;
 }
 
-// x fp32 [rows][K] -> x16 [M][K] and x16t [K][ldt] (null: not needed); M a multiple of 64, K of 32
-extern "C" int ork_mlp_stage_input(void *stream, const float *x, int rows, int M, int K, void *x16, void *x16t,
-                                   long ldt) {
-    if (M % 64 || K % 32 || M <= 0 || K <= 0) return (int)hipErrorInvalidValue;
-    stage_input_kernel<<<dim3(M / 64, K / 32), 256, 0, (hipStream_t)stream>>>(x, rows, K, (bf16 *)x16, (bf16 *)x16t, ldt);
+// rows m0 .. m1 - 1 of x fp32 [rows][K] -> x16 [M][K] and x16t [K][ldt] (null: not needed); m0 and m1 multiples of 64, K
+// of 32; x on a 16 B boundary, device or pinned host memory.  tgt_src: `rows` targets to copy to tgt, or null.
+extern "C" int ork_mlp_stage_input(void *stream, const float *x, int m0, int m1, int rows, int K, void *x16, void *x16t,
+                                   long ldt, const float *tgt_src, float *tgt) {
+    if (m0 % 64 || m1 % 64 || K % 32 || m0 < 0 || m1 <= m0 || rows <= 0 || K <= 0 || ((uintptr_t)x & 15))
+        return (int)hipErrorInvalidValue;
+    stage_input_kernel<<<dim3((m1 - m0) / 64, K / 32), 256, 0, (hipStream_t)stream>>>(
+        x, m0, rows, K, (bf16 *)x16, (bf16 *)x16t, ldt, tgt_src, tgt);
+    ORK_LAUNCH_CHECK();
+    return 0;
+}
+
+// dst = the arrays src[i] of len[i] floats (multiples of 4) one after the other; dst and every src on 16 B boundaries
+extern "C" int ork_mlp_pack(void *stream, int count, const float *const *src, const int *len, float *dst) {
+    if (count < 1 || count > PACK_MAX) return (int)hipErrorInvalidValue;
+    PackArgs a{};
+    long total = 0;
+    for (int i = 0; i < count; ++i) {
+        if (len[i] <= 0 || len[i] % 4) return (int)hipErrorInvalidValue;
+        a.src[i] = src[i];
+        a.first[i] = (int)total;
+        total += len[i] / 4;
+    }
+    if (total > (1 << 28)) return (int)hipErrorInvalidValue;
+    a.first[count] = (int)total;
+    a.count = count;
+    pack_kernel<<<(unsigned)((total + 1023) / 1024), 256, 0, (hipStream_t)stream>>>(a, (float4 *)dst);
     ORK_LAUNCH_CHECK();
     return 0;
 }
@@ -485,8 +547,8 @@ extern "C" int ork_mlp_weight_grads(void *stream, int nl, const void *const *xt,
     return 0;
 }
 
-// out[i][k] = sum_m a[i][m][k] (s[i] ? s[i][m] : 1), i < count; vout[0..1] = sums of v0 and v1 over M; part: count x 64 x
-// K floats
+// out[i][k] = sum_m a[i][m][k] (s[i] ? s[i][m] : 1), i < count; vout[0..1] = sums of v0 and v1 over M (device or pinned host
+// memory); part: count x 64 x K floats
 extern "C" int ork_mlp_colsums(void *stream, int count, const void *const *a, const float *const *s, float *const *out,
                                int M, int K, float *part, const float *v0, const float *v1, float *vout) {
     if (count < 1 || count > CS_MAX || K % 8 || K <= 0 || M <= 0) return (int)hipErrorInvalidValue;

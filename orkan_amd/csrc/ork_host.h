@@ -41,6 +41,7 @@ typedef struct {
     void *phase;           /* exp_diag per-index phases */
     size_t phase_bytes;
     double *sop2;          /* channel_2q's superoperator: 256 complex */
+    float *host;           /* ork_host_take: ORK_HOST_FLOATS, pinned */
     int noalloc_err;       /* result of ork_noalloc_setup() on this device */
 } ork_dev_t;
 
@@ -55,6 +56,14 @@ ork_dev_t *ork_dev_existing(void);
 void *ork_mem_get(size_t bytes);
 void ork_mem_put(void *p);
 void ork_mem_release(void *p);
+/* pinned host memory for arrays on their way between a caller's pageable memory and a kernel (4.25 MB: 8192 rows of 128
+ * floats and as many targets).  One buffer per device, because a new one costs 0.6 ms of page faults: made by
+ * ork_host_prepare, had by one caller at a time (ork_host_take: NULL if another has it or there is none) until
+ * ork_host_give, by when the stream must be done with it. */
+#define ORK_HOST_FLOATS ((size_t)17 << 16)
+void ork_host_prepare(void);
+float *ork_host_take(void);
+void ork_host_give(void);
 /* does p address device memory? */
 int ork_is_dev_ptr(const void *p);
 void ork_lock(void);

@@ -18,7 +18,9 @@ int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const void *B, i
                  float *c32, int ldc, const float *bias, float *pre, void *act);
 int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
                      float *c32, int ldc, const float *bias, float *pre, void *act, void *actT, long ldt);
-int ork_mlp_stage_input(void *stream, const float *x, int rows, int M, int K, void *x16, void *x16t, long ldt);
+int ork_mlp_stage_input(void *stream, const float *x, int m0, int m1, int rows, int K, void *x16, void *x16t, long ldt,
+                        const float *tgt_src, float *tgt);
+int ork_mlp_pack(void *stream, int count, const float *const *src, const int *len, float *dst);
 int ork_mlp_head_forward(void *stream, const void *h, const float *w, float b, int M, int K, float *y,
                          const float *target, float *dy, float *sqerr, int valid, float scale);
 int ork_mlp_head_backward_t(void *stream, const float *dy, const float *w, const float *pre, int M, int K, void *dpre,
@@ -41,6 +43,8 @@ int ork_mlp_adam_all(void *stream, int count, float *const *w, const float *cons
 #define MLP_MAX_LAYERS 4
 #define SPLITK_MAX 32   /* K slices of the weight-gradient products */
 #define TILE 128
+/* of a host batch: the host copies one chunk while the device reads the one before */
+#define CHUNK_FLOATS ((size_t)1 << 17)
 #define TPAD 64         /* row padding of the transposed operands: rows a power of two apart share memory channels */
 
 typedef struct {
@@ -64,7 +68,8 @@ struct orkan_mlp {
     /* transposed operands of the weight gradients: the layers' inputs and dpre, bf16 [width][M + TPAD] */
     void *in_t[MLP_MAX_LAYERS], *dpre_t[MLP_MAX_LAYERS];
     float *y, *dy, *sq, *tgt;
-    float *scal;                /* sum of squared errors, d loss / d b_out */
+    float *scal;                /* sum of squared errors, d loss / d b_out; pinned */
+    float *host;                /* the pinned buffer, while a batch staged in it is on its way */
     float *colpart;             /* (nl + 1) x 64 x hidden partial column sums */
     float *gf_dev, *u1;         /* screening: graph features [in_dim], their layer-1 share [hidden] */
     void *wpk;                  /* screening: the later layers' weights in fragment order */
@@ -79,6 +84,17 @@ static void *dmalloc(size_t bytes, int *err) {
         return NULL;
     }
     return p;
+}
+
+/* memory the HIP runtime does not know: nothing on a stream can be writing or reading it */
+static int pageable(const void *p) {
+    hipPointerAttribute_t at;
+    memset(&at, 0, sizeof(at));
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    return at.type == hipMemoryTypeUnregistered;
 }
 
 static int pad_rows(int m) { return (m + TILE - 1) / TILE * TILE; }
@@ -120,11 +136,12 @@ orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch
     q->x16 = dmalloc(M * in_dim * 2, &err);
     q->y = dmalloc(M * 4, &err); q->dy = dmalloc(M * 4, &err);
     q->sq = dmalloc(M * 4, &err); q->tgt = dmalloc(M * 4, &err);
-    q->scal = dmalloc(64, &err);
     q->colpart = dmalloc((size_t)(nhidden + 1) * 64 * H * 4, &err);
     q->gf_dev = dmalloc((size_t)in_dim * 4, &err);
     q->u1 = dmalloc(H * 4, &err);
     if (ork_mlp_screen_ok(8, hidden, nhidden)) q->wpk = dmalloc((size_t)(nhidden - 1) * H * H * 2, &err);
+    if (!err && hipHostMalloc((void **)&q->scal, 64, hipHostMallocDefault) != hipSuccess) err = 1;
+    ork_host_prepare();
     if (err) {
         orkan_mlp_destroy(q);
         return NULL;
@@ -153,10 +170,11 @@ void orkan_mlp_destroy(orkan_mlp_t *q) {
         for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
             if (p[i]) (void)hipFree(p[i]);
     }
-    void *p[] = {q->w_out, q->g_out, q->m_out, q->v_out, q->x32, q->x16, q->y, q->dy, q->sq, q->tgt, q->scal,
+    void *p[] = {q->w_out, q->g_out, q->m_out, q->v_out, q->x32, q->x16, q->y, q->dy, q->sq, q->tgt,
                  q->colpart, q->gf_dev, q->u1, q->wpk};
     for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
         if (p[i]) (void)hipFree(p[i]);
+    if (q->scal) (void)hipHostFree(q->scal);
     free(q);
 }
 
@@ -204,6 +222,39 @@ int orkan_mlp_get_weights(orkan_mlp_t *q, float *const *W, float *const *b, floa
     if (!q) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     int e = 0;
+    /* into pageable memory: packed by one kernel into pinned memory, copied from there by the host (2.4 MB of a 128 ->
+     * 512 -> 512 -> 512 -> 1 network: 240 us with a copy per array, 134 so, 44 of them the kernel) */
+    const float *src[2 * MLP_MAX_LAYERS + 1];
+    float *dst[2 * MLP_MAX_LAYERS + 1];
+    int len[2 * MLP_MAX_LAYERS + 1], n = 0, host = 1;
+    size_t total = 0;
+    for (int l = 0; l < q->nl; ++l) {
+        const layer_t *L = &q->L[l];
+        if (W && W[l]) {
+            src[n] = L->w; dst[n] = W[l]; len[n++] = L->K * L->N;
+        }
+        if (b && b[l]) {
+            src[n] = L->b; dst[n] = b[l]; len[n++] = L->N;
+        }
+    }
+    if (w_out) {
+        src[n] = q->w_out; dst[n] = w_out; len[n++] = q->hidden;
+    }
+    for (int i = 0; i < n; ++i) {
+        total += (size_t)len[i];
+        host &= pageable(dst[i]);
+    }
+    float *buf = n && host && total <= ORK_HOST_FLOATS ? ork_host_take() : NULL;
+    if (buf) {
+        e = ork_mlp_pack(st, n, src, len, buf);
+        const int es = (int)hipStreamSynchronize(st);
+        if (!e) e = es;
+        const float *from = buf;
+        for (int i = 0; i < n && !e; from += len[i++]) memcpy(dst[i], from, (size_t)len[i] * 4);
+        ork_host_give();
+        if (b_out) *b_out = q->b_out;
+        return e;
+    }
     for (int l = 0; l < q->nl; ++l) {
         layer_t *L = &q->L[l];
         if (W && W[l]) e |= (int)hipMemcpyAsync(W[l], L->w, (size_t)L->K * L->N * 4, hipMemcpyDeviceToHost, st);
@@ -236,12 +287,48 @@ static int forward_rows(orkan_mlp_t *q, int Mp, int training) {
     return 0;
 }
 
-/* x (host or device) -> bf16, padding rows zero; for training also its transpose */
-static int stage_input(orkan_mlp_t *q, const float *x, int rows, int Mp, int training) {
+/* x (host or device) -> bf16, padding rows zero */
+static int stage_input(orkan_mlp_t *q, const float *x, int rows, int Mp) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     int e = (int)hipMemcpyAsync(q->x32, x, (size_t)rows * q->in_dim * 4, hipMemcpyDefault, st);
-    if (!e) e = ork_mlp_stage_input(st, q->x32, rows, Mp, q->in_dim, q->x16, training ? q->in_t[0] : NULL, (long)Mp + TPAD);
+    if (!e) e = ork_mlp_stage_input(st, q->x32, 0, Mp, rows, q->in_dim, q->x16, NULL, 0, NULL, NULL);
     return e;
+}
+
+/* A training batch, x and target in host or device memory: x as in stage_input, its transpose and the targets.  Pageable
+ * batches that fit go through pinned memory, which the kernel reads as the host fills it, unless another thread's batch is on
+ * its way there; wait_batch gives it back.  A step of 4096 rows of 128: 245 us
+ * with hipMemcpy and a copy of the loss back, 195 so (130 with the batch on the device). */
+static int stage_batch(orkan_mlp_t *q, const float *x, const float *target, int rows, int Mp) {
+    hipStream_t st = (hipStream_t)ork_dev()->stream;
+    const size_t K = (size_t)q->in_dim;
+    const long ldt = (long)Mp + TPAD;
+    if (x && target && (size_t)rows * (K + 1) <= ORK_HOST_FLOATS && pageable(x) && pageable(target))
+        q->host = ork_host_take();
+    if (q->host) {
+        float *hx = q->host, *ht = hx + (size_t)rows * K;
+        memcpy(ht, target, (size_t)rows * 4);
+        int chunk = (int)(CHUNK_FLOATS / K) & ~63, e = 0;
+        if (chunk < 64) chunk = 64;
+        for (int m0 = 0; m0 < Mp && !e; m0 += chunk) {
+            const int m1 = Mp - m0 < chunk ? Mp : m0 + chunk, r1 = m1 < rows ? m1 : rows;
+            if (r1 > m0) memcpy(hx + (size_t)m0 * K, x + (size_t)m0 * K, (size_t)(r1 - m0) * K * 4);
+            e = ork_mlp_stage_input(st, hx, m0, m1, rows, q->in_dim, q->x16, q->in_t[0], ldt, ht, q->tgt);
+        }
+        return e;
+    }
+    int e = (int)hipMemcpyAsync(q->x32, x, (size_t)rows * K * 4, hipMemcpyDefault, st);
+    if (!e) e = (int)hipMemcpyAsync(q->tgt, target, (size_t)rows * 4, hipMemcpyDefault, st);
+    if (!e) e = ork_mlp_stage_input(st, q->x32, 0, Mp, rows, q->in_dim, q->x16, q->in_t[0], ldt, NULL, NULL);
+    return e;
+}
+
+/* the end of a call that staged a batch; e: its error so far */
+static int wait_batch(orkan_mlp_t *q, int e) {
+    const int es = (int)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
+    if (q->host) ork_host_give();
+    q->host = NULL;
+    return e ? e : es;
 }
 
 /* y[i] for batch rows of x (host or device pointer, [batch][in_dim] fp32); any batch size */
@@ -251,7 +338,7 @@ int orkan_mlp_forward(orkan_mlp_t *q, int batch, const float *x, float *y) {
     for (int r0 = 0; r0 < batch; r0 += q->max_batch) {
         const int rows = batch - r0 < q->max_batch ? batch - r0 : q->max_batch;
         const int Mp = pad_rows(rows);
-        int e = stage_input(q, x + (size_t)r0 * q->in_dim, rows, Mp, 0);
+        int e = stage_input(q, x + (size_t)r0 * q->in_dim, rows, Mp);
         if (!e) e = forward_rows(q, Mp, 0);
         if (!e) e = ork_mlp_head_forward(st, q->act[q->nl - 1], q->w_out, q->b_out, Mp, q->hidden, q->y, NULL, NULL,
                                          NULL, rows, 1.0f);
@@ -305,13 +392,12 @@ int orkan_mlp_forward_candidates(orkan_mlp_t *q, const float *gf_host, int ng, c
 
 /* gradients of the mean squared error of the staged batch into the g buffers; the sum of squared errors and
  * d loss / d b_out into scal[0] and scal[1].  12 launches (one step of 4096 rows of a 128 -> 512 -> 512 -> 512 -> 1
- * network, host batches and every fourth step's weights included: 302 us against 545 with a launch per layer and operand, 37 in all) */
-static int backward(orkan_mlp_t *q, int rows, const float *target) {
+ * network, host batches and every fourth step's weights included: 234 us against 545 with a launch per layer and operand, 37 in all) */
+static int backward(orkan_mlp_t *q, int rows) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     const int Mp = pad_rows(rows), H = q->hidden, nl = q->nl;
     const long ldt = (long)Mp + TPAD;
-    int e = (int)hipMemcpyAsync(q->tgt, target, (size_t)rows * 4, hipMemcpyDefault, st);
-    if (!e) e = forward_rows(q, Mp, 1);
+    int e = forward_rows(q, Mp, 1);
     if (!e) e = ork_mlp_head_forward(st, q->act[nl - 1], q->w_out, q->b_out, Mp, H, q->y, q->tgt, q->dy, q->sq,
                                      rows, 1.0f / (float)rows);
     if (!e) e = ork_mlp_head_backward_t(st, q->dy, q->w_out, q->pre[nl - 1], Mp, H, q->dpre[nl - 1], q->dpre_t[nl - 1],
@@ -346,19 +432,16 @@ static int backward(orkan_mlp_t *q, int rows, const float *target) {
 
 int orkan_mlp_train_step(orkan_mlp_t *q, int batch, const float *x, const float *target, float lr, float *loss) {
     if (!q || batch <= 0 || batch > q->max_batch) return (int)hipErrorInvalidValue;
-    hipStream_t st = (hipStream_t)ork_dev()->stream;
-    int e = stage_input(q, x, batch, pad_rows(batch), 1);
-    if (!e) e = backward(q, batch, target);
-    if (e) return e;
+    int e = stage_batch(q, x, target, batch, pad_rows(batch));
+    if (!e) e = backward(q, batch);
+    if (e) return wait_batch(q, e);
     q->step += 1;
     const float b1 = 0.9f, b2 = 0.999f, eps = 1e-8f;
     const float c1 = 1.0f - powf(b1, (float)q->step), c2 = 1.0f - powf(b2, (float)q->step);
     e = adam(q, 1, lr, b1, b2, eps, c1, c2);
-    float s[2] = {0.0f, 0.0f};
-    if (!e) e = (int)hipMemcpyAsync(s, q->scal, sizeof(s), hipMemcpyDeviceToHost, st);
-    if (!e) e = (int)hipStreamSynchronize(st);
+    e = wait_batch(q, e);
     if (e) return e;
-    const float gb = s[1];
+    const float *s = q->scal, gb = s[1];
     q->mb_out = b1 * q->mb_out + (1 - b1) * gb;
     q->vb_out = b2 * q->vb_out + (1 - b2) * gb * gb;
     q->b_out -= lr * (q->mb_out / c1) / (sqrtf(q->vb_out / c2) + eps);
@@ -371,17 +454,16 @@ int orkan_mlp_grads(orkan_mlp_t *q, int batch, const float *x, const float *targ
                     float *const *db, float *dw_out, float *db_out, float *loss) {
     if (!q || batch <= 0 || batch > q->max_batch) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    int e = stage_input(q, x, batch, pad_rows(batch), 1);
-    if (!e) e = backward(q, batch, target);
+    int e = stage_batch(q, x, target, batch, pad_rows(batch));
+    if (!e) e = backward(q, batch);
     for (int l = 0; l < q->nl && !e; ++l) {
         if (dW && dW[l]) e |= (int)hipMemcpyAsync(dW[l], q->L[l].g, (size_t)q->L[l].K * q->L[l].N * 4,
                                                    hipMemcpyDeviceToHost, st);
         if (db && db[l]) e |= (int)hipMemcpyAsync(db[l], q->L[l].gb, (size_t)q->L[l].N * 4, hipMemcpyDeviceToHost, st);
     }
     if (!e && dw_out) e = (int)hipMemcpyAsync(dw_out, q->g_out, (size_t)q->hidden * 4, hipMemcpyDeviceToHost, st);
-    float s[2] = {0.0f, 0.0f};
-    if (!e) e = (int)hipMemcpyAsync(s, q->scal, sizeof(s), hipMemcpyDeviceToHost, st);
-    if (!e) e = (int)hipStreamSynchronize(st);
+    e = wait_batch(q, e);
+    const float *s = q->scal;
     if (!e && db_out) *db_out = s[1];
     if (!e && loss) *loss = s[0] / (float)batch;
     return e;

@@ -14,6 +14,7 @@
 static ork_dev_t g_dev[ORK_MAX_DEV];
 static int g_ready[ORK_MAX_DEV];
 static pthread_mutex_t g_mu = PTHREAD_MUTEX_INITIALIZER;        /* ork_lock: shared staging, partials */
+static pthread_mutex_t g_host_mu = PTHREAD_MUTEX_INITIALIZER;   /* held by whoever has the pinned buffer */
 static pthread_mutex_t g_init_mu = PTHREAD_MUTEX_INITIALIZER;   /* per-device runtime creation, so that
                                                                  * ork_dev() may be called under ork_lock */
 
@@ -230,6 +231,28 @@ void ork_mem_release(void *p) {
     if (dev >= 0 && dev != cur) (void)hipSetDevice(cur);
     ork_mem_put(p);
 }
+
+void ork_host_prepare(void) {
+    ork_dev_t *d = ork_dev();
+    pthread_mutex_lock(&g_host_mu);
+    if (!d->host) {
+        void *p = NULL;
+        if (hipHostMalloc(&p, ORK_HOST_FLOATS * sizeof(float), hipHostMallocDefault) == hipSuccess)
+            d->host = memset(p, 0, ORK_HOST_FLOATS * sizeof(float));
+        else
+            (void)hipGetLastError();
+    }
+    pthread_mutex_unlock(&g_host_mu);
+}
+
+float *ork_host_take(void) {
+    float *p = NULL;
+    if (pthread_mutex_trylock(&g_host_mu) != 0) return NULL;
+    if (!(p = ork_dev()->host)) pthread_mutex_unlock(&g_host_mu);
+    return p;
+}
+
+void ork_host_give(void) { pthread_mutex_unlock(&g_host_mu); }
 
 /* ------------------------------------------------------------------------------------------------
  * extension API: stream access, device arrays, timing

@@ -1,6 +1,7 @@
 """The BF16 MFMA surrogate kernels: GEMM exactness on bf16-exact operands (pins
 the MFMA operand and accumulator lane layout), forward and backward against the
 CPU oracle (oracle/mlp_np.py, bf16 variant), and training that lowers the loss."""
+import ctypes as C
 import os
 import sys
 
@@ -212,3 +213,42 @@ def test_screening_equals_the_assembled_rows(hidden, layers, ncand):
     for p in (dang, ydev):
         lib.orkan_dev_free(p)
     m.close()
+
+
+@pytest.mark.parametrize("rows,in_dim,hidden,layers", [
+    (1, 128, 128, 1), (63, 128, 128, 2), (65, 128, 128, 1), (1023, 128, 256, 2), (1025, 128, 512, 3), (130, 2048, 128, 1),
+    (8192, 128, 128, 1), (8700, 128, 128, 1), (40, 128, 1024, 4)])
+def test_host_batches_and_parameters_equal_device_ones(rows, in_dim, hidden, layers):
+    """Two Adam steps from host batches (through pinned memory in chunks: one chunk, several, a last one of padding
+    alone; 8700 rows by plain copies) and from device batches give the same losses and parameters, bit by bit, and
+    parameters set are read back as they were (one launch, or array by array where they exceed the pinned memory)."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(rows + hidden)
+    batches = [(rng.standard_normal((rows, in_dim)).astype(np.float32), rng.standard_normal(rows).astype(np.float32))
+               for _ in range(2)]
+    res = []
+    for device in (False, True):
+        m = surrogate.Mlp(lib, in_dim=in_dim, hidden=hidden, layers=layers, max_batch=rows)
+        if not res:
+            m.init(rng)
+            start = m.get_weights()
+        m.set_weights(*start)
+        again = m.get_weights()
+        assert all(np.array_equal(a, b) for i in (0, 1) for a, b in zip(again[i], start[i]))
+        assert np.array_equal(again[2], start[2])
+        losses = []
+        for x, t in batches:
+            if not device:
+                losses.append(m.train_step(x, t, 1e-3))
+                continue
+            px, pt, loss = upload(lib, x), upload(lib, t), C.c_float()
+            assert lib.orkan_mlp_train_step(m.h, rows, C.cast(px, surrogate.FP), C.cast(pt, surrogate.FP), 1e-3,
+                                            C.byref(loss)) == 0
+            losses.append(loss.value)
+            lib.orkan_dev_free(px)
+            lib.orkan_dev_free(pt)
+        res.append((losses, m.get_weights()))
+        m.close()
+    (la, (Wa, ba, wa, oa)), (lb, (Wb, bb, wb, ob)) = res
+    assert la == lb and oa == ob and np.array_equal(wa, wb)
+    assert all(np.array_equal(a, b) for a, b in zip(Wa + ba, Wb + bb))
