@@ -24,7 +24,8 @@ __global__ __launch_bounds__(SM_THREADS) void spread_kernel(double2 *__restrict_
 }
 
 __device__ __forceinline__ cd wmul(double wr, double wi, cd x) {
-    return cmk(fma(wr, x.x, -(wi * x.y)), fma(wr, x.y, wi * x.x));
+    // the products of x.y rounded, those of x.x fused: as the compiler contracts wr x.x - wi x.y and wr x.y + wi x.x
+    return cmk(fma(wr, x.x, -(wi * x.y)), fma(wi, x.x, wr * x.y));
 }
 
 // one term of a linear combination over cnt whole vectors: acc = [acc +] w v
