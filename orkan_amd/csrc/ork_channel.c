@@ -87,13 +87,16 @@ void channel_2q(state_t *state, const superop_t *sop, qubit_t q1, qubit_t q2) {
     m.k = 2;
     m.qs[0] = q1;
     m.qs[1] = q2;
-    /* a host superoperator goes to the device as a launch's arguments: a staged copy made the host wait for the
-     * stream in every call */
+    /* a superoperator in pageable memory goes to the device as a launch's arguments: a staged copy made the host wait
+     * for the stream in every call.  Pinned and managed memory may still be written by work on the stream: those are
+     * staged, in stream order */
     ork_lock();
     ork_dev_t *d = ork_dev();
     const double *S = (const double *)sop->data;
     int e = 0;
-    if (!ork_is_dev_ptr(S)) {
+    if (!ork_is_pageable(S)) {
+        S = ork_dev_doubles(S, 2 * 256);
+    } else {
         if (!d->sop2) d->sop2 = ork_mem_get(2 * 256 * sizeof(double));
         e = d->sop2 ? ork_put256(d->stream, d->sop2, S) : (int)hipErrorOutOfMemory;
         S = d->sop2;

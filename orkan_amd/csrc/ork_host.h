@@ -66,6 +66,8 @@ float *ork_host_take(void);
 void ork_host_give(void);
 /* does p address device memory? */
 int ork_is_dev_ptr(const void *p);
+/* does p address memory that the HIP runtime does not know?  Nothing on a stream can be writing or reading it */
+int ork_is_pageable(const void *p);
 void ork_lock(void);
 void ork_unlock(void);
 

@@ -86,17 +86,6 @@ static void *dmalloc(size_t bytes, int *err) {
     return p;
 }
 
-/* memory the HIP runtime does not know: nothing on a stream can be writing or reading it */
-static int pageable(const void *p) {
-    hipPointerAttribute_t at;
-    memset(&at, 0, sizeof(at));
-    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
-        (void)hipGetLastError();
-        return 1;
-    }
-    return at.type == hipMemoryTypeUnregistered;
-}
-
 static int pad_rows(int m) { return (m + TILE - 1) / TILE * TILE; }
 
 orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch) {
@@ -242,7 +231,7 @@ int orkan_mlp_get_weights(orkan_mlp_t *q, float *const *W, float *const *b, floa
     }
     for (int i = 0; i < n; ++i) {
         total += (size_t)len[i];
-        host &= pageable(dst[i]);
+        host &= ork_is_pageable(dst[i]);
     }
     float *buf = n && host && total <= ORK_HOST_FLOATS ? ork_host_take() : NULL;
     if (buf) {
@@ -303,7 +292,7 @@ static int stage_batch(orkan_mlp_t *q, const float *x, const float *target, int 
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     const size_t K = (size_t)q->in_dim;
     const long ldt = (long)Mp + TPAD;
-    if (x && target && (size_t)rows * (K + 1) <= ORK_HOST_FLOATS && pageable(x) && pageable(target))
+    if (x && target && (size_t)rows * (K + 1) <= ORK_HOST_FLOATS && ork_is_pageable(x) && ork_is_pageable(target))
         q->host = ork_host_take();
     if (q->host) {
         float *hx = q->host, *ht = hx + (size_t)rows * K;

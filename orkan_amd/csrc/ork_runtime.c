@@ -66,6 +66,16 @@ int ork_is_dev_ptr(const void *p) {
     return at.type == hipMemoryTypeDevice;
 }
 
+int ork_is_pageable(const void *p) {
+    hipPointerAttribute_t at;
+    memset(&at, 0, sizeof(at));
+    if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+        (void)hipGetLastError();
+        return 1;
+    }
+    return at.type == hipMemoryTypeUnregistered;
+}
+
 const double *ork_dev_doubles(const double *src, size_t count) {
     if (ork_is_dev_ptr(src)) return src;
     ork_dev_t *d = ork_dev();
