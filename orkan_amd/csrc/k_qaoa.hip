@@ -33,9 +33,12 @@ namespace {
 struct QaoaEval {
     int graph;       // index into the diagonal table
     int p;           // layers
-    int angle_off;   // offset (in doubles) of this evaluation's per-layer (gamma, cos beta, sin beta)
+    int angle_off;   // first of this evaluation's layers in the angle rows
     int pad;
 };
+
+// a layer's row: gamma, cos beta, sin beta and the power of two by which the layer's phases scale the state
+constexpr int ANG = 4;
 
 struct QaoaGraph {
     u64 diag_off;    // offset (in doubles) of C in the diagonal arena
@@ -86,11 +89,30 @@ __device__ __forceinline__ void rx_pair(cd &a, cd &b, double u) {
     }
 }
 
-// psi *= exp(-i C t) (circ_pure.c:27-32)
-__device__ __forceinline__ cd phase(cd v, double d, double t) {
+// psi *= exp(-i C t) (circ_pure.c:27-32), times the power of two `scale`
+__device__ __forceinline__ cd phase(cd v, double d, double t, double scale) {
     double s, c;
     sincos(d * t, &s, &c);
+    s *= scale;
+    c *= scale;
     return cmk(c * v.x + s * v.y, c * v.y - s * v.x);
+}
+
+// The scaled rx let the squared norm of a state of n qubits grow by up to 2^n per layer: past 2^1024 the sum overflows.
+// Once it may have grown by 2^RESCALE_BITS, the next layer's phases take its root out again, a power of two that
+// rx_scale puts back: exact, so circuits keep their bits wherever nothing overflowed.
+constexpr double RESCALE_BITS = 512.0;
+
+// product over layers of the squared modulus the scaled rx leave out, once per qubit, and of the scalings undone
+__device__ double rx_scale(const double *ang, int p, int n) {
+    double scale = 1.0;
+    for (int l = 0; l < p; ++l) {
+        const double c = ang[ANG * l + 1], s = ang[ANG * l + 2], d = ang[ANG * l + 3];
+        const double f2 = fabs(c) < fabs(s) ? s * s : c * c;
+        if (d != 1.0) scale /= d * d;
+        for (int q = 0; q < n; ++q) scale *= f2;
+    }
+    return scale;
 }
 
 // LDS tiles are padded with one slot after every 8 amplitudes, so that a lane
@@ -182,24 +204,17 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
         const int n = gr.n;
         const u64 N = (u64)1 << n;
         const double *C = A.diag + gr.diag_off;
-        const double *ang = A.angles + ev.angle_off;
+        const double *ang = A.angles + (u64)ev.angle_off * ANG;
         const double amp = 1.0 / sqrt((double)N);
         double acc = 0.0;
-        // product over layers of the squared modulus the scaled rx leave out, once per qubit
-        double scale = 1.0;
-        for (int l = 0; l < ev.p; ++l) {
-            const double c = ang[3 * l + 1], s = ang[3 * l + 2];
-            const double f2 = fabs(c) < fabs(s) ? s * s : c * c;
-            for (int q = 0; q < n; ++q) scale *= f2;
-        }
 
         if (n <= LT) {
             // ---- whole state in LDS ----
             for (int x = threadIdx.x; x < (int)N; x += THREADS) tile[pad(x)] = cmk(amp, 0.0);
             __syncthreads();
             for (int l = 0; l < ev.p; ++l) {
-                const double g = ang[3 * l];
-                const RxScaled rx(ang[3 * l + 1], ang[3 * l + 2]);
+                const double g = ang[ANG * l], d = ang[ANG * l + 3];
+                const RxScaled rx(ang[ANG * l + 1], ang[ANG * l + 2]);
                 for (int u0 = 0; u0 < PER; u0 += BC) {
                     double cv[BC];
 #pragma unroll
@@ -210,7 +225,7 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 #pragma unroll
                     for (int u = 0; u < BC; ++u) {
                         const int x = threadIdx.x + (u0 + u) * THREADS;
-                        if (x < (int)N) tile[pad(x)] = phase(tile[pad(x)], cv[u], g);
+                        if (x < (int)N) tile[pad(x)] = phase(tile[pad(x)], cv[u], g, d);
                     }
                 }
                 __syncthreads();
@@ -247,9 +262,9 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
             for (int k = 0; k <= ev.p; ++k) {
                 const bool btile = k & 1;
                 const bool last = (k == ev.p);
-                const double g = last ? 0.0 : ang[3 * k];
-                const RxScaled rx(last ? 1.0 : ang[3 * k + 1], last ? 0.0 : ang[3 * k + 2]);
-                const RxScaled rxp(k ? ang[3 * (k - 1) + 1] : 1.0, k ? ang[3 * (k - 1) + 2] : 0.0);
+                const double g = last ? 0.0 : ang[ANG * k], d = last ? 1.0 : ang[ANG * k + 3];
+                const RxScaled rx(last ? 1.0 : ang[ANG * k + 1], last ? 0.0 : ang[ANG * k + 2]);
+                const RxScaled rxp(k ? ang[ANG * (k - 1) + 1] : 1.0, k ? ang[ANG * (k - 1) + 2] : 0.0);
                 for (u64 ch = 0; ch < nchunk; ++ch) {
                     const u64 lo0 = ch << ls;
                     // global index of tile element x
@@ -263,7 +278,7 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
                             LOAD_C(cv, u0)
 #pragma unroll
                             for (int u = 0; u < BC; ++u)
-                                tile[pad(threadIdx.x + (u0 + u) * THREADS)] = phase(cmk(amp, 0.0), cv[u], g);
+                                tile[pad(threadIdx.x + (u0 + u) * THREADS)] = phase(cmk(amp, 0.0), cv[u], g, d);
                         }
                         __syncthreads();
                     } else {
@@ -283,7 +298,7 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
 #pragma unroll
                                 for (int u = 0; u < BC; ++u) {
                                     const int x = threadIdx.x + (u0 + u) * THREADS;
-                                    tile[pad(x)] = phase(tile[pad(x)], cv[u], g);
+                                    tile[pad(x)] = phase(tile[pad(x)], cv[u], g, d);
                                 }
                             }
                             __syncthreads();
@@ -311,7 +326,7 @@ __global__ __launch_bounds__(THREADS) void qaoa_persistent(QaoaArgs A) {
             }
         }
         const double tot = block_sum<THREADS>(acc, red);
-        if (threadIdx.x == 0) A.out[e] = tot * scale;
+        if (threadIdx.x == 0) A.out[e] = tot * rx_scale(ang, ev.p, n);
         __syncthreads();
     }
 }
@@ -419,6 +434,15 @@ __device__ __forceinline__ void rx4(Amps &v, unsigned mask, double u) {
     }
 }
 
+// DEEP: the layers' scalings (rescale_kernel), in kernels of their own: beside the others the test alone cost 0.6 % of a batch
+__device__ __forceinline__ void scale16(Amps &v, double d) {
+#pragma unroll
+    for (int u = 0; u < 16; ++u) {
+        v.re[u] *= d;
+        v.im[u] *= d;
+    }
+}
+
 // Memory index of a tile element: f(x) = (x >> ls) << 12 | (x & (2^ls - 1)) past the chunk's own offset in a gathered tile,
 // x itself in a contiguous one.  f acts on bits and a thread's and a register's share of x have no bit in common, so the
 // two shares join by xor, also through a further map that is linear over bits.
@@ -510,28 +534,17 @@ __device__ __forceinline__ double mean16(const Amps &v, const Diag &C, const Til
     return acc;
 }
 
-// product over layers of the squared modulus the scaled rx leave out, once per qubit
-__device__ double rx_scale(const double *ang, int p, int n) {
-    double scale = 1.0;
-    for (int l = 0; l < p; ++l) {
-        const double c = ang[3 * l + 1], s = ang[3 * l + 2];
-        const double f2 = fabs(c) < fabs(s) ? s * s : c * c;
-        for (int q = 0; q < n; ++q) scale *= f2;
-    }
-    return scale;
-}
-
 // an evaluation of a launch
 struct QaoaRec {
     u64 diag_off;    // of C in the diagonal arena (doubles)
     u64 tile;        // of its first tile in the state slots (tiles of 2^12 amplitudes)
-    int angle_off;   // of its per-layer (gamma, cos beta, sin beta)
+    int angle_off;   // of its first layer in the angle rows
     int p, n, m;     // layers, qubits, bits of the stored index: n, or n - 1 (SYM)
     int out, pad;    // place of its result
 };
 
 // states of at most one tile: a workgroup runs the whole circuit
-template <int SYM>
+template <int SYM, int DEEP>
 __global__ __launch_bounds__(RT_THREADS, SYM ? 2 : 3) void qaoa_one_tile(const QaoaRec *__restrict__ recs,
                                                               const double *__restrict__ angles,
                                                               const double *__restrict__ diag, double *__restrict__ out) {
@@ -540,7 +553,7 @@ __global__ __launch_bounds__(RT_THREADS, SYM ? 2 : 3) void qaoa_one_tile(const Q
     const int t = threadIdx.x;
     const QaoaRec r = recs[blockIdx.x];
     const int n = uni(r.m), p = uni(r.p);
-    const double *ang = angles + r.angle_off;
+    const double *ang = angles + (u64)r.angle_off * ANG;
     Diag C{buffer(diag + r.diag_off, (u64)8 << n), (1u << n) - 1, false};
     // layouts 2 and 1 take turns in holding the phase, 0 in between.  Amplitudes past 2^n are 0 and stay 0 (their bits carry
     // no rx)
@@ -555,8 +568,9 @@ __global__ __launch_bounds__(RT_THREADS, SYM ? 2 : 3) void qaoa_one_tile(const Q
         v.im[u] = 0.0;
     }
     for (int l = 0; l < p; ++l) {
-        const double g = uni(ang[3 * l]);
-        const RxFlip rx(uni(ang[3 * l + 1]), uni(ang[3 * l + 2]));
+        const double g = uni(ang[ANG * l]);
+        const RxFlip rx(uni(ang[ANG * l + 1]), uni(ang[ANG * l + 2]));
+        if (DEEP) scale16(v, uni(ang[ANG * l + 3]));
         if (l & 1) {
             phase16<1, 1>(v, C, m, (unsigned)lay_base<1>(t), g);
             rx4(v, b1, rx.u);
@@ -594,7 +608,7 @@ struct SweepArgs {
     int rec[RT_CLASSES], n[RT_CLASSES];   // first record and index bits of each
 };
 
-template <int SYM>
+template <int SYM, int DEEP>
 __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
     __shared__ double lds[RT_SLOTS];
     __shared__ double red[RT_THREADS / 64];
@@ -604,15 +618,15 @@ __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
     const int n = A.n[c];
     const unsigned b = blockIdx.x - A.first[c], ch = b & ((1u << (n - RT_BITS)) - 1);
     const QaoaRec r = A.recs[A.rec[c] + (int)(b >> (n - RT_BITS))];
-    const double *ang = A.angles + r.angle_off;
+    const double *ang = A.angles + (u64)r.angle_off * ANG;
     const bool gathered = k & 1, last = k == uni(r.p);
     // the flips of the layers before k
     bool flip = false;
-    for (int l = 0; !SYM && l < k; ++l) flip ^= fabs(uni(ang[3 * l + 1])) < fabs(uni(ang[3 * l + 2]));
+    for (int l = 0; !SYM && l < k; ++l) flip ^= fabs(uni(ang[ANG * l + 1])) < fabs(uni(ang[ANG * l + 2]));
     const Diag C{buffer(A.diag + r.diag_off, (u64)8 << n), (1u << n) - 1, flip};
-    const double g = last ? 0.0 : uni(ang[3 * k]);
-    const RxFlip rx(last ? 1.0 : uni(ang[3 * k + 1]), last ? 0.0 : uni(ang[3 * k + 2]));
-    const RxFlip rxp(k ? uni(ang[3 * k - 2]) : 1.0, k ? uni(ang[3 * k - 1]) : 0.0);
+    const double g = last ? 0.0 : uni(ang[ANG * k]);
+    const RxFlip rx(last ? 1.0 : uni(ang[ANG * k + 1]), last ? 0.0 : uni(ang[ANG * k + 2]));
+    const RxFlip rxp(k ? uni(ang[ANG * k - 3]) : 1.0, k ? uni(ang[ANG * k - 2]) : 0.0);
     const int ls = 2 * RT_BITS - n;
     // layer k - 1 is left to finish on tile bits ls..11, by layout
     const unsigned f0 = ls < 4 ? 15u & (15u << ls) : 0u;
@@ -656,6 +670,7 @@ __global__ __launch_bounds__(RT_THREADS, 3) void qaoa_sweep(SweepArgs A) {
     }
     double acc = 0.0;
     if (!last) {
+        if (DEEP) scale16(v, uni(ang[ANG * k + 3]));
         phase16<2, 0, SYM ? 2 : 4>(v, C, m, coff2, g);   // 4 spill beside change_layout_flip
         rx4(v, 15u, rx.u);
         if (SYM) change_layout_flip<2, 0>(v, lds, cross, rx.u);
@@ -686,14 +701,14 @@ __global__ __launch_bounds__(256) void qaoa_finish(const QaoaRec *__restrict__ r
     double acc = 0.0;
     for (int i = threadIdx.x; i < 1 << (r.m - RT_BITS); i += 256) acc += part[r.tile + (u64)i];
     const double tot = block_sum<256>(acc, red);
-    if (threadIdx.x == 0) out[r.out] = tot * rx_scale(angles + r.angle_off, r.p, r.n);
+    if (threadIdx.x == 0) out[r.out] = tot * rx_scale(angles + (u64)r.angle_off * ANG, r.p, r.n);
 }
 
 __global__ void reset_counter(unsigned *c) {
     if (threadIdx.x == 0 && blockIdx.x == 0) *c = 0u;
 }
 
-// A call's list from pinned host memory: rows of gamma, then of beta, as the per-layer (gamma, cos beta, sin beta) that the
+// A call's list from pinned host memory: rows of gamma, then of beta, as the per-layer rows that the
 // kernels read, and the records.  One launch and no wait in place of two copies from pageable memory (25 to 30 us of every
 // call, one evaluation of 18 qubits 100 -> 77 us); the cosines took the host 0.7 of 16.8 ms for 4096 evaluations.
 __global__ __launch_bounds__(256) void stage_kernel(const double *__restrict__ gb, u64 rows, double *__restrict__ angles,
@@ -704,9 +719,27 @@ __global__ __launch_bounds__(256) void stage_kernel(const double *__restrict__ g
     const double theta = 2.0 * gb[rows + i];   // rx(q, 2 beta): the reference evaluates cos(theta / 2) and sin(theta / 2)
     double s, c;
     sincos(theta / 2.0, &s, &c);
-    angles[3 * i] = gb[i];
-    angles[3 * i + 1] = c;
-    angles[3 * i + 2] = s;
+    angles[ANG * i] = gb[i];
+    angles[ANG * i + 1] = c;
+    angles[ANG * i + 2] = s;
+    angles[ANG * i + 3] = 1.0;
+}
+
+// the scalings of circuits deep enough to need any: one thread per evaluation
+__global__ __launch_bounds__(64) void rescale_kernel(const QaoaRec *__restrict__ recs, int count, double *__restrict__ angles) {
+    const int i = blockIdx.x * 64 + threadIdx.x;
+    if (i >= count) return;
+    const QaoaRec r = recs[i];
+    double *ang = angles + (u64)r.angle_off * ANG, grown = 0.0;   // log2 of the squared norm's growth since the last
+    for (int l = 0; l < r.p; ++l) {
+        if (grown >= RESCALE_BITS) {
+            const int h = (int)(grown * 0.5);
+            grown -= 2.0 * h;
+            ang[ANG * l + 3] = ldexp(1.0, -h);
+        }
+        const double c = ang[ANG * l + 1], s = ang[ANG * l + 2];
+        grown -= (double)r.n * log2(fmax(c * c, s * s));
+    }
 }
 
 // C(x) = sum_(i,j) w_ij [x_i != x_j] for one graph
@@ -790,8 +823,8 @@ extern "C" int ork_qaoa_launch(void *stream, int lt, int threads, int grid, cons
 
 // recs: `count` QaoaRec on the device, all of one form (sym), sorted by index bits, then by layers, both descending; n and p:
 // their index bits and layers on the host; the states of more than 12 bits have their tiles in `states`, one partial sum per
-// tile in `part`
-extern "C" int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const int *n, const int *p, int count,
+// tile in `part`; deep: their layers' scalings are not all 1
+extern "C" int ork_qaoa_sweeps(void *stream, int sym, int deep, const void *recs, const int *n, const int *p, int count,
                                const double *angles, const double *diag, void *states, double *part, double *out) {
     hipStream_t st = (hipStream_t)stream;
     const QaoaRec *r = (const QaoaRec *)recs;
@@ -802,8 +835,9 @@ extern "C" int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const in
         ++large;
     }
     if (count > large) {
-        if (sym) qaoa_one_tile<1><<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
-        else qaoa_one_tile<0><<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
+        auto *kernel = sym ? (deep ? qaoa_one_tile<1, 1> : qaoa_one_tile<1, 0>)
+                           : (deep ? qaoa_one_tile<0, 1> : qaoa_one_tile<0, 0>);
+        kernel<<<count - large, RT_THREADS, 0, st>>>(r + large, angles, diag, out);
         ORK_LAUNCH_CHECK();
     }
     for (int k = 0; k <= pmax && large; ++k) {
@@ -828,8 +862,8 @@ extern "C" int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const in
             i = j;
         }
         A.first[A.nclass] = blocks;
-        if (sym) qaoa_sweep<1><<<blocks, RT_THREADS, 0, st>>>(A);
-        else qaoa_sweep<0><<<blocks, RT_THREADS, 0, st>>>(A);
+        auto *kernel = sym ? (deep ? qaoa_sweep<1, 1> : qaoa_sweep<1, 0>) : (deep ? qaoa_sweep<0, 1> : qaoa_sweep<0, 0>);
+        kernel<<<blocks, RT_THREADS, 0, st>>>(A);
         ORK_LAUNCH_CHECK();
     }
     if (large) {
@@ -849,6 +883,14 @@ extern "C" int ork_qaoa_stage(void *stream, const double *gb, uint64_t rows, dou
     return 0;
 }
 
+// recs_dev: `count` staged records; where n p < 768 for all of them the state's squared norm stays below 2^768 and no
+// scaling is needed
+extern "C" int ork_qaoa_rescale(void *stream, const void *recs_dev, int count, double *angles) {
+    rescale_kernel<<<(unsigned)(count + 63) / 64, 64, 0, (hipStream_t)stream>>>((const QaoaRec *)recs_dev, count, angles);
+    ORK_LAUNCH_CHECK();
+    return 0;
+}
+
 extern "C" int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs, const double *diag, double *info) {
     diag_info_kernel<<<ngraphs, 256, 0, (hipStream_t)stream>>>((const QaoaGraph *)graphs, diag, info);
     ORK_LAUNCH_CHECK();
@@ -858,7 +900,7 @@ extern "C" int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs,
 extern "C" int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu) {
     hipError_t e = hipErrorInvalidValue;
     if (lt == RT_BITS && threads == RT_THREADS)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_sweep<0>, RT_THREADS, 0);
+        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_sweep<0, 0>, RT_THREADS, 0);
 #define ORK_QOCC(L, TH) \
     if (lt == L && threads == TH) e = hipOccupancyMaxActiveBlocksPerMultiprocessor(blocks_per_cu, qaoa_persistent<L, TH>, TH, 0);
     ORK_QOCC(10, 256) ORK_QOCC(10, 512) ORK_QOCC(10, 1024)

@@ -19,9 +19,10 @@ int ork_qaoa_launch(void *stream, int lt, int threads, int grid, const void *eva
                     const int *nevals, const void *graphs, const double *angles, const double *diag, void *states,
                     uint64_t slot_elems, double *out, unsigned *counter);
 int ork_qaoa_occupancy(int lt, int threads, int *blocks_per_cu);
-int ork_qaoa_sweeps(void *stream, int sym, const void *recs, const int *n, const int *p, int count, const double *angles,
+int ork_qaoa_sweeps(void *stream, int sym, int deep, const void *recs, const int *n, const int *p, int count, const double *angles,
                     const double *diag, void *states, double *part, double *out);
 int ork_qaoa_stage(void *stream, const double *gb, uint64_t rows, double *angles, const void *recs, int nrecs, void *recs_dst);
+int ork_qaoa_rescale(void *stream, const void *recs_dev, int count, double *angles);
 int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs, const double *diag, double *info);
 int ork_maxcut_diag(void *stream, double *out, int n, int ne, const int *ei, const int *ej, const double *w);
 
@@ -54,6 +55,7 @@ struct orkan_qaoa {
     unsigned char *sym_h;
     int states_short;      /* the device had no memory for all the scratch asked for */
     size_t room;           /* tiles per round of launches, as the staged records number them */
+    int deep;              /* the staged list holds a circuit that needs scalings (DEEP) */
     int wide;              /* the staged list holds a phase too large for the register kernel's sincos */
     hipGraph_t graph;
     hipGraphExec_t exec;
@@ -77,6 +79,8 @@ static int cus(void) {
 #define REG_THREADS 256
 #define REG_PHASE_MAX 1125899906842624.0   /* 2^50 */
 #define WIDE_THREADS 512
+/* qubits times layers from which a state's squared norm may outgrow the number range unless it is scaled down on the way */
+#define DEEP 768
 #define TILE_BYTES ((size_t)16 << REG_LT)
 /* state slots of the register kernels: evaluations beyond them go in further rounds of launches. 4096 evaluations of 10 to
  * 20 qubits: 29.0 ms with 64 or 128 MB, which the last-level cache can hold from one sweep to the next, 29.6 with 256 MB
@@ -218,7 +222,7 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     if (hipMalloc(&q->recs_d, (size_t)max_evals * sizeof(q_rec_t)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->order_d, (size_t)max_evals * sizeof(int)) != hipSuccess) goto fail;
     if (hipMalloc((void **)&q->nevals_d, sizeof(int)) != hipSuccess) goto fail;
-    if (hipMalloc((void **)&q->angles_d, (size_t)max_evals * max_p * 3 * sizeof(double)) != hipSuccess) goto fail;
+    if (hipMalloc((void **)&q->angles_d, (size_t)max_evals * max_p * 4 * sizeof(double)) != hipSuccess) goto fail;
     if (hipHostMalloc((void **)&q->gb_h, (size_t)max_evals * max_p * 2 * sizeof(double), hipHostMallocDefault) !=
             hipSuccess ||
         hipHostMalloc((void **)&q->recs_h, (size_t)max_evals * sizeof(q_rec_t), hipHostMallocDefault) != hipSuccess ||
@@ -351,17 +355,18 @@ static int next_round(const orkan_qaoa_t *q, int at) {
 static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma, const double *beta,
                  int any_shape) {
     if (nevals < 0 || nevals > q->max_evals) return (int)hipErrorInvalidValue;
-    q->wide = 0;
+    q->wide = q->deep = 0;
     for (int e = 0; e < nevals; ++e) {
         if (graph[e] < 0 || graph[e] >= q->ngraphs || p[e] < 1 || p[e] > q->max_p) return (int)hipErrorInvalidValue;
         q->evals_h[e].graph = graph[e];
         q->evals_h[e].p = p[e];
-        q->evals_h[e].angle_off = e * q->max_p * 3;
+        q->evals_h[e].angle_off = e * q->max_p;
         const double *g = gamma + (size_t)e * q->max_p, *b = beta + (size_t)e * q->max_p;
         memcpy(q->gb_h + (size_t)e * q->max_p, g, (size_t)p[e] * sizeof(double));
         memcpy(q->gb_h + ((size_t)nevals + e) * q->max_p, b, (size_t)p[e] * sizeof(double));
         for (int l = 0; l < p[e]; ++l)
             if (!(fabs(g[l]) * q->info_h[2 * graph[e]] < REG_PHASE_MAX)) q->wide = 1;
+        q->deep |= q->graphs_h[graph[e]].n >= (DEEP + p[e] - 1) / p[e];
         q->order_h[e] = e;
     }
     q->nstaged = nevals;
@@ -369,7 +374,7 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
     int e = ensure_states(q);
     if (e) return e;
     int nrecs = 0;
-    if (nevals > 0 && (any_shape || (is_reg(q) && !q->wide))) {
+    if (nevals > 0 && (any_shape || q->deep || (is_reg(q) && !q->wide))) {
         sort_recs(q, nevals);
         /* every round numbers its tiles from 0 */
         q->room = tile_room(q);
@@ -384,6 +389,7 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
     }
     if (nevals > 0) {
         e = ork_qaoa_stage(st, q->gb_h, (uint64_t)nevals * q->max_p, q->angles_d, q->recs_h, nrecs, q->recs_d);
+        if (!e && q->deep) e = ork_qaoa_rescale(st, q->recs_d, nrecs, q->angles_d);
         if (e) return e;
     }
     if (any_shape || !is_reg(q) || q->wide) {
@@ -415,7 +421,7 @@ int orkan_qaoa_launch_staged(orkan_qaoa_t *q) {
         for (int at = 0; at < q->nstaged;) {
             const int m = next_round(q, at);
             if (m == 0) return (int)hipErrorInvalidValue;
-            const int e = ork_qaoa_sweeps(st, q->sym_h[at], (const q_rec_t *)q->recs_d + at, q->n_h + at, q->p_h + at, m, q->angles_d,
+            const int e = ork_qaoa_sweeps(st, q->sym_h[at], q->deep, (const q_rec_t *)q->recs_d + at, q->n_h + at, q->p_h + at, m, q->angles_d,
                                           q->diag_d, q->states_d, (double *)((char *)q->states_d + q->room * TILE_BYTES),
                                           q->out_h);
             if (e) return e;
