@@ -74,6 +74,11 @@ int orkan_state_download(const state_t *state, void *host);
 double *orkan_dev_alloc(idx_t count);
 int orkan_dev_upload(double *dst_dev, const double *src_host, idx_t count);
 void orkan_dev_free(void *p);
+/* The storage of a freed state stays allocated, for the next state of nearly the same size: at most 8 GiB per device,
+ * given back when an allocation of the library finds the device full.  orkan_mem_trim gives it back now, the longest
+ * unused first, until at most keep_bytes are left on the current device (0: all of it, for other allocators of the
+ * process); returns the bytes still kept. */
+size_t orkan_mem_trim(size_t keep_bytes);
 /* byte copies between host memory and device memory from orkan_dev_alloc (stream-ordered, then waited for) */
 int orkan_copy_to_host(void *dst_host, const void *src_dev, size_t bytes);
 int orkan_copy_to_device(void *dst_dev, const void *src_host, size_t bytes);

@@ -30,6 +30,7 @@ EXTRA = {
     "orkan_dev_alloc": (C.c_void_p, [C.c_uint64]),
     "orkan_dev_upload": (C.c_int, [C.c_void_p, C.c_void_p, C.c_uint64]),
     "orkan_dev_free": (None, [C.c_void_p]),
+    "orkan_mem_trim": (C.c_size_t, [C.c_size_t]),
     "orkan_copy_to_host": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t]),
     "orkan_copy_to_device": (C.c_int, [C.c_void_p, C.c_void_p, C.c_size_t]),
     "orkan_stream": (C.c_void_p, []),

@@ -30,7 +30,7 @@ static void exp_any(state_t *state, const double *diag, double t) {
             }
             d->phase = NULL;
             d->phase_bytes = 0;
-            ORK_HIP("exp_diag scratch", hipMalloc(&d->phase, need));
+            ORK_HIP("exp_diag scratch", ork_dev_malloc(&d->phase, need));
             d->phase_bytes = need;
         }
         e = ork_dm_exp_diag(d->stream, ork_prec(state), ork_layout(state), LOG_TILE_DIM, state->data, state->qubits,

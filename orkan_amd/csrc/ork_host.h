@@ -56,6 +56,9 @@ ork_dev_t *ork_dev_existing(void);
 void *ork_mem_get(size_t bytes);
 void ork_mem_put(void *p);
 void ork_mem_release(void *p);
+/* hipMalloc for everything else that lives on the device: where the device has none left, the kept blocks go back to it
+ * first.  Returns a hipError_t; *p NULL on failure; freed with hipFree. */
+int ork_dev_malloc(void **p, size_t bytes);
 /* pinned host memory for arrays on their way between a caller's pageable memory and a kernel (4.25 MB: 8192 rows of 128
  * floats and as many targets).  One buffer per device, because a new one costs 0.6 ms of page faults: made by
  * ork_host_prepare, had by one caller at a time (ork_host_take: NULL if another has it or there is none) until

@@ -79,7 +79,7 @@ struct orkan_mlp {
 static void *dmalloc(size_t bytes, int *err) {
     void *p = NULL;
     if (*err) return NULL;
-    if (hipMalloc(&p, bytes ? bytes : 16) != hipSuccess) {
+    if (ork_dev_malloc(&p, bytes ? bytes : 16) != 0) {
         *err = 1;
         return NULL;
     }

@@ -131,12 +131,11 @@ static int ensure_states(orkan_qaoa_t *q) {
     q->states_bytes = 0;
     q->states_short = 0;
     drop_graph(q);
-    int e = (int)hipMalloc(&q->states_d, need);
+    int e = ork_dev_malloc(&q->states_d, need);
     while (e && need / 2 >= least) {
-        (void)hipGetLastError();
         need /= 2;
         q->states_short = 1;
-        e = (int)hipMalloc(&q->states_d, need);
+        e = ork_dev_malloc(&q->states_d, need);
     }
     if (e) {
         q->states_d = NULL;
@@ -209,26 +208,26 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
         total += (uint64_t)1 << nq[g];
         if (nq[g] > q->nmax) q->nmax = nq[g];
     }
-    if (hipMalloc((void **)&q->diag_d, total * sizeof(double)) != hipSuccess) goto fail;
+    if (ork_dev_malloc((void **)&q->diag_d, total * sizeof(double)) != 0) goto fail;
     for (int g = 0; g < ngraphs; ++g)
         if (hipMemcpyAsync(q->diag_d + q->graphs_h[g].diag_off, diags[g], ((size_t)1 << nq[g]) * sizeof(double),
                            hipMemcpyDefault, st) != hipSuccess)
             goto fail;
-    if (hipMalloc(&q->graphs_d, (size_t)ngraphs * sizeof(q_graph_t)) != hipSuccess) goto fail;
+    if (ork_dev_malloc(&q->graphs_d, (size_t)ngraphs * sizeof(q_graph_t)) != 0) goto fail;
     if (hipMemcpyAsync(q->graphs_d, q->graphs_h, (size_t)ngraphs * sizeof(q_graph_t), hipMemcpyHostToDevice, st) !=
         hipSuccess)
         goto fail;
-    if (hipMalloc(&q->evals_d, (size_t)max_evals * sizeof(q_eval_t)) != hipSuccess) goto fail;
-    if (hipMalloc(&q->recs_d, (size_t)max_evals * sizeof(q_rec_t)) != hipSuccess) goto fail;
-    if (hipMalloc((void **)&q->order_d, (size_t)max_evals * sizeof(int)) != hipSuccess) goto fail;
-    if (hipMalloc((void **)&q->nevals_d, sizeof(int)) != hipSuccess) goto fail;
-    if (hipMalloc((void **)&q->angles_d, (size_t)max_evals * max_p * 4 * sizeof(double)) != hipSuccess) goto fail;
+    if (ork_dev_malloc(&q->evals_d, (size_t)max_evals * sizeof(q_eval_t)) != 0) goto fail;
+    if (ork_dev_malloc(&q->recs_d, (size_t)max_evals * sizeof(q_rec_t)) != 0) goto fail;
+    if (ork_dev_malloc((void **)&q->order_d, (size_t)max_evals * sizeof(int)) != 0) goto fail;
+    if (ork_dev_malloc((void **)&q->nevals_d, sizeof(int)) != 0) goto fail;
+    if (ork_dev_malloc((void **)&q->angles_d, (size_t)max_evals * max_p * 4 * sizeof(double)) != 0) goto fail;
     if (hipHostMalloc((void **)&q->gb_h, (size_t)max_evals * max_p * 2 * sizeof(double), hipHostMallocDefault) !=
             hipSuccess ||
         hipHostMalloc((void **)&q->recs_h, (size_t)max_evals * sizeof(q_rec_t), hipHostMallocDefault) != hipSuccess ||
         hipHostMalloc((void **)&q->out_h, (size_t)max_evals * sizeof(double), hipHostMallocDefault) != hipSuccess)
         goto fail;
-    if (hipMalloc((void **)&q->counter_d, sizeof(unsigned)) != hipSuccess) goto fail;
+    if (ork_dev_malloc((void **)&q->counter_d, sizeof(unsigned)) != 0) goto fail;
     {
         double *info = ork_mem_get((size_t)ngraphs * 2 * sizeof(double));
         const int bad = !info || ork_qaoa_diag_info(st, ngraphs, q->graphs_d, q->diag_d, info) ||

@@ -87,7 +87,7 @@ const double *ork_dev_doubles(const double *src, size_t count) {
         }
         d->stage = NULL;
         d->stage_bytes = 0;
-        ORK_HIP("hipMalloc(stage)", hipMalloc(&d->stage, bytes));
+        ORK_HIP("hipMalloc(stage)", ork_dev_malloc(&d->stage, bytes));
         d->stage_bytes = bytes;
     }
     ORK_HIP("hipMemcpyAsync(stage)", hipMemcpyAsync(d->stage, src, bytes, hipMemcpyHostToDevice, (hipStream_t)d->stream));
@@ -102,8 +102,8 @@ const double *ork_dev_doubles(const double *src, size_t count) {
  * hipMalloc and hipFree map and unmap pages: a state_cp, relayout and precision conversion of a 12-qubit density
  * matrix (134 MB each) spent 9.2 of their 9.6 ms there, a sample_matrix call on 18 qubits about 1 of 4 ms.  Blocks given
  * back are therefore kept, per device, for the next request of nearly the same size.  At most ORK_MEM_KEEP bytes are
- * kept (the oldest blocks go back to the device first, larger ones at once), and all of them go back when the device
- * runs out.  A block is only handed out for use on the library stream, after everything that used it.
+ * kept (the oldest blocks go back to the device first, larger ones at once), and all of them go back when an allocation
+ * of the library finds the device full (ork_mem_get, ork_dev_malloc) or a caller asks (orkan_mem_trim).  A block is only handed out for use on the library stream, after everything that used it.
  * ---------------------------------------------------------------------------------------------- */
 #define ORK_MEM_KEEP ((size_t)8 << 30)
 #define ORK_MEM_BUCKETS 1024
@@ -152,6 +152,43 @@ static void mem_trim(int dev, size_t keep) {
     }
 }
 
+/* hipMalloc, a second time with the kept blocks given back */
+static int malloc_or_trim(int dev, void **p, size_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess && g_mem_kept[dev] > 0) {
+        (void)hipGetLastError();
+        mem_trim(dev, 0);
+        e = hipMalloc(p, bytes);
+    }
+    if (e != hipSuccess) {
+        (void)hipGetLastError();
+        *p = NULL;
+    }
+    return (int)e;
+}
+
+int ork_dev_malloc(void **p, size_t bytes) {
+    int dev = 0;
+    *p = NULL;
+    const hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return (int)e;
+    pthread_mutex_lock(&g_mem_mu);
+    const int r = malloc_or_trim(dev, p, bytes);
+    if (!r) mem_forget(*p);   /* an entry of this address is of a block that was freed elsewhere */
+    pthread_mutex_unlock(&g_mem_mu);
+    return r;
+}
+
+size_t orkan_mem_trim(size_t keep_bytes) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    pthread_mutex_lock(&g_mem_mu);
+    mem_trim(dev, keep_bytes);
+    const size_t kept = g_mem_kept[dev];
+    pthread_mutex_unlock(&g_mem_mu);
+    return kept;
+}
+
 void *ork_mem_get(size_t bytes) {
     int dev = 0;
     void *p = NULL;
@@ -167,16 +204,7 @@ void *ork_mem_get(size_t bytes) {
         mem_unkeep(best);
         p = best->p;
     } else {
-        if (hipMalloc(&p, bytes) != hipSuccess) {
-            (void)hipGetLastError();
-            mem_trim(dev, 0);
-            p = NULL;
-            if (hipMalloc(&p, bytes) != hipSuccess) {
-                (void)hipGetLastError();
-                p = NULL;
-            }
-        }
-        if (p) {
+        if (malloc_or_trim(dev, &p, bytes) == 0) {
             mem_forget(p);   /* an entry of this address is of a block that was freed elsewhere */
             mem_block_t *b = calloc(1, sizeof(*b));
             if (b) {
@@ -274,8 +302,7 @@ int orkan_sync(void) { return (int)hipStreamSynchronize((hipStream_t)ork_dev()->
 
 double *orkan_dev_alloc(idx_t count) {
     void *p = NULL;
-    if (hipMalloc(&p, (size_t)count * sizeof(double)) != hipSuccess) return NULL;
-    return (double *)p;
+    return ork_dev_malloc(&p, (size_t)count * sizeof(double)) == 0 ? (double *)p : NULL;
 }
 
 int orkan_dev_upload(double *dst_dev, const double *src_host, idx_t count) {

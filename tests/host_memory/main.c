@@ -1,0 +1,143 @@
+/*
+ * Drives the library's device-memory bookkeeping on a small device that exists only here: the HIP calls below hand out
+ * host memory against a capacity, in pages, and know what is live.  tests/test_host_memory.py links it with the C17 host
+ * layer and empty kernels and runs one case per process.
+ */
+#include "ork_host.h"
+#include "orkan.h"
+#include "orkan_amd.h"
+
+#include <stdio.h>
+#include <stdlib.h>
+#include <string.h>
+#include <hip/hip_runtime_api.h>
+
+#define MB ((size_t)1 << 20)
+#define PAGE ((size_t)4096)
+
+static struct { char *p; size_t bytes; } live[65536];
+static int nlive, nmallocs;
+static size_t used, capacity = 64 * MB;
+
+static size_t pages(size_t n) { return (n + PAGE - 1) / PAGE * PAGE; }
+
+hipError_t hipMalloc(void **p, size_t n) {
+    *p = NULL;
+    ++nmallocs;
+    if (used + pages(n) > capacity || nlive == 65536) return hipErrorOutOfMemory;
+    *p = aligned_alloc(PAGE, pages(n));
+    live[nlive].p = *p;
+    live[nlive++].bytes = n;
+    used += pages(n);
+    return hipSuccess;
+}
+hipError_t hipFree(void *p) {
+    for (int i = 0; i < nlive; ++i)
+        if (live[i].p == p) {
+            used -= pages(live[i].bytes);
+            live[i] = live[--nlive];
+            free(p);
+            return hipSuccess;
+        }
+    return p ? hipErrorInvalidValue : hipSuccess;
+}
+static int is_live(const void *p) {
+    for (int i = 0; i < nlive; ++i)
+        if (live[i].p == p) return 1;
+    return 0;
+}
+hipError_t hipMemGetAddressRange(hipDeviceptr_t *base, size_t *size, hipDeviceptr_t p) {
+    for (int i = 0; i < nlive; ++i)
+        if ((char *)p >= live[i].p && (char *)p < live[i].p + live[i].bytes) {
+            *base = live[i].p;
+            *size = live[i].bytes;
+            return hipSuccess;
+        }
+    return hipErrorInvalidValue;
+}
+hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *p) {
+    hipDeviceptr_t b;
+    size_t n;
+    memset(a, 0, sizeof *a);
+    a->type = hipMemGetAddressRange(&b, &n, (hipDeviceptr_t)p) == hipSuccess ? hipMemoryTypeDevice
+                                                                             : hipMemoryTypeUnregistered;
+    return hipSuccess;
+}
+hipError_t hipHostMalloc(void **p, size_t n, unsigned f) { (void)f; return (*p = calloc(1, n ? n : 1)) ? hipSuccess : hipErrorOutOfMemory; }
+hipError_t hipHostFree(void *p) { free(p); return hipSuccess; }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t st) { (void)k; (void)st; memmove(d, s, n); return hipSuccess; }
+hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) { (void)st; memset(d, v, n); return hipSuccess; }
+hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
+hipError_t hipSetDevice(int d) { (void)d; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = 4; return hipSuccess; }
+hipError_t hipGetLastError(void) { return hipSuccess; }
+const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
+int ork_qaoa_occupancy(int lt, int threads, int *blocks) { (void)lt; (void)threads; *blocks = 2; return 0; }
+
+typedef struct orkan_mlp orkan_mlp_t;
+orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch);
+
+#define CHECK(c)                                                                       \
+    do {                                                                               \
+        if (!(c)) {                                                                    \
+            fprintf(stderr, "host_memory: check failed: %s (line %d)\n", #c, __LINE__); \
+            exit(2);                                                                   \
+        }                                                                              \
+    } while (0)
+
+/* n qubits of 2^n x 16 B: 21 qubits are 32 MB */
+static state_t pure(qubit_t n) {
+    state_t s = {PURE, NULL, 0};
+    state_init(&s, n, NULL);
+    CHECK(s.data);
+    return s;
+}
+
+/* leaves 32 MB of the 64 kept beside a live state of 1 MB */
+static state_t fill(void) {
+    state_t s = pure(16), big = pure(21);
+    state_free(&big);
+    CHECK(used >= 33 * MB);
+    return s;
+}
+
+int main(int argc, char **argv) {
+    const char *what = argc > 1 ? argv[1] : "";
+    state_t s = fill();
+    if (!strcmp(what, "dev_alloc")) {
+        CHECK(orkan_dev_alloc(40 * MB / 8));
+    } else if (!strcmp(what, "staging")) {
+        double *host = calloc(40 * MB, 1);
+        CHECK(ork_dev_doubles(host, 40 * MB / 8));
+    } else if (!strcmp(what, "phases")) {
+        /* a packed state of 8 qubits, then phase scratch of 16 B per index on a device with a page left for it */
+        state_t m = {MIXED_PACKED, NULL, 0};
+        state_init(&m, 8, NULL);
+        capacity = used;
+        double *diag = calloc(256, 8);
+        CHECK(ork_dev_doubles(diag, 256));
+        exp_diag(&m, diag, 0.5);
+    } else if (!strcmp(what, "mlp")) {
+        CHECK(orkan_mlp_create(128, 128, 3, 8192));
+    } else if (!strcmp(what, "qaoa")) {
+        /* one 20-qubit graph: 8 MB of diagonal, 16 MB of state, and the whole scratch, not half of it */
+        const unsigned char nq = 20;
+        double *diag = calloc(8, 1 << 20);
+        const double *d = diag;
+        capacity = used + 4 * MB;
+        orkan_qaoa_t *q = orkan_qaoa_create(1, &nq, &d, 1, 2);
+        CHECK(q);
+        CHECK(used >= 1 * MB + 8 * MB + 16 * MB);
+    } else if (!strcmp(what, "trim")) {
+        size_t (*trim)(size_t) = orkan_mem_trim;
+        CHECK(trim((size_t)-1) >= 32 * MB);
+        CHECK(used >= 33 * MB);
+        CHECK(trim(0) == 0);
+        CHECK(used < 2 * MB);
+    } else {
+        return 3;
+    }
+    CHECK(is_live(s.data));
+    printf("host_memory ok %s\n", what);
+    return 0;
+}
