@@ -101,12 +101,15 @@ const double *ork_dev_doubles(const double *src, size_t count) {
  *
  * hipMalloc and hipFree map and unmap pages: a state_cp, relayout and precision conversion of a 12-qubit density
  * matrix (134 MB each) spent 9.2 of their 9.6 ms there, a sample_matrix call on 18 qubits about 1 of 4 ms.  Blocks given
- * back are therefore kept, per device, for the next request of nearly the same size.  At most ORK_MEM_KEEP bytes are
- * kept (the oldest blocks go back to the device first, larger ones at once), and all of them go back when an allocation
+ * back are therefore kept, per device, for the next request of nearly the same size.  At most ORK_MEM_KEEP bytes and
+ * ORK_MEM_BLOCKS blocks are kept (the oldest go back to the device first, larger ones at once), and all of them go back when an allocation
  * of the library finds the device full (ork_mem_get, ork_dev_malloc) or a caller asks (orkan_mem_trim).  A block is only handed out for use on the library stream, after everything that used it.
  * ---------------------------------------------------------------------------------------------- */
 #define ORK_MEM_KEEP ((size_t)8 << 30)
+#define ORK_MEM_BLOCKS 4096
 #define ORK_MEM_BUCKETS 1024
+/* size classes, eight per power of two: a request looks at the blocks of its own and the next one or two only */
+#define ORK_MEM_CLASSES (64 * 8)
 
 typedef struct mem_block {
     void *p;
@@ -115,12 +118,26 @@ typedef struct mem_block {
     int kept;                          /* given back, in its device's list */
     struct mem_block *chain;           /* next block of the same bucket */
     struct mem_block *older, *newer;   /* kept blocks of a device, by the time they came back */
+    struct mem_block *prev, *next;     /* ... of one size class */
 } mem_block_t;
 
 static pthread_mutex_t g_mem_mu = PTHREAD_MUTEX_INITIALIZER;
 static mem_block_t *g_mem_table[ORK_MEM_BUCKETS];
 static mem_block_t *g_mem_oldest[ORK_MAX_DEV], *g_mem_newest[ORK_MAX_DEV];
+static mem_block_t *g_mem_class[ORK_MAX_DEV][ORK_MEM_CLASSES];
 static size_t g_mem_kept[ORK_MAX_DEV];
+static int g_mem_blocks[ORK_MAX_DEV];
+
+/* what an allocation of `bytes` takes from the device (hipMemGetInfo): pages of 4 KB, from 2 MB on pages of 2 MB */
+static size_t mem_round(size_t bytes) {
+    const size_t page = (size_t)(bytes >= 2 << 20 ? 2 << 20 : 4 << 10);
+    return bytes == 0 ? page : bytes > SIZE_MAX - page ? bytes : (bytes + page - 1) / page * page;
+}
+
+static int mem_class(size_t bytes) {   /* bytes >= 4096 */
+    const int b = 63 - __builtin_clzll(bytes);
+    return b * 8 + (int)(bytes >> (b - 3) & 7);
+}
 
 static mem_block_t **mem_slot(const void *p) {
     mem_block_t **s = &g_mem_table[((uintptr_t)p >> 12) % ORK_MEM_BUCKETS];
@@ -131,7 +148,10 @@ static mem_block_t **mem_slot(const void *p) {
 static void mem_unkeep(mem_block_t *b) {
     *(b->older ? &b->older->newer : &g_mem_oldest[b->dev]) = b->newer;
     *(b->newer ? &b->newer->older : &g_mem_newest[b->dev]) = b->older;
+    *(b->prev ? &b->prev->next : &g_mem_class[b->dev][mem_class(b->bytes)]) = b->next;
+    if (b->next) b->next->prev = b->prev;
     g_mem_kept[b->dev] -= b->bytes;
+    g_mem_blocks[b->dev] -= 1;
     b->kept = 0;
 }
 
@@ -145,7 +165,7 @@ static void mem_forget(const void *p) {
 
 /* kept blocks of the device back to it, the oldest first, until at most `keep` bytes are left */
 static void mem_trim(int dev, size_t keep) {
-    while (g_mem_kept[dev] > keep) {
+    while (g_mem_kept[dev] > keep || g_mem_blocks[dev] > ORK_MEM_BLOCKS) {
         void *p = g_mem_oldest[dev]->p;
         mem_forget(p);
         (void)hipFree(p);
@@ -194,12 +214,14 @@ void *ork_mem_get(size_t bytes) {
     void *p = NULL;
     ork_dev();
     if (hipGetDevice(&dev) != hipSuccess) return NULL;
-    if (bytes < 256) bytes = 256;
+    bytes = mem_round(bytes);
     pthread_mutex_lock(&g_mem_mu);
     /* the smallest kept block that holds the request and is at most an eighth larger */
     mem_block_t *best = NULL;
-    for (mem_block_t *b = g_mem_newest[dev]; b; b = b->older)
-        if (b->bytes >= bytes && b->bytes - bytes <= bytes / 8 && (!best || b->bytes < best->bytes)) best = b;
+    const size_t most = bytes > SIZE_MAX - bytes / 8 ? bytes : bytes + bytes / 8;
+    for (int c = mem_class(bytes); c <= mem_class(most) && !best; ++c)
+        for (mem_block_t *b = g_mem_class[dev][c]; b && !(best && best->bytes == bytes); b = b->next)
+            if (b->bytes >= bytes && b->bytes <= most && (!best || b->bytes < best->bytes)) best = b;
     if (best) {
         mem_unkeep(best);
         p = best->p;
@@ -245,7 +267,13 @@ void ork_mem_put(void *p) {
         b->older = g_mem_newest[b->dev];
         *(b->older ? &b->older->newer : &g_mem_oldest[b->dev]) = b;
         g_mem_newest[b->dev] = b;
+        mem_block_t **first = &g_mem_class[b->dev][mem_class(b->bytes)];
+        b->prev = NULL;
+        b->next = *first;
+        if (*first) (*first)->prev = b;
+        *first = b;
         g_mem_kept[b->dev] += b->bytes;
+        g_mem_blocks[b->dev] += 1;
         mem_trim(b->dev, ORK_MEM_KEEP);
     } else {
         mem_forget(p);

@@ -128,6 +128,65 @@ int main(int argc, char **argv) {
         orkan_qaoa_t *q = orkan_qaoa_create(1, &nq, &d, 1, 2);
         CHECK(q);
         CHECK(used >= 1 * MB + 8 * MB + 16 * MB);
+    } else if (!strcmp(what, "count")) {
+        /* many tiny states: each holds a page, whatever its length, and a bounded number of them is kept */
+        static state_t t[6000];
+        for (int i = 0; i < 6000; ++i) t[i] = pure((qubit_t)(1 + i % 4));
+        for (int i = 0; i < 6000; ++i) state_free(&t[i]);
+        CHECK(used <= 1 * MB + 4096 * PAGE);
+        CHECK(orkan_mem_trim((size_t)-1) == used - 1 * MB);
+        /* the block for the next one is found, not allocated */
+        const int before = nmallocs;
+        for (int i = 0; i < 100; ++i) t[i] = pure(3);
+        CHECK(nmallocs == before);
+    } else if (!strcmp(what, "classes")) {
+        /* for every size, a block of it or of up to an eighth more is taken, the nearest one first; a larger one is not */
+        for (size_t n = 5000; n < 24 * MB; n += n / 3 + 4096) {
+            orkan_mem_trim(0);
+            void *exact = ork_mem_get(n), *more = ork_mem_get(n + n / 16 + (n >= 1 * MB ? 2 * MB : 4096));
+            ork_mem_put(exact);
+            ork_mem_put(more);
+            CHECK(ork_mem_get(n) == exact);
+            ork_mem_put(exact);
+            orkan_mem_trim(0);
+            void *twice = ork_mem_get(2 * n + 8192);
+            ork_mem_put(twice);
+            void *q = ork_mem_get(n);
+            CHECK(q && q != twice);
+            ork_mem_put(q);
+            CHECK(ork_mem_get(2 * n + 8192) == twice);
+            ork_mem_put(twice);
+        }
+    } else if (!strcmp(what, "cap")) {
+        /* five states of 4 GB (nothing touches their memory here): at most 8 GB stay, a larger block does not */
+        capacity = (size_t)1 << 40;
+        orkan_mem_trim(0);
+        const size_t base = used;
+        state_t big[5];
+        for (int i = 0; i < 5; ++i) {
+            big[i] = (state_t){PURE, NULL, 0};
+            state_plus(&big[i], 28);
+            CHECK(big[i].data);
+        }
+        for (int i = 0; i < 5; ++i) state_free(&big[i]);
+        CHECK(used - base == 8192 * MB);
+        big[0] = (state_t){PURE, NULL, 0};
+        state_plus(&big[0], 30);
+        state_free(&big[0]);
+        CHECK(used - base <= 8192 * MB);
+    } else if (!strcmp(what, "behind")) {
+        /* a state's storage freed by its address: releasing the state then frees nothing else, and the address may come
+         * back as somebody else's */
+        state_t a = pure(12);
+        void *p = a.data, *q;
+        CHECK(hipFree(p) == hipSuccess);
+        state_free(&a);
+        CHECK(hipMalloc(&q, 16 << 11) == hipSuccess);
+        state_t b = pure(12), c = pure(12);
+        CHECK(b.data != c.data && (void *)b.data != q && (void *)c.data != q && is_live(q));
+        state_free(&b);
+        state_free(&c);
+        CHECK(is_live(q));
     } else if (!strcmp(what, "trim")) {
         size_t (*trim)(size_t) = orkan_mem_trim;
         CHECK(trim((size_t)-1) >= 32 * MB);

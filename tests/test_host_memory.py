@@ -50,5 +50,11 @@ def test_kept_storage_goes_back_when_the_device_runs_out(program, what):
     run(program, what)
 
 
+@pytest.mark.parametrize("what", ["count", "classes", "cap", "behind"])
+def test_what_is_kept(program, what):
+    """By pages and by number, by size, at most 8 GB, and with an address freed behind the library's back."""
+    run(program, what)
+
+
 def test_kept_storage_is_released_on_request(program):
     run(program, "trim")
