@@ -83,8 +83,8 @@ static int cus(void) {
 #define DEEP 768
 #define TILE_BYTES ((size_t)16 << REG_LT)
 /* state slots of the register kernels: evaluations beyond them go in further rounds of launches. 4096 evaluations of 10 to
- * 20 qubits: 29.0 ms with 64 or 128 MB, which the last-level cache can hold from one sweep to the next, 29.6 with 256 MB
- * to 16 GB */
+ * 20 qubits, half states: 15.0 ms a call with 128 to 176 MB, which the last-level cache can hold from one sweep to the next;
+ * 17.3 with 64 MB, 16.2 with 256, 15.3 with 1 GB; 14.95 in one round, which takes 6.3 GB */
 #define SWEEP_BYTES ((size_t)128 << 20)
 
 static int is_reg(const orkan_qaoa_t *q) { return q->lt == REG_LT && q->threads == REG_THREADS; }
@@ -97,32 +97,40 @@ static void drop_graph(orkan_qaoa_t *q) {
     q->graph_ok = 0;
 }
 
+/* scratch of the register kernels: a slot for each evaluation up to SWEEP_BYTES, at least one of the largest state, and 8 B
+ * per tile for the partial sums */
+static size_t reg_bytes(const orkan_qaoa_t *q) {
+    if (q->nmax <= REG_LT) return 16;
+    const size_t slot = (size_t)16 << q->nmax;
+    size_t all = 0;
+    for (int g = 0; g < q->ngraphs; ++g)
+        if (q->graphs_h[g].n > REG_LT) all += (size_t)16 << q->graphs_h[g].n;
+    const size_t rounds = ((size_t)q->max_evals + q->ngraphs - 1) / q->ngraphs;
+    size_t need = all > SWEEP_BYTES / rounds ? SWEEP_BYTES : all * rounds;
+    if (need / slot > (size_t)q->max_evals) need = (size_t)q->max_evals * slot;
+    if (need < slot) need = slot;
+    return need + need / TILE_BYTES * sizeof(double) + 16;
+}
+
 /* The state scratch of the current configuration (and, for it, of the staged list). The LDS kernels need a slot of 2^nmax
- * for each workgroup. The register kernels take what there is: a slot for each evaluation up to SWEEP_BYTES and 8 B per
- * tile for the partial sums, halved while memory is short down to one slot of the largest state. */
-static int ensure_states(orkan_qaoa_t *q) {
+ * for each workgroup. The register kernels take what there is, halved while memory is short down to one slot of the
+ * largest state. shrink: what another configuration or list needed beyond that goes back. */
+static int ensure_states(orkan_qaoa_t *q, int shrink) {
     const size_t slot = (size_t)16 << q->nmax;
     size_t need = 16, least;
     if (is_reg(q)) {
         least = (q->nmax > REG_LT ? slot + slot / TILE_BYTES * sizeof(double) : 0) + 16;
-        if (q->nmax > REG_LT) {
-            size_t all = 0;
-            for (int g = 0; g < q->ngraphs; ++g)
-                if (q->graphs_h[g].n > REG_LT) all += (size_t)16 << q->graphs_h[g].n;
-            const size_t rounds = ((size_t)q->max_evals + q->ngraphs - 1) / q->ngraphs;
-            need = all > SWEEP_BYTES / rounds ? SWEEP_BYTES : all * rounds;
-            if (need / slot > (size_t)q->max_evals) need = (size_t)q->max_evals * slot;
-            if (need < slot) need = slot;
-            need += need / TILE_BYTES * sizeof(double) + 16;
-            /* qaoa_persistent takes lists with phases beyond REG_PHASE_MAX */
-            const size_t slots = q->max_evals < cus() ? (size_t)q->max_evals : (size_t)cus();
-            if (q->wide && need < slots * slot) need = slots * slot;
-        }
+        need = reg_bytes(q);
+        /* qaoa_persistent takes lists with phases beyond REG_PHASE_MAX */
+        const size_t slots = q->max_evals < cus() ? (size_t)q->max_evals : (size_t)cus();
+        if (q->nmax > REG_LT && q->wide && need < slots * slot) need = slots * slot;
     } else {
         if (q->nmax > q->lt) need = (size_t)q->grid * slot;
         least = need;
     }
-    if (q->states_bytes >= need || (q->states_bytes >= least && q->states_short)) return 0;
+    if ((q->states_bytes >= need || (q->states_bytes >= least && q->states_short)) &&
+        !(shrink && q->states_bytes > need))
+        return 0;
     if (q->states_d) {
         (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
         (void)hipFree(q->states_d);
@@ -145,13 +153,16 @@ static int ensure_states(orkan_qaoa_t *q) {
     return 0;
 }
 
-/* tiles of the register kernels that the state scratch holds, their partial sums behind them */
+/* Tiles of the register kernels that the state scratch holds, their partial sums behind them: of what they ask for, also
+ * where the scratch is larger for an LDS shape or a list with wide phases, so that a list runs in the rounds that the
+ * autotuner timed. */
 static size_t tile_room(const orkan_qaoa_t *q) {
-    return q->states_bytes < 16 ? 0 : (q->states_bytes - 16) / (TILE_BYTES + sizeof(double));
+    const size_t want = reg_bytes(q), have = q->states_bytes < want ? q->states_bytes : want;
+    return have < 16 ? 0 : (have - 16) / (TILE_BYTES + sizeof(double));
 }
 
 /* caller holds ork_lock (the state scratch may be freed and the graph dropped) */
-static int set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu) {
+static int set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu, int shrink) {
     if (2 * lt < q->nmax) return (int)hipErrorInvalidValue;     /* pass B needs n <= 2 LT */
     int occ = 0;
     int e = ork_qaoa_occupancy(lt, threads, &occ);
@@ -164,13 +175,13 @@ static int set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu) {
     q->threads = threads;
     q->grid = cus() * blocks_per_cu;
     if (q->grid > q->max_evals) q->grid = q->max_evals;   /* a workgroup takes at least one evaluation */
-    return ensure_states(q);
+    return ensure_states(q, shrink);
 }
 
 int orkan_qaoa_set_config(orkan_qaoa_t *q, int lt, int threads, int blocks_per_cu) {
     if (!q) return (int)hipErrorInvalidValue;
     ork_lock();
-    const int e = set_config(q, lt, threads, blocks_per_cu);
+    const int e = set_config(q, lt, threads, blocks_per_cu, 1);
     ork_unlock();
     return e;
 }
@@ -244,7 +255,7 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
         int lt = REG_LT;
         while (2 * lt < q->nmax) ++lt;
         ork_lock();
-        const int e = set_config(q, lt, lt >= 13 ? 1024 : REG_THREADS, 0);
+        const int e = set_config(q, lt, lt >= 13 ? 1024 : REG_THREADS, 0, 0);
         ork_unlock();
         if (e) goto fail;
     }
@@ -370,7 +381,7 @@ static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, co
     }
     q->nstaged = nevals;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    int e = ensure_states(q);
+    int e = ensure_states(q, 0);
     if (e) return e;
     int nrecs = 0;
     if (nevals > 0 && (any_shape || q->deep || (is_reg(q) && !q->wide))) {
@@ -477,7 +488,7 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
     /* the whole search holds the library lock: staging, every reconfiguration and launch */
     ork_lock();
     /* the register kernels' records number tiles of the scratch: it has its size for them first */
-    if (2 * REG_LT >= q->nmax) (void)set_config(q, REG_LT, REG_THREADS, 0);
+    if (2 * REG_LT >= q->nmax) (void)set_config(q, REG_LT, REG_THREADS, 0, 0);
     int e = stage(q, nevals, graph, p, gamma, beta, 1);
     if (e) {
         ork_unlock();
@@ -488,7 +499,7 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
     double best = 1e30;
     int best_i = -1;
     for (size_t i = 0; i < sizeof(cand) / sizeof(cand[0]); ++i) {
-        if (set_config(q, cand[i][0], cand[i][1], 0)) continue;
+        if (set_config(q, cand[i][0], cand[i][1], 0, 0)) continue;
         if (orkan_qaoa_launch_staged(q)) continue;
         float t[15];
         int ok = 1;
@@ -516,7 +527,7 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
         return (int)hipErrorInvalidConfiguration;
     }
     if (best_ms) *best_ms = best;
-    e = set_config(q, cand[best_i][0], cand[best_i][1], 0);
+    e = set_config(q, cand[best_i][0], cand[best_i][1], 0, 1);
     ork_unlock();
     return e;
 }

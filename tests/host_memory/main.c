@@ -7,6 +7,7 @@
 #include "orkan.h"
 #include "orkan_amd.h"
 
+#include <math.h>
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -69,10 +70,14 @@ hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hip
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t st) { (void)st; memset(d, v, n); return hipSuccess; }
 hipError_t hipGetDevice(int *d) { *d = 0; return hipSuccess; }
 hipError_t hipSetDevice(int d) { (void)d; return hipSuccess; }
-hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = 4; return hipSuccess; }
+hipError_t hipDeviceGetAttribute(int *v, hipDeviceAttribute_t a, int d) { (void)a; (void)d; *v = 64; return hipSuccess; }
 hipError_t hipGetLastError(void) { return hipSuccess; }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
 int ork_qaoa_occupancy(int lt, int threads, int *blocks) { (void)lt; (void)threads; *blocks = 2; return 0; }
+
+hipError_t hipEventElapsedTime(float *ms, hipEvent_t a, hipEvent_t b) { (void)a; (void)b; *ms = 1.0f; return hipSuccess; }
+static int rounds;   /* rounds of register-kernel launches */
+int ork_qaoa_sweeps() { ++rounds; return 0; }
 
 typedef struct orkan_mlp orkan_mlp_t;
 orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch);
@@ -128,6 +133,30 @@ int main(int argc, char **argv) {
         orkan_qaoa_t *q = orkan_qaoa_create(1, &nq, &d, 1, 2);
         CHECK(q);
         CHECK(used >= 1 * MB + 8 * MB + 16 * MB);
+    } else if (!strcmp(what, "qaoa_scratch")) {
+        /* 64 evaluations of 20 qubits: 128 MB of scratch, 8 states in a round.  The LDS shapes' GB, in the autotuner's
+         * search or a configuration, neither stay nor change the rounds. */
+        capacity = (size_t)8 << 30;
+        const unsigned char nq = 20;
+        double *diag = calloc(8, 1 << 20), *g = calloc(64 * 2, 8), *b = calloc(64 * 2, 8), out[64];
+        const double *d = diag;
+        static int graph[64], p[64];
+        for (int i = 0; i < 64; ++i) p[i] = 2;
+        orkan_qaoa_t *q = orkan_qaoa_create(1, &nq, &d, 64, 2);
+        CHECK(q);
+        const size_t at_first = used;
+        CHECK(orkan_qaoa_eval(q, 64, graph, p, g, b, out) == 0 && rounds == 8);
+        CHECK(orkan_qaoa_autotune(q, 64, graph, p, g, b, 1, NULL) == 0);
+        CHECK(orkan_qaoa_set_config(q, 12, 512, 0) == 0 && used > at_first + 64 * MB);
+        CHECK(orkan_qaoa_set_config(q, 12, 256, 0) == 0 && used == at_first);
+        rounds = 0;
+        CHECK(orkan_qaoa_eval(q, 64, graph, p, g, b, out) == 0 && rounds == 8);
+        /* nor do the slots of a list with a phase that the register kernels leave to an LDS one */
+        g[0] = INFINITY;
+        CHECK(orkan_qaoa_eval(q, 64, graph, p, g, b, out) == 0 && rounds == 8);
+        g[0] = 0.0;
+        CHECK(orkan_qaoa_eval(q, 64, graph, p, g, b, out) == 0 && rounds == 16);
+        orkan_qaoa_destroy(q);
     } else if (!strcmp(what, "count")) {
         /* many tiny states: each holds a page, whatever its length, and a bounded number of them is kept */
         static state_t t[6000];

@@ -58,3 +58,7 @@ def test_what_is_kept(program, what):
 
 def test_kept_storage_is_released_on_request(program):
     run(program, "trim")
+
+
+def test_batched_qaoa_scratch_is_that_of_the_configuration(program):
+    run(program, "qaoa_scratch")
