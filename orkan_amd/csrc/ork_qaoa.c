@@ -360,14 +360,20 @@ static int next_round(const orkan_qaoa_t *q, int at) {
     return i - at;
 }
 
+static int list_ok(const orkan_qaoa_t *q, int nevals, const int *graph, const int *p) {
+    if (nevals < 0 || nevals > q->max_evals) return 0;
+    for (int e = 0; e < nevals; ++e)
+        if (graph[e] < 0 || graph[e] >= q->ngraphs || p[e] < 1 || p[e] > q->max_p) return 0;
+    return 1;
+}
+
 /* stage the evaluation list; angles: rows of max_p gammas and betas.  any_shape: for every kernel, not only the one the
  * configuration and the list's phases call for */
 static int stage(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma, const double *beta,
                  int any_shape) {
-    if (nevals < 0 || nevals > q->max_evals) return (int)hipErrorInvalidValue;
+    if (!list_ok(q, nevals, graph, p)) return (int)hipErrorInvalidValue;   /* before anything changes */
     q->wide = q->deep = 0;
     for (int e = 0; e < nevals; ++e) {
-        if (graph[e] < 0 || graph[e] >= q->ngraphs || p[e] < 1 || p[e] > q->max_p) return (int)hipErrorInvalidValue;
         q->evals_h[e].graph = graph[e];
         q->evals_h[e].p = p[e];
         q->evals_h[e].angle_off = e * q->max_p;
@@ -469,13 +475,22 @@ int orkan_qaoa_get_config(const orkan_qaoa_t *q, int *lt, int *threads, int *gri
     return 0;
 }
 
+/* the configuration as it was before a search that found none */
+static void back_to(orkan_qaoa_t *q, int lt, int threads, int grid) {
+    drop_graph(q);
+    q->lt = lt;
+    q->threads = threads;
+    q->grid = grid;
+    (void)ensure_states(q, 1);
+}
+
 /* Autotuner: time every (tile, workgroup size) candidate the largest state
  * allows on the caller's evaluation list (one untimed launch, then the median
  * of `reps` launches), keep the fastest. */
 int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int *p, const double *gamma,
                         const double *beta, int reps, double *best_ms) {
     static const int cand[][2] = {{11, 256}, {11, 512}, {12, 256}, {12, 512}, {12, 1024}, {13, 512}, {13, 1024}};
-    if (!q) return (int)hipErrorInvalidValue;
+    if (!q || !list_ok(q, nevals, graph, p)) return (int)hipErrorInvalidValue;
     if (reps < 1) reps = 1;
     if (reps > 15) reps = 15;
     hipStream_t st = (hipStream_t)ork_dev()->stream;
@@ -487,10 +502,12 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
     }
     /* the whole search holds the library lock: staging, every reconfiguration and launch */
     ork_lock();
+    const int lt0 = q->lt, threads0 = q->threads, grid0 = q->grid;
     /* the register kernels' records number tiles of the scratch: it has its size for them first */
     if (2 * REG_LT >= q->nmax) (void)set_config(q, REG_LT, REG_THREADS, 0, 0);
     int e = stage(q, nevals, graph, p, gamma, beta, 1);
     if (e) {
+        back_to(q, lt0, threads0, grid0);
         ork_unlock();
         (void)hipEventDestroy(a);
         (void)hipEventDestroy(b);
@@ -523,6 +540,7 @@ int orkan_qaoa_autotune(orkan_qaoa_t *q, int nevals, const int *graph, const int
     (void)hipEventDestroy(a);
     (void)hipEventDestroy(b);
     if (best_i < 0) {
+        back_to(q, lt0, threads0, grid0);
         ork_unlock();
         return (int)hipErrorInvalidConfiguration;
     }

@@ -157,6 +157,27 @@ int main(int argc, char **argv) {
         g[0] = 0.0;
         CHECK(orkan_qaoa_eval(q, 64, graph, p, g, b, out) == 0 && rounds == 16);
         orkan_qaoa_destroy(q);
+    } else if (!strcmp(what, "qaoa_refused")) {
+        /* a search on a list that is refused leaves the configuration and the scratch as they were */
+        capacity = (size_t)8 << 30;
+        const unsigned char nq = 14;
+        double *diag = calloc(8, 1 << 14), g[2] = {0}, b[2] = {0}, out[1];
+        const double *d = diag;
+        int graph = 0, p = 3, lt, th, gr;
+        orkan_qaoa_t *q = orkan_qaoa_create(1, &nq, &d, 8, 2);
+        CHECK(q && orkan_qaoa_set_config(q, 11, 512, 1) == 0);
+        const size_t before = used;
+        CHECK(orkan_qaoa_autotune(q, 1, &graph, &p, g, b, 1, NULL) != 0);
+        CHECK(orkan_qaoa_get_config(q, &lt, &th, &gr) == 0 && lt == 11 && th == 512 && gr == 8 && used == before);
+        p = 2;
+        graph = 1;
+        CHECK(orkan_qaoa_autotune(q, 1, &graph, &p, g, b, 1, NULL) != 0);
+        CHECK(orkan_qaoa_autotune(q, 9, &graph, &p, g, b, 1, NULL) != 0);
+        CHECK(orkan_qaoa_eval(q, 1, &graph, &p, g, b, out) != 0);
+        CHECK(orkan_qaoa_get_config(q, &lt, &th, &gr) == 0 && lt == 11 && th == 512 && gr == 8 && used == before);
+        graph = 0;
+        CHECK(orkan_qaoa_autotune(q, 1, &graph, &p, g, b, 1, NULL) == 0);
+        orkan_qaoa_destroy(q);
     } else if (!strcmp(what, "count")) {
         /* many tiny states: each holds a page, whatever its length, and a bounded number of them is kept */
         static state_t t[6000];

@@ -62,3 +62,7 @@ def test_kept_storage_is_released_on_request(program):
 
 def test_batched_qaoa_scratch_is_that_of_the_configuration(program):
     run(program, "qaoa_scratch")
+
+
+def test_refused_search_changes_nothing(program):
+    run(program, "qaoa_refused")
