@@ -85,23 +85,14 @@ __global__ __launch_bounds__(GT) void gemm_nt_kernel(const bf16 *__restrict__ A,
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+            const long col = n0 + wn * 64 + j * 32 + l32;
+            const float bias = EPI == EPI_BIAS_GELU ? ep.bias[col] : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const long row = m0 + wm * 64 + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                const long col = n0 + wn * 64 + j * 32 + l32;
-                const long at = row * ep.ldc + col;
-                const float v = acc[i][j][r];
-                if constexpr (EPI == EPI_F32) ep.c32[at] = v;
-                else if constexpr (EPI == EPI_F32_ACC) ep.c32[at] += v;
-                else if constexpr (EPI == EPI_BIAS_GELU) {
-                    const float z = v + ep.bias[col];
-                    if (ep.pre) ep.pre[at] = z;
-                    ep.act[at] = (bf16)gelu(z);
-                } else {
-                    ep.act[at] = (bf16)(v * gelu_grad(ep.pre[at]));
-                }
-            }
+            for (int q = 0; q < 4; ++q)
+                epilogue4<EPI>(ep, m0 + wm * 64 + i * 32 + 8 * q + 4 * lhi, col, bias,
+                               {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]});
+        }
 }
 
 // ---- 256 x 256 tile variant: 8 waves of 128 x 64 (4 x 2 MFMA tiles each), K steps of 64 ------
@@ -182,23 +173,14 @@ __global__ __launch_bounds__(GT2) void gemm_nt_big_kernel(const bf16 *__restrict
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+            const long col = n0 + wn * 64 + j * 32 + l32;
+            const float bias = EPI == EPI_BIAS_GELU ? ep.bias[col] : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const long row = m0 + wm * 128 + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                const long col = n0 + wn * 64 + j * 32 + l32;
-                const long at = row * ep.ldc + col;
-                const float v = acc[i][j][r];
-                if constexpr (EPI == EPI_F32) ep.c32[at] = v;
-                else if constexpr (EPI == EPI_F32_ACC) ep.c32[at] += v;
-                else if constexpr (EPI == EPI_BIAS_GELU) {
-                    const float z = v + ep.bias[col];
-                    if (ep.pre) ep.pre[at] = z;
-                    ep.act[at] = (bf16)gelu(z);
-                } else {
-                    ep.act[at] = (bf16)(v * gelu_grad(ep.pre[at]));
-                }
-            }
+            for (int q = 0; q < 4; ++q)
+                epilogue4<EPI>(ep, m0 + wm * 128 + i * 32 + 8 * q + 4 * lhi, col, bias,
+                               {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]});
+        }
 }
 constexpr int BIG_LDS = 2 * (BM2 + BN2) * KP2 * (int)sizeof(bf16);
 
@@ -302,23 +284,14 @@ __global__ __launch_bounds__(GT3) void gemm_nt_dma_kernel(const bf16 *__restrict
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+            const long col = n0 + wn * 64 + j * 32 + l32;
+            const float bias = EPI == EPI_BIAS_GELU ? ep.bias[col] : 0.0f;
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const long row = m0 + wm * 128 + i * 32 + 8 * (r >> 2) + 4 * lhi + (r & 3);
-                const long col = n0 + wn * 64 + j * 32 + l32;
-                const long at = row * ep.ldc + col;
-                const float v = acc[i][j][r];
-                if constexpr (EPI == EPI_F32) ep.c32[at] = v;
-                else if constexpr (EPI == EPI_F32_ACC) ep.c32[at] += v;
-                else if constexpr (EPI == EPI_BIAS_GELU) {
-                    const float z = v + ep.bias[col];
-                    if (ep.pre) ep.pre[at] = z;
-                    ep.act[at] = (bf16)gelu(z);
-                } else {
-                    ep.act[at] = (bf16)(v * gelu_grad(ep.pre[at]));
-                }
-            }
+            for (int q = 0; q < 4; ++q)
+                epilogue4<EPI>(ep, m0 + wm * 128 + i * 32 + 8 * q + 4 * lhi, col, bias,
+                               {acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]});
+        }
 }
 
 
@@ -512,11 +485,12 @@ extern "C" int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, c
                                 int K, float *c32, int ldc, const float *bias, float *pre, void *act, void *actT,
                                 long ldt);
 
-// epi: 0 fp32 C, 1 bias+GELU, 2 GELU backward, 3 fp32 C +=
+// epi: 0 fp32 C, 1 bias+GELU, 2 GELU backward; actT: the bf16 result transposed as well ([N][ldt]), or null
 extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
-                            float *c32, int ldc, const float *bias, float *pre, void *act) {
-    if (M % BM || N % BN || K % BK || M <= 0 || N <= 0 || K <= 0) return (int)hipErrorInvalidValue;
-    EpiArgs ep{c32, ldc, bias, pre, (bf16 *)act};
+                            float *c32, int ldc, const float *bias, float *pre, void *act, void *actT, long ldt) {
+    if (M % BM || N % BN || K % BK || M <= 0 || N <= 0 || K <= 0 || ldt % 4 || ((uintptr_t)actT & 7))
+        return (int)hipErrorInvalidValue;
+    EpiArgs ep{c32, ldc, bias, pre, (bf16 *)act, (bf16 *)actT, ldt};
     hipStream_t st = (hipStream_t)stream;
     const bf16 *a = (const bf16 *)A, *b = (const bf16 *)B;
     // the DMA moves 16 B per lane: rows of both operands must start on 16 B boundaries
@@ -528,7 +502,6 @@ extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const
         case EPI_F32: gemm_nt_dma_kernel<EPI_F32><<<grid3, GT3, 0, st>>>(a, lda, b, ldb, K, ep); break;
         case EPI_BIAS_GELU: gemm_nt_dma_kernel<EPI_BIAS_GELU><<<grid3, GT3, 0, st>>>(a, lda, b, ldb, K, ep); break;
         case EPI_GELU_BWD: gemm_nt_dma_kernel<EPI_GELU_BWD><<<grid3, GT3, 0, st>>>(a, lda, b, ldb, K, ep); break;
-        case EPI_F32_ACC: gemm_nt_dma_kernel<EPI_F32_ACC><<<grid3, GT3, 0, st>>>(a, lda, b, ldb, K, ep); break;
         default: return (int)hipErrorInvalidValue;
         }
         ORK_LAUNCH_CHECK();
@@ -540,22 +513,24 @@ extern "C" int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const
         case EPI_F32: gemm_nt_big_kernel<EPI_F32><<<grid2, GT2, BIG_LDS, st>>>(a, lda, b, ldb, K, ep); break;
         case EPI_BIAS_GELU: gemm_nt_big_kernel<EPI_BIAS_GELU><<<grid2, GT2, BIG_LDS, st>>>(a, lda, b, ldb, K, ep); break;
         case EPI_GELU_BWD: gemm_nt_big_kernel<EPI_GELU_BWD><<<grid2, GT2, BIG_LDS, st>>>(a, lda, b, ldb, K, ep); break;
-        case EPI_F32_ACC: gemm_nt_big_kernel<EPI_F32_ACC><<<grid2, GT2, BIG_LDS, st>>>(a, lda, b, ldb, K, ep); break;
         default: return (int)hipErrorInvalidValue;
         }
         ORK_LAUNCH_CHECK();
         return 0;
     }
-    // Fewer 256 x 256 tiles than CUs: 128 x 64 tiles, four times the workgroups (4096 x 512 x 512 with its fused
-    // epilogue: 11 us against 28 on 32 workgroups of 256 x 256); also for shapes the large tile does not divide
-    if (g_gemm_big == 2 && aligned16 && epi != EPI_F32_ACC)
-        return ork_mlp_gemm_mid(stream, epi, A, lda, B, ldb, M, N, K, c32, ldc, bias, pre, act, nullptr, 0);
+    // Up to one 128 x 64 tile per CU: those, twice the workgroups of 128 x 128 and the operands by DMA.  A second round of
+    // them costs more than the better reuse of 128 x 128 saves.  Three forward layers from 128 to H, H and H wide with
+    // 128 x 64, 128 x 128 and (where it divides) 256 x 256 tiles, at `tiles` of 128 x 128:
+    //   H 512, tiles 128: 46 us, 64, 108    188: 66.7, 65.6, -    316: 87, 75, -    768: 149, 102, 123    2044: 357, 213, -
+    //   H 128, tiles 128: 46 us, 58, -    192: 61.2, 59.3, -    512: 104, 82, -
+    //   H 1024, tiles 128: 55 us, 79, 124    256: 81.9, 82.9, 126    1024: -, 172, 130    2040: 461, 275, -
+    if (g_gemm_big == 2 && aligned16 && (long)(M / BM) * (N / BN) <= 128)
+        return ork_mlp_gemm_mid(stream, epi, A, lda, B, ldb, M, N, K, c32, ldc, bias, pre, act, actT, ldt);
     dim3 grid(N / BN, M / BM);
     switch (epi) {
     case EPI_F32: gemm_nt_kernel<EPI_F32><<<grid, GT, 0, st>>>(a, lda, b, ldb, K, ep); break;
     case EPI_BIAS_GELU: gemm_nt_kernel<EPI_BIAS_GELU><<<grid, GT, 0, st>>>(a, lda, b, ldb, K, ep); break;
     case EPI_GELU_BWD: gemm_nt_kernel<EPI_GELU_BWD><<<grid, GT, 0, st>>>(a, lda, b, ldb, K, ep); break;
-    case EPI_F32_ACC: gemm_nt_kernel<EPI_F32_ACC><<<grid, GT, 0, st>>>(a, lda, b, ldb, K, ep); break;
     default: return (int)hipErrorInvalidValue;
     }
     ORK_LAUNCH_CHECK();

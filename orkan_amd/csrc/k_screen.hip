@@ -20,8 +20,6 @@
 // nothing (1.53-1.57 ms).
 #include "k_mlp.hpp"
 
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
 namespace {
 
 constexpr int SC_ROWS = 64, SC_THREADS = 256, SC_MAX = 3, SC_NA = 8;

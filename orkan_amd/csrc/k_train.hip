@@ -10,8 +10,6 @@
 // layer and operand had a launch of its own).
 #include "k_mlp.hpp"
 
-typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
-
 namespace {
 
 // ---- GEMM C[M x N] = A[M x K] B[N x K]^T on 128 x 64 tiles -----------------------------------------
@@ -28,26 +26,18 @@ typedef __attribute__((address_space(3))) void lds_void;
 
 __device__ __forceinline__ int swz8(int row, int chunk) { return chunk ^ (row & 7); }
 
-struct MidArgs {
-    EpiArgs ep;
-    bf16 *actT;   // act transposed, [N][ldt], or null
-    long ldt;
-    int ntn;      // N / 64
-};
-
 template <int EPI>
 __global__ __launch_bounds__(MT) void gemm_nt_mid_kernel(const bf16 *__restrict__ A, int lda,
-                                                         const bf16 *__restrict__ B, int ldb, int K, MidArgs ma) {
+                                                         const bf16 *__restrict__ B, int ldb, int K, EpiArgs ep, int ntn) {
     __shared__ __attribute__((aligned(16))) bf16 sa0[MM * MK], sa1[MM * MK], sa2[MM * MK], sa3[MM * MK];
     __shared__ __attribute__((aligned(16))) bf16 sb0[MN * MK], sb1[MN * MK], sb2[MN * MK], sb3[MN * MK];
-    const EpiArgs &ep = ma.ep;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave >> 1, wn = wave & 1;
     // workgroups go round-robin over the 8 XCDs: give each XCD a contiguous run of row panels with all their columns,
     // so that an A panel is fetched into one XCD's L2 only
     unsigned t = blockIdx.x;
     if ((gridDim.x & 7) == 0) t = (t & 7) * (gridDim.x >> 3) + (t >> 3);
-    const long m0 = (long)(t / (unsigned)ma.ntn) * MM, n0 = (long)(t % (unsigned)ma.ntn) * MN;
+    const long m0 = (long)(t / (unsigned)ntn) * MM, n0 = (long)(t % (unsigned)ntn) * MN;
     // DMA: one instruction fills 8 rows (64 lanes x 16 B); wave w fills A rows 32 w .. + 31 and B rows 16 w .. + 15.
     // Lane l lands in row l / 8 of the 8 at chunk position l % 8, which holds chunk (l % 8) ^ (row & 7).
     const int drow = lane >> 3, dchunk = swz8(drow, lane & 7);
@@ -119,35 +109,15 @@ __global__ __launch_bounds__(MT) void gemm_nt_mid_kernel(const bf16 *__restrict_
 #undef STEP
 #undef MMA
 #undef DMA
-    // lane holds C[row][col] with col = l32, row = 8 (r / 4) + 4 lhi + (r % 4): four consecutive rows per r / 4, one
-    // 8 B store of the transposed copy
+    // lane holds C[row][col] with col = l32, row = 8 (r / 4) + 4 lhi + (r % 4)
     const long col = n0 + wn * 32 + l32;
     const float bias = EPI == EPI_BIAS_GELU ? ep.bias[col] : 0.0f;
 #pragma unroll
     for (int i = 0; i < 2; ++i)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            const long row0 = m0 + wm * 64 + i * 32 + 8 * q + 4 * lhi;
-            bf16x4 o;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const long at = (row0 + j) * ep.ldc + col;
-                const float v = acc[i][4 * q + j];
-                if constexpr (EPI == EPI_F32) {
-                    ep.c32[at] = v;
-                } else if constexpr (EPI == EPI_BIAS_GELU) {
-                    const float z = v + bias;
-                    if (ep.pre) ep.pre[at] = z;
-                    o[j] = (bf16)gelu(z);
-                    ep.act[at] = o[j];
-                } else {
-                    o[j] = (bf16)(v * gelu_grad(ep.pre[at]));
-                    ep.act[at] = o[j];
-                }
-            }
-            if constexpr (EPI != EPI_F32)
-                if (ma.actT) *(bf16x4 *)(ma.actT + col * ma.ldt + row0) = o;
-        }
+        for (int q = 0; q < 4; ++q)
+            epilogue4<EPI>(ep, m0 + wm * 64 + i * 32 + 8 * q + 4 * lhi, col, bias,
+                           {acc[i][4 * q], acc[i][4 * q + 1], acc[i][4 * q + 2], acc[i][4 * q + 3]});
 }
 
 // ---- operand preparation ------------------------------------------------------------------------
@@ -463,15 +433,15 @@ extern "C" int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, c
     if (M % MM || N % MN || K % 32 || M <= 0 || N <= 0 || K <= 0 || lda % 8 || ldb % 8 || ((uintptr_t)A & 15) ||
         ((uintptr_t)B & 15) || ldt % 4)
         return (int)hipErrorInvalidValue;
-    MidArgs ma{EpiArgs{c32, ldc, bias, pre, (bf16 *)act}, (bf16 *)actT, ldt, N / MN};
+    const EpiArgs ep{c32, ldc, bias, pre, (bf16 *)act, (bf16 *)actT, ldt};
     const long tiles = (long)(M / MM) * (N / MN);
     if (tiles >= (1L << 31)) return (int)hipErrorInvalidValue;
     hipStream_t st = (hipStream_t)stream;
     const bf16 *a = (const bf16 *)A, *b = (const bf16 *)B;
     switch (epi) {
-    case EPI_F32: gemm_nt_mid_kernel<EPI_F32><<<(unsigned)tiles, MT, 0, st>>>(a, lda, b, ldb, K, ma); break;
-    case EPI_BIAS_GELU: gemm_nt_mid_kernel<EPI_BIAS_GELU><<<(unsigned)tiles, MT, 0, st>>>(a, lda, b, ldb, K, ma); break;
-    case EPI_GELU_BWD: gemm_nt_mid_kernel<EPI_GELU_BWD><<<(unsigned)tiles, MT, 0, st>>>(a, lda, b, ldb, K, ma); break;
+    case EPI_F32: gemm_nt_mid_kernel<EPI_F32><<<(unsigned)tiles, MT, 0, st>>>(a, lda, b, ldb, K, ep, N / MN); break;
+    case EPI_BIAS_GELU: gemm_nt_mid_kernel<EPI_BIAS_GELU><<<(unsigned)tiles, MT, 0, st>>>(a, lda, b, ldb, K, ep, N / MN); break;
+    case EPI_GELU_BWD: gemm_nt_mid_kernel<EPI_GELU_BWD><<<(unsigned)tiles, MT, 0, st>>>(a, lda, b, ldb, K, ep, N / MN); break;
     default: return (int)hipErrorInvalidValue;
     }
     ORK_LAUNCH_CHECK();

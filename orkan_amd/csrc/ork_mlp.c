@@ -15,9 +15,7 @@
 #include <hip/hip_runtime_api.h>
 
 int ork_mlp_gemm(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
-                 float *c32, int ldc, const float *bias, float *pre, void *act);
-int ork_mlp_gemm_mid(void *stream, int epi, const void *A, int lda, const void *B, int ldb, int M, int N, int K,
-                     float *c32, int ldc, const float *bias, float *pre, void *act, void *actT, long ldt);
+                 float *c32, int ldc, const float *bias, float *pre, void *act, void *actT, long ldt);
 int ork_mlp_stage_input(void *stream, const float *x, int m0, int m1, int rows, int K, void *x16, void *x16t, long ldt,
                         const float *tgt_src, float *tgt);
 int ork_mlp_pack(void *stream, int count, const float *const *src, const int *len, float *dst);
@@ -265,10 +263,10 @@ static int forward_rows(orkan_mlp_t *q, int Mp, int training) {
         layer_t *L = &q->L[l];
         int e;
         if (training)
-            e = ork_mlp_gemm_mid(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, q->pre[l], q->act[l],
+            e = ork_mlp_gemm(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, q->pre[l], q->act[l],
                                  l + 1 < q->nl ? q->in_t[l + 1] : NULL, (long)Mp + TPAD);
         else
-            e = ork_mlp_gemm(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, NULL, q->act[l]);
+            e = ork_mlp_gemm(st, 1, in, ld, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, NULL, q->act[l], NULL, 0);
         if (e) return e;
         in = q->act[l];
         ld = L->N;
@@ -369,7 +367,7 @@ int orkan_mlp_forward_candidates(orkan_mlp_t *q, const float *gf_host, int ng, c
         const void *in = q->act[0];
         for (int l = 1; l < q->nl && !e; ++l) {
             layer_t *L = &q->L[l];
-            e = ork_mlp_gemm(st, 1, in, L->K, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, NULL, q->act[l]);
+            e = ork_mlp_gemm(st, 1, in, L->K, L->wtb, L->K, Mp, L->N, L->K, NULL, L->N, L->b, NULL, q->act[l], NULL, 0);
             in = q->act[l];
         }
         if (!e) e = ork_mlp_head_forward(st, q->act[q->nl - 1], q->w_out, q->b_out, Mp, H, y_dev + r0, NULL, NULL,
@@ -394,7 +392,7 @@ static int backward(orkan_mlp_t *q, int rows) {
     /* dP_{l-1} = (dP_l W_l^T) * gelu'(pre_{l-1}) */
     for (int l = nl - 1; l > 0 && !e; --l) {
         layer_t *L = &q->L[l];
-        e = ork_mlp_gemm_mid(st, 2, q->dpre[l], L->N, L->wb, L->N, Mp, L->K, L->N, NULL, L->K, NULL, q->pre[l - 1],
+        e = ork_mlp_gemm(st, 2, q->dpre[l], L->N, L->wb, L->N, Mp, L->K, L->N, NULL, L->K, NULL, q->pre[l - 1],
                              q->dpre[l - 1], q->dpre_t[l - 1], ldt);
     }
     const void *xt[MLP_MAX_LAYERS], *dt[MLP_MAX_LAYERS], *cols[MLP_MAX_LAYERS + 1];
@@ -506,7 +504,7 @@ int orkan_topk_f32(const float *y_dev, long n, int k, int *idx_host, float *val_
 /* C = A B^T for bf16 A [M][K], B [N][K] (device pointers), fp32 C [M][N]: exposed for testing the MFMA GEMM */
 int orkan_mlp_gemm_test(int M, int N, int K, const void *A, const void *B, float *C) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
-    int e = ork_mlp_gemm(st, 0, A, K, B, K, M, N, K, C, N, NULL, NULL, NULL);
+    int e = ork_mlp_gemm(st, 0, A, K, B, K, M, N, K, C, N, NULL, NULL, NULL, NULL, 0);
     if (!e) e = (int)hipStreamSynchronize(st);
     return e;
 }
