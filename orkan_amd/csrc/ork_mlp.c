@@ -62,9 +62,12 @@ struct orkan_mlp {
     void *x16;                  /* bf16 [M][in_dim] */
     float *pre[MLP_MAX_LAYERS]; /* fp32 [M][hidden] */
     void *act[MLP_MAX_LAYERS];  /* bf16 [M][hidden] */
-    void *dpre[MLP_MAX_LAYERS]; /* bf16 [M][hidden] */
-    /* transposed operands of the weight gradients: the layers' inputs and dpre, bf16 [width][M + TPAD] */
-    void *in_t[MLP_MAX_LAYERS], *dpre_t[MLP_MAX_LAYERS];
+    /* transposed operands of the weight gradients: the layers' inputs, bf16 [width][M + TPAD] */
+    void *in_t[MLP_MAX_LAYERS];
+    /* gradients of the pre-activations, bf16 [M][hidden], and their transposes [hidden][M + TPAD].  The last layer's have
+     * memory of their own; an earlier layer's take the place of what the backward pass no longer reads by then: its
+     * activations, and the pre-activations of the layer after it */
+    void *dpre[MLP_MAX_LAYERS], *dpre_t[MLP_MAX_LAYERS];
     float *y, *dy, *sq, *tgt;
     float *scal;                /* sum of squared errors, d loss / d b_out; pinned */
     float *host;                /* the pinned buffer, while a batch staged in it is on its way */
@@ -113,9 +116,10 @@ orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch
         q->act[l] = dmalloc(M * H * 2, &err);
     }
     for (int l = 0; l < nhidden; ++l) {
-        q->dpre[l] = dmalloc(M * H * 2, &err);
+        const int last = l == nhidden - 1;
         q->in_t[l] = dmalloc((M + TPAD) * (size_t)q->L[l].K * 2, &err);
-        q->dpre_t[l] = dmalloc((M + TPAD) * H * 2, &err);
+        q->dpre[l] = last ? dmalloc(M * H * 2, &err) : q->act[l];
+        q->dpre_t[l] = last ? dmalloc((M + TPAD) * H * 2, &err) : (void *)q->pre[l + 1];   /* M >= TILE > TPAD */
     }
     q->w_out = dmalloc(H * 4, &err); q->g_out = dmalloc(H * 4, &err);
     q->m_out = dmalloc(H * 4, &err); q->v_out = dmalloc(H * 4, &err);
@@ -152,8 +156,9 @@ void orkan_mlp_destroy(orkan_mlp_t *q) {
     (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
     for (int l = 0; l < MLP_MAX_LAYERS; ++l) {
         layer_t *L = &q->L[l];
+        const int last = l == q->nl - 1;
         void *p[] = {L->w, L->g, L->m, L->v, L->b, L->gb, L->mb, L->vb, L->wb, L->wtb, q->pre[l], q->act[l],
-                     q->dpre[l], q->in_t[l], q->dpre_t[l]};
+                     q->in_t[l], last ? q->dpre[l] : NULL, last ? q->dpre_t[l] : NULL};
         for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
             if (p[i]) (void)hipFree(p[i]);
     }

@@ -66,3 +66,8 @@ def test_batched_qaoa_scratch_is_that_of_the_configuration(program):
 
 def test_refused_search_changes_nothing(program):
     run(program, "qaoa_refused")
+
+
+def test_network_holds_each_gradient_once(program):
+    """Gradients of the pre-activations take the place of activations that the backward pass is done with."""
+    run(program, "mlp_size")
