@@ -62,12 +62,13 @@ struct orkan_mlp {
     void *x16;                  /* bf16 [M][in_dim] */
     float *pre[MLP_MAX_LAYERS]; /* fp32 [M][hidden] */
     void *act[MLP_MAX_LAYERS];  /* bf16 [M][hidden] */
-    /* transposed operands of the weight gradients: the layers' inputs, bf16 [width][M + TPAD] */
-    void *in_t[MLP_MAX_LAYERS];
-    /* gradients of the pre-activations, bf16 [M][hidden], and their transposes [hidden][M + TPAD].  The last layer's have
-     * memory of their own; an earlier layer's take the place of what the backward pass no longer reads by then: its
-     * activations, and the pre-activations of the layer after it */
-    void *dpre[MLP_MAX_LAYERS], *dpre_t[MLP_MAX_LAYERS];
+    /* gradients of the pre-activations, bf16 [M][hidden]: the last layer's in memory of their own, an earlier layer's in
+     * place of its activations, which the backward pass does not read.  (Their transposes could take the place of the
+     * pre-activations of the layer after: that made each backward product 1 us slower, 13.4 -> 14.5 at 4096 x 512.) */
+    void *dpre[MLP_MAX_LAYERS];
+    /* transposed operands of the weight gradients: the layers' inputs and dpre, bf16 [width][M + TPAD], in one allocation
+     * (one each took 100 us and more: the padding puts them past a 2 MB page) */
+    void *in_t[MLP_MAX_LAYERS], *dpre_t[MLP_MAX_LAYERS], *transposes;
     float *y, *dy, *sq, *tgt;
     float *scal;                /* sum of squared errors, d loss / d b_out; pinned */
     float *host;                /* the pinned buffer, while a batch staged in it is on its way */
@@ -115,11 +116,13 @@ orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch
         q->pre[l] = dmalloc(M * H * 4, &err);
         q->act[l] = dmalloc(M * H * 2, &err);
     }
-    for (int l = 0; l < nhidden; ++l) {
-        const int last = l == nhidden - 1;
-        q->in_t[l] = dmalloc((M + TPAD) * (size_t)q->L[l].K * 2, &err);
-        q->dpre[l] = last ? dmalloc(M * H * 2, &err) : q->act[l];
-        q->dpre_t[l] = last ? dmalloc((M + TPAD) * H * 2, &err) : (void *)q->pre[l + 1];   /* M >= TILE > TPAD */
+    const size_t column = (M + TPAD) * 2;
+    char *t = q->transposes = dmalloc(column * ((size_t)in_dim + (2 * (size_t)nhidden - 1) * H), &err);
+    for (int l = 0; l < nhidden && t; ++l) {
+        q->in_t[l] = t;
+        q->dpre_t[l] = t += column * (size_t)q->L[l].K;
+        t += column * H;
+        q->dpre[l] = l == nhidden - 1 ? dmalloc(M * H * 2, &err) : q->act[l];
     }
     q->w_out = dmalloc(H * 4, &err); q->g_out = dmalloc(H * 4, &err);
     q->m_out = dmalloc(H * 4, &err); q->v_out = dmalloc(H * 4, &err);
@@ -156,14 +159,13 @@ void orkan_mlp_destroy(orkan_mlp_t *q) {
     (void)hipStreamSynchronize((hipStream_t)ork_dev()->stream);
     for (int l = 0; l < MLP_MAX_LAYERS; ++l) {
         layer_t *L = &q->L[l];
-        const int last = l == q->nl - 1;
         void *p[] = {L->w, L->g, L->m, L->v, L->b, L->gb, L->mb, L->vb, L->wb, L->wtb, q->pre[l], q->act[l],
-                     q->in_t[l], last ? q->dpre[l] : NULL, last ? q->dpre_t[l] : NULL};
+                     l == q->nl - 1 ? q->dpre[l] : NULL};
         for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
             if (p[i]) (void)hipFree(p[i]);
     }
     void *p[] = {q->w_out, q->g_out, q->m_out, q->v_out, q->x32, q->x16, q->y, q->dy, q->sq, q->tgt,
-                 q->colpart, q->gf_dev, q->u1, q->wpk};
+                 q->colpart, q->gf_dev, q->u1, q->wpk, q->transposes};
     for (size_t i = 0; i < sizeof(p) / sizeof(p[0]); ++i)
         if (p[i]) (void)hipFree(p[i]);
     if (q->scal) (void)hipHostFree(q->scal);

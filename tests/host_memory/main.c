@@ -126,11 +126,11 @@ int main(int argc, char **argv) {
         CHECK(orkan_mlp_create(128, 128, 3, 8192));
     } else if (!strcmp(what, "mlp_size")) {
         /* three layers of 128, 8192 rows: per row and column 12 B of pre-activations, 6 of activations, 6 of transposed
-         * inputs, 4 of gradients with their transpose; 6 B per input; the parameters */
+         * inputs, 2 of gradients and 6 of their transposes; 6 B per input; the parameters */
         orkan_mem_trim(0);
         const size_t before = used, mh = (size_t)8192 * 128;
         CHECK(orkan_mlp_create(128, 128, 3, 8192));
-        CHECK(used - before <= 28 * mh + 6 * mh + 2 * MB);
+        CHECK(used - before <= 32 * mh + 6 * mh + 2 * MB);
     } else if (!strcmp(what, "qaoa")) {
         /* one 20-qubit graph: 8 MB of diagonal, 16 MB of state, and the whole scratch, not half of it */
         const unsigned char nq = 20;
