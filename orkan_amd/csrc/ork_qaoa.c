@@ -23,7 +23,7 @@ int ork_qaoa_sweeps(void *stream, int sym, int deep, const void *recs, const int
                     const double *diag, void *states, double *part, double *out);
 int ork_qaoa_stage(void *stream, const double *gb, uint64_t rows, double *angles, const void *recs, int nrecs, void *recs_dst);
 int ork_qaoa_rescale(void *stream, const void *recs_dev, int count, double *angles);
-int ork_qaoa_diag_info(void *stream, int ngraphs, const void *graphs, const double *diag, double *info);
+int ork_qaoa_diag_info(void *stream, int ngraphs, int nmax, const void *graphs, const double *diag, uint64_t *info);
 int ork_maxcut_diag(void *stream, double *out, int n, int ne, const int *ei, const int *ej, const double *w);
 
 typedef struct { int graph, p, angle_off, pad; } q_eval_t;
@@ -49,7 +49,7 @@ struct orkan_qaoa {
     int nevals_h;          /* host source of the nevals_d upload */
     double *info_h;        /* per graph: largest |C|; 1 if C(x) = C(~x) for every x, else 0 */
     /* the register kernels' list: records sorted by form, then index bits, then layers, all descending; n_h: index bits */
-    q_rec_t *recs_h;       /* pinned */
+    q_rec_t *recs_h;
     void *recs_d;
     int *n_h, *p_h, *start_h, nstaged;
     unsigned char *sym_h;
@@ -63,7 +63,8 @@ struct orkan_qaoa {
     /* host staging */
     q_eval_t *evals_h;
     int *order_h;
-    double *gb_h, *out_h;  /* pinned: rows of gamma, then of beta; the results */
+    double *gb_h, *out_h;  /* rows of gamma, then of beta; the results */
+    void *pinned;          /* gb_h, out_h and recs_h: each allocation and release of pinned memory takes 30 us and more */
 };
 
 static int cus(void) {
@@ -233,22 +234,30 @@ orkan_qaoa_t *orkan_qaoa_create(int ngraphs, const unsigned char *nq, const doub
     if (ork_dev_malloc((void **)&q->order_d, (size_t)max_evals * sizeof(int)) != 0) goto fail;
     if (ork_dev_malloc((void **)&q->nevals_d, sizeof(int)) != 0) goto fail;
     if (ork_dev_malloc((void **)&q->angles_d, (size_t)max_evals * max_p * 4 * sizeof(double)) != 0) goto fail;
-    if (hipHostMalloc((void **)&q->gb_h, (size_t)max_evals * max_p * 2 * sizeof(double), hipHostMallocDefault) !=
-            hipSuccess ||
-        hipHostMalloc((void **)&q->recs_h, (size_t)max_evals * sizeof(q_rec_t), hipHostMallocDefault) != hipSuccess ||
-        hipHostMalloc((void **)&q->out_h, (size_t)max_evals * sizeof(double), hipHostMallocDefault) != hipSuccess)
-        goto fail;
+    {
+        const size_t rows = (size_t)max_evals * max_p * 2, info = (size_t)ngraphs * 2;
+        const size_t bytes = (rows + max_evals) * sizeof(double) + (size_t)max_evals * sizeof(q_rec_t);
+        if (hipHostMalloc(&q->pinned, bytes > info * sizeof(uint64_t) ? bytes : info * sizeof(uint64_t),
+                          hipHostMallocDefault) != hipSuccess)
+            goto fail;
+        q->gb_h = q->pinned;
+        q->out_h = q->gb_h + rows;
+        q->recs_h = (q_rec_t *)(q->out_h + max_evals);
+    }
     if (ork_dev_malloc((void **)&q->counter_d, sizeof(unsigned)) != 0) goto fail;
     {
-        double *info = ork_mem_get((size_t)ngraphs * 2 * sizeof(double));
-        const int bad = !info || ork_qaoa_diag_info(st, ngraphs, q->graphs_d, q->diag_d, info) ||
-                        hipMemcpyAsync(q->info_h, info, (size_t)ngraphs * 2 * sizeof(double), hipMemcpyDeviceToHost, st) !=
-                            hipSuccess;
-        if (hipStreamSynchronize(st) != hipSuccess || bad) {
-            ork_mem_put(info);
-            goto fail;
-        }
+        const size_t bytes = (size_t)ngraphs * 2 * sizeof(uint64_t);
+        uint64_t *info = ork_mem_get(bytes), *host = q->pinned;
+        const int bad = !info || hipMemsetAsync(info, 0, bytes, st) != hipSuccess ||
+                        ork_qaoa_diag_info(st, ngraphs, q->nmax, q->graphs_d, q->diag_d, info) ||
+                        hipMemcpyAsync(host, info, bytes, hipMemcpyDeviceToHost, st) != hipSuccess;
+        const int waited = hipStreamSynchronize(st) == hipSuccess;
         ork_mem_put(info);
+        if (bad || !waited) goto fail;
+        for (int g = 0; g < ngraphs; ++g) {
+            memcpy(&q->info_h[2 * g], &host[2 * g], sizeof(double));
+            q->info_h[2 * g + 1] = host[2 * g + 1] == 0;
+        }
     }
     {
         /* default: 4096 amplitudes in the registers of 256 threads; 8192 in LDS when the largest state needs it */
@@ -273,9 +282,7 @@ void orkan_qaoa_destroy(orkan_qaoa_t *q) {
                     q->angles_d, q->counter_d, q->states_d, q->recs_d};
     for (size_t i = 0; i < sizeof(bufs) / sizeof(bufs[0]); ++i)
         if (bufs[i]) (void)hipFree(bufs[i]);
-    void *pinned[] = {q->gb_h, q->recs_h, q->out_h};
-    for (size_t i = 0; i < sizeof(pinned) / sizeof(pinned[0]); ++i)
-        if (pinned[i]) (void)hipHostFree(pinned[i]);
+    if (q->pinned) (void)hipHostFree(q->pinned);
     free(q->graphs_h);
     free(q->evals_h);
     free(q->order_h);
