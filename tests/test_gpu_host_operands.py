@@ -47,3 +47,32 @@ def test_superoperator_written_by_the_stream(n):
         e.free(st)
     dev.api.orkan_dev_free(src)
     assert hip.hipHostFree(pin) == 0
+
+
+@pytest.mark.parametrize("nonzero", [0, 1, 127, 128, 129, 255, 256])
+def test_superoperators_of_every_density(nonzero):
+    """Host superoperators travel by their nonzero entries, 128 to a launch: counts at and beside that, with a zero of
+    either sign among them.  1e-12 per stored entry, as in every parity test."""
+    dev, orc = engines.DeviceEngine(orkan_amd.lib_path(5), 5), engines.oracle(5)
+    rng = np.random.default_rng(nonzero)
+    # maps of Hermitian matrices to Hermitian ones: S[ij,kl] = conj(S[ji,lk]); entries of i = j, k = l are their own partners
+    i, j, k, l = np.unravel_index(rng.permutation(256), (4, 4, 4, 4))
+    at, partner = (i * 4 + j) * 16 + k * 4 + l, (j * 4 + i) * 16 + l * 4 + k
+    S = np.full(256, -0.0 if nonzero == 129 else 0.0, np.complex128)
+    singles, pairs = at[at == partner], [(a, b) for a, b in zip(at, partner) if a < b]
+    own = nonzero % 2 if nonzero <= 240 else nonzero - 240
+    S[singles[:own]] = rng.standard_normal(own) / 16
+    for a, b in pairs[:(nonzero - own) // 2]:
+        S[a] = (rng.standard_normal() + 1j * rng.standard_normal()) / 16
+        S[b] = np.conj(S[a])
+    assert np.count_nonzero(S) == nonzero
+    full = np.full(256, 0.25 + 0.0j)
+    for n in (2, 5):
+        data = to_layout(random_rho(n, rng), MIXED_TILED, 5)
+        sd, so = dev.new(MIXED_TILED, n, data), orc.new(MIXED_TILED, n, data)
+        for T in (full, S):      # the entries of an earlier one must not stay
+            dev.channel2(sd, T, 0, n - 1)
+            orc.channel2(so, T, 0, n - 1)
+        assert np.abs(dev.read(sd) - orc.read(so)).max() <= 1e-12
+        dev.free(sd)
+        orc.free(so)
