@@ -379,7 +379,7 @@ __global__ __launch_bounds__(256) void colsums_finish_kernel(ColsumArgs c) {
 constexpr int ADAM_MAX = 2 * DW_MAX + 1;
 struct AdamArgs {
     float *w[ADAM_MAX], *m[ADAM_MAX], *v[ADAM_MAX];
-    const float *g[ADAM_MAX];      // null: zero gradients
+    const float *g[ADAM_MAX];      // null: no step, only the bf16 copies, and the moments cleared
     bf16 *wb[ADAM_MAX], *wtb[ADAM_MAX];
     int rows[ADAM_MAX], cols[ADAM_MAX], first[ADAM_MAX + 1];
     int count;
@@ -400,14 +400,17 @@ __global__ __launch_bounds__(256) void adam_all_kernel(AdamArgs a) {
         const int r = matrix ? e >> 5 : 0, c = matrix ? e & 31 : e;
         if (!matrix && c0 + c >= N) continue;
         const long at = (long)(r0 + r) * N + c0 + c;
-        const float gi = a.g[i] ? a.g[i][at] : 0.0f;
-        // products fused explicitly, so that the rounding does not depend on what the compiler contracts
-        const float mi = fmaf(1.0f - a.b1, gi, a.b1 * a.m[i][at]);
-        const float vi = fmaf(gi, (1.0f - a.b2) * gi, a.b2 * a.v[i][at]);
+        float mi = 0.0f, vi = 0.0f, wi = a.w[i][at];
+        if (a.g[i]) {
+            const float gi = a.g[i][at];
+            // products fused explicitly, so that the rounding does not depend on what the compiler contracts
+            mi = fmaf(1.0f - a.b1, gi, a.b1 * a.m[i][at]);
+            vi = fmaf(gi, (1.0f - a.b2) * gi, a.b2 * a.v[i][at]);
+            wi -= a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
+            a.w[i][at] = wi;
+        }
         a.m[i][at] = mi;
         a.v[i][at] = vi;
-        const float wi = a.w[i][at] - a.lr * (mi / a.c1) / (sqrtf(vi / a.c2) + a.eps);
-        a.w[i][at] = wi;
         if (matrix) {
             a.wb[i][at] = (bf16)wi;
             tile[c][r] = (bf16)wi;
@@ -543,7 +546,7 @@ extern "C" int ork_mlp_colsums(void *stream, int count, const void *const *a, co
 }
 
 // one Adam step on `count` arrays of rows[i] x cols[i]; with wb and wtb (rows and cols multiples of 32) the bf16 copies
-// are written, else the array is a vector (rows 1); g[i] null: zero gradients
+// are written, else the array is a vector (rows 1); g[i] null: the copies only, and the moments cleared
 extern "C" int ork_mlp_adam_all(void *stream, int count, float *const *w, const float *const *g, float *const *m,
                                 float *const *v, void *const *wb, void *const *wtb, const int *rows, const int *cols,
                                 float lr, float b1, float b2, float eps, float c1, float c2) {

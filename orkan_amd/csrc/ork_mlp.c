@@ -172,7 +172,8 @@ void orkan_mlp_destroy(orkan_mlp_t *q) {
     free(q);
 }
 
-/* one Adam launch over the weight matrices (without `all`: zero gradients) and, with `all`, every bias and the head */
+/* one Adam launch: with `all` a step of every weight matrix, bias and the head, without it the bf16 copies of the weight
+ * matrices rewritten and their moments cleared */
 static int adam(orkan_mlp_t *q, int all, float lr, float b1, float b2, float eps, float c1, float c2) {
     float *w[2 * MLP_MAX_LAYERS + 1], *m[2 * MLP_MAX_LAYERS + 1], *v[2 * MLP_MAX_LAYERS + 1];
     const float *g[2 * MLP_MAX_LAYERS + 1];
@@ -204,7 +205,6 @@ int orkan_mlp_set_weights(orkan_mlp_t *q, const float *const *W, const float *co
         e |= (int)hipMemcpyAsync(L->w, W[l], (size_t)L->K * L->N * 4, hipMemcpyHostToDevice, st);
         e |= (int)hipMemcpyAsync(L->b, b[l], (size_t)L->N * 4, hipMemcpyHostToDevice, st);
     }
-    /* a step of zero gradients and lr = 0 only rewrites the bf16 copies (and clears the matrices' moments) */
     if (!e) e = adam(q, 0, 0.0f, 0.0f, 0.0f, 1.0f, 1.0f, 1.0f);
     if (!e) e = (int)hipMemcpyAsync(q->w_out, w_out, (size_t)q->hidden * 4, hipMemcpyHostToDevice, st);
     q->b_out = b_out;

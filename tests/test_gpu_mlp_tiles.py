@@ -88,3 +88,19 @@ def test_screening_in_one_kernel_and_layer_by_layer(hidden, layers, ncand):
         lib.orkan_dev_free(dy)
     assert np.array_equal(out[0], out[1])
     m.close()
+
+
+def test_weights_set_after_a_diverged_step():
+    """set_weights stores what it is given, also where a batch has left the weights and Adam's moments without values."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(3)
+    m, (W, b, wo, bo) = _net(lib, rng, 128, 2, 128)
+    x = rng.standard_normal((100, 128)).astype(np.float32)
+    y = m.forward(x)
+    m.train_step(np.full((100, 128), np.nan, np.float32), np.zeros(100, np.float32), 1e-3)
+    assert np.isnan(m.get_weights()[0][0]).all()
+    m.set_weights(W, b, wo, bo)
+    got = m.get_weights()
+    assert all(np.array_equal(a, c) for a, c in zip(got[0] + got[1], W + b)) and np.array_equal(got[2], wo)
+    assert np.array_equal(m.forward(x), y)
+    m.close()
