@@ -206,6 +206,7 @@ int orkan_maxcut_diag_dev(int n, int nedges, const int *ei, const int *ej, const
  * ---------------------------------------------------------------------------------------------- */
 typedef struct orkan_mlp orkan_mlp_t;
 
+/* device memory, training included: 10 B per hidden layer, column and row of max_batch, 8 B per input and row, 20 B per weight */
 orkan_mlp_t *orkan_mlp_create(int in_dim, int hidden, int nhidden, int max_batch);
 void orkan_mlp_destroy(orkan_mlp_t *m);
 /* W[l]: fp32 [K_l][hidden] row-major (K_0 = in_dim, else hidden); b[l]: [hidden]; w_out: [hidden] */

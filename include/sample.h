@@ -27,7 +27,10 @@ typedef struct {
  * K_{lstar-1} ... K_1 |iota>; pass a copy to keep it).  obs: 2^n doubles (host or device).
  * workspace_bytes caps the state vectors the call holds besides iota: 2B leaves (B = the leaf block,
  * at most 64; B where it holds every leaf) and, for the linear combinations, two vectors or as many
- * pairs, at most B, as the rest of the cap allows: at least 4 x 16 x 2^n bytes.
+ * pairs, at most B, as the rest of the cap allows: at least 4 x 16 x 2^n bytes.  Beside the cap the call holds obs and the
+ * product's partial sums, 16 B^2 bytes for every 16 amplitudes, at most 64 MiB.
+ * The operations are called as often and in the order that the blocks call for: a channel's operation on several leaves
+ * before its next operation, leaves of earlier blocks again.  They have to act the same way in every call.
  * Both triangles are filled, S_ba = conj(S_ab) exactly, the diagonal is real.  The result does not
  * depend on the block size.  Returns QS_OK, QS_ERR_NULL, QS_ERR_TYPE (iota not PURE complex128),
  * QS_ERR_PARAM (lstar out of range, a channel without operations or, other than at lstar, without

@@ -15,8 +15,8 @@
 //
 // Measured on 1,000,003 candidates, 128 -> 512 -> 512 -> 512 -> 1: 1.53 ms, 690 TFLOP/s, against 3.1 ms layer by layer
 // (GEMMs 74 us per 65536 rows and layer, layer 1 45 us, head 13 us).  Bound by the matrix work and the GELUs together:
-// with the GELUs left out the kernel takes 1.13 ms, with the weight loads left out as well 0.95; 192 GELUs per candidate
-// and wave lane add up to 1 ms of vector issue.  Wave priorities and a staggered start of a CU's two workgroups changed
+// with the GELUs left out the kernel takes 1.13 ms, with the weight loads left out as well 0.95; 1536 GELUs per candidate,
+// 6 per thread of the workgroup, add up to 1 ms of vector issue.  Wave priorities and a staggered start of a CU's two workgroups changed
 // nothing (1.53-1.57 ms).
 #include "k_mlp.hpp"
 

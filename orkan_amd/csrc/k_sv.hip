@@ -762,8 +762,8 @@ __global__ __launch_bounds__(THREADS) void sv_layer_kernel(S *__restrict__ psi, 
 
 // The same sweep with the tile of 2^12 amplitudes in registers (k_tile.hpp).  PASS 0: the contiguous tile,
 // qubits 0-11 in three layouts; PASS 1: a run of 2^r amplitudes, 4 <= r < 8, matrices on tile bits r..11 in two layouts;
-// PASS 2: r >= 8, one layout, no LDS.  The qubits above 11 go in equal shares, so the runs are 0.5 to 4 KB and each thread
-// has 16 loads in flight in four workgroups per CU; the LDS kernel moves 256 B runs, its last sweep a tile of as few as 32
+// PASS 2: r >= 8, one layout, no LDS.  The qubits above 11 go in equal shares, so the runs are 4 KB (21 qubits) to 256 B (27
+// and 28 qubits, shares of 8; 128 B in complex64) and each thread has 16 loads in flight in four workgroups per CU; the LDS kernel moves 256 B runs, its last sweep a tile of as few as 32
 // amplitudes per workgroup, and every three qubits go through LDS.  Bound by memory: n = 25 (512 MB) 566 us, three sweeps
 // at 5.7 TB/s, against 857; n = 21 43 against 210, n = 23 158 against 391, n = 28 4.78 ms against 4.85 (complex64: 364
 // against 711, 48 / 220, 101 / 381, 3.28 / 3.97).  Below 2^21 amplitudes a launch is one round of workgroups and waits on

@@ -19,7 +19,8 @@
  *   mixed, h / hy / rx / ry / single_from_mat: tile-group kernel with the
  *                gate's 4x4 superoperator; its entries are the coefficients of
  *                the reference's closed forms (src/gate/packed/gate_packed_1q.c:205-594)
- *   two_from_mat: tile-group kernel, dense 4x4 U rho U^dagger
+ *   two_from_mat: dense 4x4 U rho U^dagger on groups of 32 x 32 entries, four waves
+ *                each; the tile-group kernel where groups are smaller (below 5 qubits)
  */
 #include "ork_host.h"
 #include "orkan_backend.h"

@@ -385,8 +385,9 @@ int orkan_mlp_forward_candidates(orkan_mlp_t *q, const float *gf_host, int ng, c
 }
 
 /* gradients of the mean squared error of the staged batch into the g buffers; the sum of squared errors and
- * d loss / d b_out into scal[0] and scal[1].  12 launches (one step of 4096 rows of a 128 -> 512 -> 512 -> 512 -> 1
- * network, host batches and every fourth step's weights included: 234 us against 545 with a launch per layer and operand, 37 in all) */
+ * d loss / d b_out into scal[0] and scal[1].  Ten launches for three layers, besides the batch's and Adam's (4096 rows of a
+ * 128 -> 512 -> 512 -> 512 -> 1 network: 190 us a step from a host batch, 125 from a device one; four host steps and a
+ * read of the weights 895 us, 2190 with a launch per layer and operand, 37 a step) */
 static int backward(orkan_mlp_t *q, int rows) {
     hipStream_t st = (hipStream_t)ork_dev()->stream;
     const int Mp = pad_rows(rows), H = q->hidden, nl = q->nl;
