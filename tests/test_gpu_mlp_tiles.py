@@ -104,3 +104,22 @@ def test_weights_set_after_a_diverged_step():
     assert all(np.array_equal(a, c) for a, c in zip(got[0] + got[1], W + b)) and np.array_equal(got[2], wo)
     assert np.array_equal(m.forward(x), y)
     m.close()
+
+
+@pytest.mark.parametrize("n,k", [(40, 31), (40, 33), (300, 65), (70000, 65536)])
+def test_topk_order(n, k):
+    """Beside the sorting runs of 32, and the largest k: values descending, ties by index, zeros of either sign alike."""
+    lib = orkan_amd.load(5)
+    rng = np.random.default_rng(k)
+    y = rng.integers(-50, 50, n).astype(np.float32) / 8
+    y[rng.integers(0, n, n // 10)] = -0.0
+    y[: n // 3] += rng.standard_normal(n // 3).astype(np.float32)
+    dev = lib.orkan_dev_alloc((n + 1) // 2)
+    assert lib.orkan_copy_to_device(dev, y.ctypes.data, y.nbytes) == 0
+    idx, val = np.empty(k, np.int32), np.empty(k, np.float32)
+    assert lib.orkan_topk_f32(dev, n, k, idx.ctypes.data_as(C.POINTER(C.c_int)), val.ctypes.data_as(surrogate.FP)) == 0
+    lib.orkan_dev_free(dev)
+    want = np.lexsort((np.arange(n), -y))[:k]
+    assert np.array_equal(val, y[want]) and np.array_equal(y[idx], val)
+    tie = np.flatnonzero(val[1:] == val[:-1])
+    assert np.all(idx[tie] < idx[tie + 1]) and len(set(idx.tolist())) == k
