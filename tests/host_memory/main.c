@@ -203,6 +203,7 @@ int main(int argc, char **argv) {
         CHECK(nmallocs == before);
     } else if (!strcmp(what, "classes")) {
         /* for every size, a block of it or of up to an eighth more is taken, the nearest one first; a larger one is not */
+        capacity = 256 * MB;
         for (size_t n = 5000; n < 24 * MB; n += n / 3 + 4096) {
             orkan_mem_trim(0);
             void *exact = ork_mem_get(n), *more = ork_mem_get(n + n / 16 + (n >= 1 * MB ? 2 * MB : 4096));
