@@ -192,6 +192,7 @@ int ork_dev_malloc(void **p, size_t bytes) {
     *p = NULL;
     const hipError_t e = hipGetDevice(&dev);
     if (e != hipSuccess) return (int)e;
+    if (dev < 0 || dev >= ORK_MAX_DEV) return (int)hipErrorInvalidDevice;
     pthread_mutex_lock(&g_mem_mu);
     const int r = malloc_or_trim(dev, p, bytes);
     if (!r) mem_forget(*p);   /* an entry of this address is of a block that was freed elsewhere */
@@ -201,7 +202,7 @@ int ork_dev_malloc(void **p, size_t bytes) {
 
 size_t orkan_mem_trim(size_t keep_bytes) {
     int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= ORK_MAX_DEV) return 0;
     pthread_mutex_lock(&g_mem_mu);
     mem_trim(dev, keep_bytes);
     const size_t kept = g_mem_kept[dev];
